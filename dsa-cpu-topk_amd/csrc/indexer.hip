@@ -5,10 +5,13 @@
 // above the diagonal (written only on request -- the public drop-in asks for
 // it because callers check it, the internal split pipeline does not).
 //
-// Two kernels:
+// Three kernels:
 //
-// indexer_qtile_kernel (query-stationary; used whenever a 4-query tile of q
-//   fits in LDS).  A block owns TQ = 4*NQ consecutive queries of one batch
+// indexer_split_kernel (fp32, DI >= 32): the same query-stationary tiles with
+//   every fp32 product taken as three f16 products; its comment has the reasons.
+//
+// indexer_qtile_kernel (query-stationary; 16-bit and fp8, and fp32 at DI = 16;
+//   used whenever a 4-query tile of q fits in LDS).  A block owns TQ = 4*NQ consecutive queries of one batch
 //   element.  It stages their q rows (all heads) into LDS once, already in
 //   MFMA fragment order, so every later A-operand read is one conflict-free
 //   ds_read_b128 per lane, and their w rows next to them.  Its 16 waves (4
@@ -24,7 +27,7 @@
 //   x = (batch, 16-query tile), y = 256-key chunk; each wave owns 4 queries
 //   and walks its chunk with indexer_rows (indexer_tile.h).
 //
-// Both skip key blocks wholly above the diagonal (no MFMA work there); they
+// All skip key blocks wholly above the diagonal (no MFMA work there); they
 // only write -inf when asked, which is what the reference's kernel computes
 // for those tiles anyway (lightning_indexer.py:92-94).
 #include "dsa_launch.h"
@@ -422,6 +425,352 @@ __global__ __launch_bounds__((64 * qtile_waves<Tag, DI, NQ>())) void indexer_qti
   }
 }
 
+// ---------------------------------------------------------------------------
+// Query-stationary kernel for fp32 inputs on the f16 MFMA.
+//
+// The fp32 MFMA (16x16x4, 32 cycles) is what bounded the kernel above on
+// fp32 rows: 72% of its peak at config 3, and the matrix cores do 16 times as
+// many f16 products a cycle.  A float scaled to the f16 range is the sum of
+// two f16 values to 23 bits (h = round(x), l = round(x - h)), so
+//   <q,k> = <qh,kh> + <qh,kl> + <ql,kh>   (+ <ql,kl>, below 2^-24 |q||k|)
+// is three f16 MFMAs with fp32 accumulation per 32 dims: 96 cycles where the
+// fp32 MFMA takes 256.  The products of f16 values are exact in fp32, and 32
+// of them are summed per accumulation instead of 4, so the scores are no
+// further from float64 than the fp32 MFMA's (B = 4, T = 2047, HI = 8, DI = 64:
+// relative error 1.0e-7 against 1.5e-7, and 43 us with the -inf upper triangle
+// against 91; config 3, causal half: 0.31 -> 0.115 ms).  A k row is split by
+// every query tile that reads it, about 60 VALU instructions per 16 keys
+// against 48 MFMAs at HI = 8, DI = 64.
+//
+// Range: each (token, head) row of q and each k row is scaled by the power of
+// two that puts its largest element in [2^14, 2^15) -- exact, with elements
+// down to 2^-15 of the row's largest keeping all 23 bits and smaller ones an
+// absolute error of 2^-39 of it, far below what the fp32 sum itself drops.
+// Positive scales leave the ReLU: q's inverse is folded into w, k's multiplies
+// each finished score.  A super-block whose q rows, w rows or k rows hold a
+// non-finite value, or a scale too far out for that folding (rows beyond
+// 2^+-60, w outside [2^-40, 2^60]), is summed in plain fp32 from memory
+// instead: the split would turn inf into inf - inf.
+// ---------------------------------------------------------------------------
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// x, y (scaled) as two f16 pieces each, packed in pairs.
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32_t& l) {
+  const f16x2 hv = __builtin_convertvector((f32x2{x, y}), f16x2);
+  const f16x2 lv =
+      __builtin_convertvector((f32x2{x - static_cast<float>(hv[0]), y - static_cast<float>(hv[1])}), f16x2);
+  h = __builtin_bit_cast(uint32_t, hv);
+  l = __builtin_bit_cast(uint32_t, lv);
+}
+// Scale exponent of a row whose largest magnitude has these bits (sign
+// cleared): x * 2^sh puts it in [2^14, 2^15); 0 for a row of zeros.
+__device__ __forceinline__ bool split_scale(uint32_t maxbits, int& sh) {
+  const int e = static_cast<int>(maxbits >> 23);
+  sh = maxbits == 0u ? 0 : 141 - e;
+  return maxbits == 0u || (e >= 127 - 60 && e <= 127 + 60);
+}
+__device__ __forceinline__ float pow2f(int e) {  // 2^e, -126 <= e <= 127
+  return __uint_as_float(static_cast<uint32_t>(e + 127) << 23);
+}
+__device__ __forceinline__ uint32_t max_xor16_u32(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
+}
+__device__ __forceinline__ uint32_t max_xor32_u32(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
+}
+
+template <int DI>
+size_t split_lds_bytes(QTileShape sh) {
+  // both q pieces, w, and the inverse q scales
+  return static_cast<size_t>(sh.nq) * sh.nhg * (2 * (DI / 32) * 1024 + 64 + 64);
+}
+
+// LDS layout: qf[quad][hg][chunk][piece][lane] : uint4 (chunk = 8 of the lane
+// group's DI/4 dims), wf as in the kernel above, then the inverse q scales in
+// wf's layout.
+template <int DI, int KB, int NQ, int NW>
+__global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a) {
+  constexpr int E = DI / 4;      // dims per lane
+  constexpr int NCH = E / 8;     // 8-dim steps (one MFMA K each)
+  constexpr int TQ = 4 * NQ;
+  constexpr int SB = 16 * KB;
+  constexpr int NT = 64 * NW;
+  extern __shared__ __align__(16) uint4 lds[];
+  __shared__ uint32_t qbad;
+  const int T = a.T;
+  const int HI = a.HI;
+  const int nhg = (HI + 3) >> 2;
+  const int ntile = (T + TQ - 1) / TQ;
+  int64_t b;
+  int tile;
+  causal_block_tile(blockIdx.x, a.B, ntile, b, tile);  // longest rows first
+  const int t0 = tile * TQ;
+  const int tid = threadIdx.x;
+  const int wave = tid >> 6;
+  const int lane = lane_id();
+  const int g = lane >> 4, r16 = lane & 15;
+
+  const float* q = static_cast<const float*>(a.q) + b * T * a.ldq;
+  const float* k = static_cast<const float*>(a.k) + b * T * a.ldk;
+  const float* w = static_cast<const float*>(a.w) + b * T * a.ldw;
+  float* out = a.scores + (b * T) * a.ld;
+
+  uint4* qf = lds;
+  float* wf = reinterpret_cast<float*>(lds + static_cast<size_t>(NQ) * nhg * NCH * 2 * 64);
+  float* qs = wf + static_cast<size_t>(NQ) * nhg * 16;
+  if (tid == 0) qbad = 0u;
+  __syncthreads();
+
+  // Stage q: one 8-dim chunk (32 bytes) per thread-iteration; the DI/8
+  // threads of a (token, head) row are neighbouring lanes of one wave.
+  {
+    constexpr int RL = DI / 8;  // lanes per row
+    const int hp4 = 4 * nhg;
+    const int total = TQ * hp4 * RL;  // a multiple of RL: rows are whole or absent
+    for (int u = tid; u < total; u += NT) {
+      const int row = u / RL;
+      const int c8 = u % RL;
+      const int tl = row / hp4;
+      const int h = row - tl * hp4;
+      const int t = t0 + tl;
+      float x[8];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) x[i] = 0.f;
+      if (t < T && h < HI) load_f32<8>(q + static_cast<int64_t>(t) * a.ldq + h * DI + 8 * c8, x);
+      uint32_t mb = 0u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) mb = max(mb, __float_as_uint(x[i]) & 0x7fffffffu);
+#pragma unroll
+      for (int o = 1; o < RL; o <<= 1) mb = max(mb, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mb), o, kWave)));
+      int sh;
+      const bool ok = split_scale(mb, sh);
+      const float sc = ok ? pow2f(sh) : 0.f;
+      uint4 hv, lv;
+      split_pair(x[0] * sc, x[1] * sc, hv.x, lv.x);
+      split_pair(x[2] * sc, x[3] * sc, hv.y, lv.y);
+      split_pair(x[4] * sc, x[5] * sc, hv.z, lv.z);
+      split_pair(x[6] * sc, x[7] * sc, hv.w, lv.w);
+      const int gg = (8 * c8) / E;
+      const int c = (8 * c8 - gg * E) / 8;
+      const int ln = gg * 16 + 4 * (tl & 3) + (h & 3);
+      const size_t at = (static_cast<size_t>(tl >> 2) * nhg + (h >> 2)) * NCH + c;
+      qf[(2 * at) * 64 + ln] = hv;
+      qf[(2 * at + 1) * 64 + ln] = lv;
+      if (c8 == 0) {
+        qs[((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3)] = pow2f(-sh);
+        if (!ok) qbad = 1u;
+      }
+    }
+  }
+  __syncthreads();
+  {
+    const int hp4 = 4 * nhg;
+    for (int u = tid; u < TQ * hp4; u += NT) {
+      const int tl = u / hp4;
+      const int h = u - tl * hp4;
+      const int t = t0 + tl;
+      const float wv = (t < T && h < HI) ? w[static_cast<int64_t>(t) * a.ldw + h] : 0.f;
+      const uint32_t wb = __float_as_uint(wv) & 0x7fffffffu;
+      if (wb != 0u && (wb < (127u - 40u) << 23 || wb > (127u + 60u) << 23)) qbad = 1u;
+      const int at = ((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3);
+      wf[at] = wv * qs[at];
+    }
+  }
+  __syncthreads();
+  const bool bad_q = qbad != 0u;
+
+  const float ninf = -__builtin_huge_valf();
+  const int t_end = (t0 + TQ < T) ? t0 + TQ : T;  // keys [0, t_end) can be causal
+  const int nsb = (t_end + SB - 1) / SB;
+
+  auto store = [&](int qd, int s0, const float (&sc)[KB]) {
+    const int tq = t0 + 4 * qd + g;  // this lane's output query
+    if (tq < T) {
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) {
+        const int s = s0 + 16 * kb + r16;
+        if (s < T && (s <= tq || a.write_upper))
+          out[static_cast<int64_t>(tq) * a.ld + s] = (s <= tq) ? sc[kb] : ninf;
+      }
+    }
+  };
+
+  bool any_bad = bad_q;  // some super-block of this wave is left to the plain fp32 pass below
+  for (int sb = wave; sb < nsb && !bad_q; sb += NW) {
+    const int s0 = sb * SB;
+    // k rows of the super-block: loads first, then each block's scale and
+    // pieces (rows past T are clamped to row T-1, never stored).
+    float x[KB][E];
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+      load_f32<E>(k + static_cast<int64_t>(min(s0 + 16 * kb + r16, T - 1)) * a.ldk + g * E, x[kb]);
+    uint4 bh[KB][NCH], bl[KB][NCH];
+    float kinv[KB];
+    bool ok = true;
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb) {
+      uint32_t mb = 0u;
+#pragma unroll
+      for (int e = 0; e < E; ++e) mb = max(mb, __float_as_uint(x[kb][e]) & 0x7fffffffu);
+      mb = max_xor32_u32(max_xor16_u32(mb));
+      int sh;
+      ok &= split_scale(mb, sh);
+      kinv[kb] = pow2f(-min(max(sh, -120), 120));
+      const float sc = pow2f(min(max(sh, -120), 120));
+#pragma unroll
+      for (int c = 0; c < NCH; ++c) {
+        split_pair(x[kb][8 * c] * sc, x[kb][8 * c + 1] * sc, bh[kb][c].x, bl[kb][c].x);
+        split_pair(x[kb][8 * c + 2] * sc, x[kb][8 * c + 3] * sc, bh[kb][c].y, bl[kb][c].y);
+        split_pair(x[kb][8 * c + 4] * sc, x[kb][8 * c + 5] * sc, bh[kb][c].z, bl[kb][c].z);
+        split_pair(x[kb][8 * c + 6] * sc, x[kb][8 * c + 7] * sc, bh[kb][c].w, bl[kb][c].w);
+      }
+    }
+    if (ballot(!ok) != 0u) {
+      any_bad = true;
+      continue;
+    }
+    const uint4* qa = qf + lane;
+    const float4* wq = reinterpret_cast<const float4*>(wf) + g;
+#pragma unroll 1
+    for (int qd = 0; qd < NQ; ++qd) {
+      float sc[KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) sc[kb] = 0.f;
+      for (int hg = 0; hg < nhg; ++hg) {
+        const int unit = qd * nhg + hg;
+        f32x4 acc[KB];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) acc[kb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        auto mm = [](const uint4& x, const uint4& y, f32x4 c) {
+          return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, x),
+                                                        __builtin_bit_cast(f16x8, y), c, 0, 0, 0);
+        };
+        constexpr int AG = NCH < 4 ? NCH : 4;  // chunks whose A fragments are read at once
+#pragma unroll
+        for (int c0 = 0; c0 < NCH; c0 += AG) {
+          uint4 ah[AG], al[AG];
+#pragma unroll
+          for (int c = 0; c < AG; ++c) {
+            ah[c] = qa[(2 * (unit * NCH + c0 + c)) * 64];
+            al[c] = qa[(2 * (unit * NCH + c0 + c) + 1) * 64];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+          __builtin_amdgcn_s_setprio(1);
+          // the small terms first
+#pragma unroll
+          for (int c = 0; c < AG; ++c) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) acc[kb] = mm(al[c], bh[kb][c0 + c], acc[kb]);
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) acc[kb] = mm(ah[c], bl[kb][c0 + c], acc[kb]);
+          }
+#pragma unroll
+          for (int c = 0; c < AG; ++c)
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb) acc[kb] = mm(ah[c], bh[kb][c0 + c], acc[kb]);
+          __builtin_amdgcn_s_setprio(0);
+        }
+        const float4 wv = wq[unit * 4];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          sc[kb] = fmaf(wv.x, relu_f32(acc[kb][0]), sc[kb]);
+          sc[kb] = fmaf(wv.y, relu_f32(acc[kb][1]), sc[kb]);
+          sc[kb] = fmaf(wv.z, relu_f32(acc[kb][2]), sc[kb]);
+          sc[kb] = fmaf(wv.w, relu_f32(acc[kb][3]), sc[kb]);
+        }
+      }
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) sc[kb] *= kinv[kb];
+      store(qd, s0, sc);
+    }
+  }
+
+  // The super-blocks skipped above, in plain fp32 from memory, each lane its
+  // own (query, key) pairs.
+  for (int sb = wave; sb < nsb && any_bad; sb += NW) {
+    const int s0 = sb * SB;
+    if (!bad_q) {
+      bool ok = true;
+      for (int kb = 0; kb < KB; ++kb) {
+        const float* kr = k + static_cast<int64_t>(min(s0 + 16 * kb + r16, T - 1)) * a.ldk + g * E;
+        uint32_t mb = 0u;
+        for (int e = 0; e < E; ++e) mb = max(mb, __float_as_uint(kr[e]) & 0x7fffffffu);
+        mb = max_xor32_u32(max_xor16_u32(mb));
+        int sh;
+        ok &= split_scale(mb, sh);
+      }
+      if (ballot(!ok) == 0u) continue;
+    }
+#pragma unroll 1
+    for (int qd = 0; qd < NQ; ++qd) {
+      const int tq = min(t0 + 4 * qd + g, T - 1);
+      float sc[KB];
+#pragma unroll
+      for (int kb = 0; kb < KB; ++kb) sc[kb] = 0.f;
+#pragma unroll 1
+      for (int h = 0; h < HI; ++h) {
+        const float* qr = q + static_cast<int64_t>(tq) * a.ldq + h * DI;
+        const float wv = w[static_cast<int64_t>(tq) * a.ldw + h];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) {
+          const float* kr = k + static_cast<int64_t>(min(s0 + 16 * kb + r16, T - 1)) * a.ldk;
+          float d = 0.f;
+#pragma unroll 1
+          for (int e = 0; e < DI; ++e) d = fmaf(qr[e], kr[e], d);
+          sc[kb] = fmaf(wv, relu_f32(d), sc[kb]);
+        }
+      }
+      store(qd, s0, sc);
+    }
+  }
+
+  // Keys past the last super-block are above the diagonal for every query.
+  if (a.write_upper) {
+    const int s_lo = nsb * SB;
+    if (s_lo < T) {
+      for (int tl = wave; tl < TQ; tl += NW) {
+        const int t = t0 + tl;
+        if (t >= T) break;
+        for (int s = s_lo + lane; s < T; s += 64) out[static_cast<int64_t>(t) * a.ld + s] = ninf;
+      }
+    }
+  }
+}
+
+template <int DI, int KB, int NQ, int NW>
+hipError_t launch_split(const IndexerArgs& a, QTileShape sh, hipStream_t stream) {
+  auto kern = indexer_split_kernel<DI, KB, NQ, NW>;
+  static const bool attr_set = [&] {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             static_cast<int>(kQTileLds - 64));
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e == hipSuccess;
+  }();
+  (void)attr_set;
+  const int64_t nblk = a.B * ((a.T + 4 * NQ - 1) / (4 * NQ));
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(nblk)), dim3(64 * NW),
+                     split_lds_bytes<DI>(sh), stream, a);
+  return hipGetLastError();
+}
+
+// The fp32 launch on f16 pieces: the most quads whose q pieces leave two
+// 8-wave blocks per CU, else (wide q rows) one 16-wave block.
+// hipErrorNotSupported when one quad does not fit (the streaming kernel runs).
+template <int DI, int KB>
+hipError_t dispatch_split(const IndexerArgs& a, hipStream_t stream) {
+  const int nhg = (a.HI + 3) / 4;
+  auto lds = [&](int nq) { return split_lds_bytes<DI>(QTileShape{nq, nhg}); };
+  if (lds(4) <= kQTileLds / 2 - 64) return launch_split<DI, KB, 4, 8>(a, {4, nhg}, stream);
+  if (lds(2) <= kQTileLds / 2 - 64) return launch_split<DI, KB, 2, 8>(a, {2, nhg}, stream);
+  if (lds(2) <= kQTileLds - 64) return launch_split<DI, KB, 2, 16>(a, {2, nhg}, stream);
+  if (lds(1) <= kQTileLds - 64) return launch_split<DI, KB, 1, 16>(a, {1, nhg}, stream);
+  return hipErrorNotSupported;
+}
+
 template <typename Tag, int DI, int KB, int NQ, bool KS = false>
 hipError_t launch_qtile(const IndexerArgs& a, QTileShape sh, hipStream_t stream) {
   auto kern = indexer_qtile_kernel<Tag, DI, KB, NQ, KS>;
@@ -496,12 +845,20 @@ hipError_t dispatch_di(const IndexerArgs& a, int DI, hipStream_t stream) {
       case 256: return launch<Tag, 256, 2>(a, stream);
     }
   } else if constexpr (Tag::kBytes == 4) {
+    hipError_t e = hipErrorNotSupported;
+    switch (DI) {
+      case 32: e = dispatch_split<32, 4>(a, stream); break;
+      case 64: e = dispatch_split<64, 4>(a, stream); break;
+      case 128: e = dispatch_split<128, 2>(a, stream); break;
+      case 256: e = dispatch_split<256, 1>(a, stream); break;
+    }
+    if (e != hipErrorNotSupported) return e;
     switch (DI) {
       case 16: return launch<Tag, 16, 4>(a, stream);
-      case 32: return launch<Tag, 32, 4>(a, stream);
-      case 64: return launch<Tag, 64, 4>(a, stream);
-      case 128: return launch<Tag, 128, 2>(a, stream);
-      case 256: return launch<Tag, 256, 1>(a, stream);
+      case 32: return launch_stream<Tag, 32, 4>(a, stream);
+      case 64: return launch_stream<Tag, 64, 4>(a, stream);
+      case 128: return launch_stream<Tag, 128, 2>(a, stream);
+      case 256: return launch_stream<Tag, 256, 1>(a, stream);
     }
   } else {
     switch (DI) {

@@ -2,6 +2,8 @@
 for fp32 inputs, 2e-2 for 16-bit inputs; off-causal entries exactly -inf)."""
 from __future__ import annotations
 
+import math
+
 import pytest
 import torch
 
@@ -323,3 +325,65 @@ def test_fp8_scales_need_fp8_inputs(dev):
     k = torch.zeros(1, 8, 64, device=dev)
     with pytest.raises(AssertionError):
         indexer_scores_hip(q, k, torch.zeros(1, 8, 4, device=dev), k_scale=torch.ones(1, 8, device=dev))
+
+
+# ---------------------------------------------------------------------------
+# fp32 rows of DI >= 32 on f16 pieces (three f16 MFMAs per product).  Bound,
+# per score: each product keeps 2^-22 of itself (two 23-bit operands, the
+# dropped l*l term), and every fp32 addition it passes through 2^-24:
+# 3*DI/32 accumulations, HI head sums, the weight and scale products.  So
+# |err| <= (4 + (3*DI/32 + HI + 4) * 2) * 2^-24 * sum_h |w_h| sum_e |q_he k_e|.
+# ---------------------------------------------------------------------------
+def _split_bound(q, k, w):
+    B, T, HI, DI = q.shape
+    q, k, w = q.double().abs(), k.double().abs(), w.double().abs()
+    l1 = torch.einsum("bth,bths->bts", w, torch.einsum("bthd,bsd->bths", q, k))
+    return (4 + (3 * DI / 32 + HI + 4) * 2) * 2.0 ** -24 * l1
+
+
+@pytest.mark.parametrize("T,HI,DI", [(1, 1, 32), (15, 3, 64), (64, 8, 64), (65, 5, 128), (130, 4, 32),
+                                     (333, 9, 64), (50, 4, 256), (100, 40, 128), (90, 80, 128)])
+def test_fp32_pieces_shapes_and_scales(dev, T, HI, DI):
+    """Edges of the query and key tiles, one and two blocks per CU, one-quad
+    tiles; rows of very different magnitude (scales 2^-50 .. 2^50, and beyond
+    the split's 2^+-60, which takes the plain fp32 pass)."""
+    q, k, w, *_ = O.make_inputs(2, T, HI, DI, 1, 1, 1, seed0=T)
+    g = torch.Generator().manual_seed(T + 1)
+    for span in (0, 50, 66):
+        eq = torch.randint(-span, span + 1, (2, T, HI, 1), generator=g).float()
+        ek = torch.randint(-span // 2, span // 2 + 1, (2, T, 1), generator=g).float()
+        qs, ks = q * torch.exp2(eq), k * torch.exp2(ek)
+        ks[0, T // 2] = 0.0
+        # a row whose elements span many binades
+        qs[1, T - 1] *= torch.exp2(torch.randint(-12, 1, (HI, DI), generator=g).float())
+        say(f"indexer pieces T={T} HI={HI} DI={DI} span={span}")
+        out = indexer_scores_hip(qs.to(dev), ks.to(dev), w.to(dev)).cpu()
+        ref = O.indexer_scores(qs, ks, w)
+        causal = torch.ones(T, T, dtype=torch.bool).tril()
+        err = (out.double() - ref)[:, causal].abs()
+        assert bool((err <= _split_bound(qs, ks, w)[:, causal] + 1e-37).all()), float(err.max())
+        assert bool(torch.isneginf(out[:, ~causal]).all())
+
+
+def test_fp32_pieces_nonfinite_rows(dev):
+    """inf and NaN in q, k or w give what the plain fp32 sum gives (the
+    pieces of inf would be inf - inf); rows without them are untouched."""
+    T, HI, DI = 150, 8, 64
+    q, k, w, *_ = O.make_inputs(1, T, HI, DI, 1, 1, 1, seed0=5)
+    w = w.abs()
+    clean = indexer_scores_hip(q.to(dev), k.to(dev), w.to(dev)).cpu()
+    q[0, 40, 2, 7] = math.inf
+    q[0, 140, 0, 0] = math.nan
+    k[0, 70, 9] = -math.inf
+    k[0, 71, 0] = math.nan
+    w[0, 100, 3] = math.inf
+    w[0, 120, 1] = 1e-30
+    out = indexer_scores_hip(q.to(dev), k.to(dev), w.to(dev)).cpu()
+    ref = O.indexer_scores(q, k, w)
+    causal = torch.ones(T, T, dtype=torch.bool).tril()
+    assert torch.equal(torch.isnan(out), torch.isnan(ref))
+    assert torch.equal(torch.isinf(out), torch.isinf(ref))
+    fin = torch.isfinite(ref) & causal
+    assert bool(((out.double() - ref).abs()[fin] <= 1e-4 + 1e-4 * ref.abs()[fin]).all())
+    # 64-query rows away from the planted queries, keys before the planted keys
+    assert torch.equal(out[0, :32], clean[0, :32])
