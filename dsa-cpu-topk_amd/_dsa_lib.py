@@ -54,6 +54,12 @@ _SIGNATURES = {
     "dsa_sparse_attn_threshold_staged_ws": ([_P, _I64, _P, _P, _P, _P, _I, _I64, _I64, _I, _I,
                                              _I, _F, _P, _P, _I64, _P], _I),
     "dsa_sparse_attn_workspace_bytes": ([_I, _I, _I64, _I64, _I, _I, _I, _I64], _I64),
+    "dsa_sparse_attn_dense_workspace_bytes": ([_I, _I64, _I64, _I, _I, _I], _I64),
+    "dsa_sparse_attn_pick": ([_I, _I64, _I64, _I, _I, _I, _I64], _I),
+    "dsa_sparse_attn_gather": ([_P, _I64, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _F, _P, _P],
+                               _I),
+    "dsa_sparse_attn_dense": ([_P, _I64, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _F, _P, _P,
+                               _I64, _P], _I),
     "dsa_fused_forward": ([_P, _P, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _I, _I, _I, _F,
                            _P, _P], _I),
     "dsa_selection_mask": ([_P, _I64, _P, _I64, _I64, _P, _I64, _P], _I),

@@ -26,7 +26,7 @@ CPU_SOURCES = ["topk_cpu.cpp"]
 # -ffast-math (score rows hold -inf and NaN must order as torch.topk orders it).
 CXXFLAGS = ["-O3", "-std=c++17", "-fPIC", "-fopenmp", "-Wall", "-Wextra"]
 SOURCES = ["capi.cpp", "topk.hip", "indexer.hip", "sparse_attn.hip", "tile_attn.hip",
-           "staged_attn.hip", "fused.hip"]
+           "staged_attn.hip", "dense_attn.hip", "fused.hip"]
 
 HIPFLAGS = [
     "--offload-arch=gfx950",

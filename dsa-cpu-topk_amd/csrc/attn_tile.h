@@ -84,7 +84,9 @@ __device__ __forceinline__ void load_query(const typename Tag::raw* __restrict__
 }
 
 // Q/K/V point at this batch element: Q row t is Q + t*HQ*DQ, etc.
-// load4(s, sv) loads scores s..s+3 (s <= t, s % 4 == 0) of this query's row.
+// segment(s0) writes the selected keys of s0 .. s0 + kListCap - 1 to `list` in
+// index order and returns how many (attend_query: from scores, load4(s, sv)
+// loading scores s..s+3, s <= t, s % 4 == 0, of this query's row).
 // qpre: this lane's query slice from load_query, loaded early by the caller
 // (nullptr: loaded here).  PIPE: overlap each group's loads with the
 // neighbouring group's arithmetic (below); it needs more registers, which
@@ -93,15 +95,15 @@ __device__ __forceinline__ void load_query(const typename Tag::raw* __restrict__
 // wave's registers).  Then Q/K/V/out_row point at the chunk's first head
 // and RQ / RV give the full row lengths (elements of a Q or K row, of a V
 // row); 0 means the row is exactly the HQ heads.
-template <typename Tag, int EK, int EV, bool PIPE = false, typename Load4>
-__device__ __forceinline__ void attend_query(const typename Tag::raw* __restrict__ Q,
-                                             const typename Tag::raw* __restrict__ K,
-                                             const typename Tag::raw* __restrict__ V, int t,
-                                             int HQ, int DQ, int DV, float scale_log2,
-                                             float thr, Load4&& load4, int* list,
-                                             float* __restrict__ out_row,
-                                             const float* qpre = nullptr, int RQ = 0,
-                                             int RV = 0) {
+template <typename Tag, int EK, int EV, bool PIPE = false, typename Segment>
+__device__ __forceinline__ void attend_query_on(const typename Tag::raw* __restrict__ Q,
+                                                const typename Tag::raw* __restrict__ K,
+                                                const typename Tag::raw* __restrict__ V, int t,
+                                                int HQ, int DQ, int DV, float scale_log2,
+                                                Segment&& segment, int* list,
+                                                float* __restrict__ out_row,
+                                                const float* qpre = nullptr, int RQ = 0,
+                                                int RV = 0) {
   using raw = typename Tag::raw;
   const int lane = lane_id();
   const int EQ = HQ * DQ;
@@ -346,7 +348,7 @@ __device__ __forceinline__ void attend_query(const typename Tag::raw* __restrict
   };
 
   for (int s0 = 0; s0 <= t; s0 += kListCap) {
-    const int total = compact_segment(s0, t, thr, load4, list);
+    const int total = segment(s0);
     wave_lds_sync();
     if (use_rs) run_groups(total, half_a_rs, half_b_rs);
     else run_groups(total, half_a, half_b);
@@ -366,6 +368,22 @@ __device__ __forceinline__ void attend_query(const typename Tag::raw* __restrict
 #pragma unroll
     for (int e = 0; e < EV; ++e) out_row[lane * EV + e] = acc[e] * inv;
   }
+}
+
+// The same with the selection read from the score row.
+template <typename Tag, int EK, int EV, bool PIPE = false, typename Load4>
+__device__ __forceinline__ void attend_query(const typename Tag::raw* __restrict__ Q,
+                                             const typename Tag::raw* __restrict__ K,
+                                             const typename Tag::raw* __restrict__ V, int t,
+                                             int HQ, int DQ, int DV, float scale_log2,
+                                             float thr, Load4&& load4, int* list,
+                                             float* __restrict__ out_row,
+                                             const float* qpre = nullptr, int RQ = 0,
+                                             int RV = 0) {
+  attend_query_on<Tag, EK, EV, PIPE>(
+      Q, K, V, t, HQ, DQ, DV, scale_log2,
+      [&](int s0) { return compact_segment(s0, t, thr, load4, list); }, list, out_row, qpre, RQ,
+      RV);
 }
 
 // Elements [4j, 4j + 4), j = lane % 32, of fp32 query row t (rows of 128
@@ -398,13 +416,13 @@ __device__ __forceinline__ void load_query_pair(const float* __restrict__ Q, int
 // V loads go out together (overlapping them with the neighbouring group's
 // arithmetic, as attend_query's PIPE form does, measured 2% slower here: the
 // gathers are bound by the CU's load issue, not by their latency).
-template <typename Load4>
-__device__ __forceinline__ void attend_query_pair(const float* __restrict__ Q,
-                                                  const float* __restrict__ K,
-                                                  const float* __restrict__ V, int t, int DQ,
-                                                  float scale_log2, float thr, Load4&& load4,
-                                                  int* list, float* __restrict__ out_row,
-                                                  const float* qpre = nullptr) {
+template <typename Segment>
+__device__ __forceinline__ void attend_query_pair_on(const float* __restrict__ Q,
+                                                     const float* __restrict__ K,
+                                                     const float* __restrict__ V, int t, int DQ,
+                                                     float scale_log2, Segment&& segment, int* list,
+                                                     float* __restrict__ out_row,
+                                                     const float* qpre = nullptr) {
   constexpr uint32_t kRowBytes = 128 * 4;
   constexpr int NL = 8;  // loads per group: 16 keys
   const int lane = lane_id();
@@ -498,7 +516,7 @@ __device__ __forceinline__ void attend_query_pair(const float* __restrict__ Q,
   float kv[NL][4], vv[NL][4];
   bool okk[NL], okv[NL];
   for (int s0 = 0; s0 <= t; s0 += kListCap) {
-    const int total = compact_segment(s0, t, thr, load4, list);
+    const int total = segment(s0);
     wave_lds_sync();
     for (int i = 0; i < total; i += 2 * NL) {
       const int nu = min(2 * NL, total - i);
@@ -517,6 +535,19 @@ __device__ __forceinline__ void attend_query_pair(const float* __restrict__ Q,
     *reinterpret_cast<float4*>(out_row + j4) =
         make_float4(acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv);
   }
+}
+
+// The same with the selection read from the score row.
+template <typename Load4>
+__device__ __forceinline__ void attend_query_pair(const float* __restrict__ Q,
+                                                  const float* __restrict__ K,
+                                                  const float* __restrict__ V, int t, int DQ,
+                                                  float scale_log2, float thr, Load4&& load4,
+                                                  int* list, float* __restrict__ out_row,
+                                                  const float* qpre = nullptr) {
+  attend_query_pair_on(
+      Q, K, V, t, DQ, scale_log2,
+      [&](int s0) { return compact_segment(s0, t, thr, load4, list); }, list, out_row, qpre);
 }
 
 }  // namespace dsa

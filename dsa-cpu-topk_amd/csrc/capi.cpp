@@ -339,6 +339,53 @@ int dsa_sparse_attn_threshold_staged(const float* scores, int64_t ld, const floa
                                              scale, out, nullptr, 0, stream);
 }
 
+int64_t dsa_sparse_attn_dense_workspace_bytes(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV) {
+  if (!dtype_ok(dtype) || B <= 0 || T <= 0 || HQ < 1 || DQ < 1 || DV < 1 ||
+      !dsa::dense_attn_supported(dtype, T, HQ, DQ, DV))
+    return 0;
+  return dsa::dense_attn_workspace(dtype, B, T, HQ, DQ);
+}
+
+int dsa_sparse_attn_pick(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int64_t top_k) {
+  if (!dtype_ok(dtype) || B <= 0 || T <= 0 || HQ < 1 || DQ < 1 || DV < 1 || top_k < 0) return 0;
+  return static_cast<int>(dsa::pick_sparse_attn(dtype, B, T, HQ, DQ, DV, top_k));
+}
+
+int dsa_sparse_attn_gather(const float* scores, int64_t ld, const float* thr, const void* Q,
+                           const void* K, const void* V, int dtype, int64_t B, int64_t T, int HQ,
+                           int DQ, int DV, float scale, float* out, void* stream) {
+  int rc = check_attn(dtype, B, T, HQ, DQ, DV, Q, K, V, out, "sparse_attn_gather");
+  if (rc != DSA_OK) return rc;
+  if (ld < T) return fail(DSA_EINVAL, "sparse_attn_gather: ld=%lld < T=%lld", (long long)ld, (long long)T);
+  if (!std::isfinite(scale)) return fail(DSA_EINVAL, "sparse_attn_gather: scale must be finite");
+  if (B * T == 0) return DSA_OK;
+  if (!scores || !thr) return fail(DSA_EINVAL, "sparse_attn_gather: null pointer");
+  return hip_status(dsa::launch_sparse_attn_gather(scores, ld, thr, Q, K, V, dtype, B, T, HQ, DQ, DV,
+                                                   scale, out, static_cast<hipStream_t>(stream)),
+                    "dsa_sparse_attn_gather");
+}
+
+int dsa_sparse_attn_dense(const float* scores, int64_t ld, const float* thr, const void* Q,
+                          const void* K, const void* V, int dtype, int64_t B, int64_t T, int HQ,
+                          int DQ, int DV, float scale, float* out, void* workspace,
+                          int64_t workspace_bytes, void* stream) {
+  int rc = check_attn(dtype, B, T, HQ, DQ, DV, Q, K, V, out, "sparse_attn_dense");
+  if (rc != DSA_OK) return rc;
+  if (ld < T) return fail(DSA_EINVAL, "sparse_attn_dense: ld=%lld < T=%lld", (long long)ld, (long long)T);
+  if (!std::isfinite(scale)) return fail(DSA_EINVAL, "sparse_attn_dense: scale must be finite");
+  if (workspace_bytes < 0) return fail(DSA_EINVAL, "sparse_attn_dense: negative workspace size");
+  if (!dsa::dense_attn_supported(dtype, T, HQ, DQ, DV))
+    return fail(DSA_EUNSUPPORTED, "sparse_attn_dense: needs DQ = DV in {64,128} and T <= 2^20 (T=%lld HQ=%d DQ=%d DV=%d dtype %d)", (long long)T, HQ, DQ, DV, dtype);
+  if (B * T == 0) return DSA_OK;
+  if (!scores || !thr) return fail(DSA_EINVAL, "sparse_attn_dense: null pointer");
+  const int64_t need = dsa::dense_attn_workspace(dtype, B, T, HQ, DQ);
+  if (!workspace || !aligned16(workspace) || workspace_bytes < need)
+    return fail(DSA_EINVAL, "sparse_attn_dense: needs a 16-byte aligned workspace of %lld bytes (got %lld)", (long long)need, (long long)workspace_bytes);
+  return hip_status(dsa::launch_dense_attn(scores, ld, thr, Q, K, V, dtype, B, T, HQ, DQ, scale, out,
+                                           workspace, static_cast<hipStream_t>(stream)),
+                    "dsa_sparse_attn_dense");
+}
+
 int dsa_fused_forward(const void* q_idx, const void* k_idx, const void* w_idx, const void* Q,
                       const void* K, const void* V, int dtype, int64_t B, int64_t T, int HI,
                       int DI, int HQ, int DQ, int DV, int top_k, float scale, float* out,

@@ -327,6 +327,45 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_rsrc(const char* base, in
                                            0x00020000);
 }
 
+// ---------------------------------------------------------------------------
+// fp32 values as two f16 pieces: x = h + l to 23 bits (h = round(x),
+// l = round(x - h)) for |x| in [2^-1, 2^15); smaller values of a scaled row
+// keep an absolute error of 2^-25.
+// ---------------------------------------------------------------------------
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+
+// x, y (scaled) as two f16 pieces each, packed in pairs.  The remainders are
+// one v_fma_mix_f32 each (x * 1 - h with h read as f16: exact); written in C
+// the compiler converts h back to fp32 first, two instructions.
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32_t& l) {
+  h = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{x, y}), f16x2));
+  float lx, ly;
+  __asm__("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[0,0,1]" : "=v"(lx) : "v"(x), "v"(h));
+  __asm__("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[0,0,1] op_sel_hi:[0,0,1]"
+          : "=v"(ly)
+          : "v"(y), "v"(h));
+  l = __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lx, ly}), f16x2));
+}
+// Scale exponent of a row whose largest magnitude has these bits (sign
+// cleared): x * 2^sh puts it in [2^14, 2^15); 0 for a row of zeros.
+__device__ __forceinline__ bool split_scale(uint32_t maxbits, int& sh) {
+  const int e = static_cast<int>(maxbits >> 23);
+  sh = maxbits == 0u ? 0 : 141 - e;
+  return maxbits == 0u || (e >= 127 - 60 && e <= 127 + 60);
+}
+__device__ __forceinline__ float pow2f(int e) {  // 2^e, -126 <= e <= 127
+  return __uint_as_float(static_cast<uint32_t>(e + 127) << 23);
+}
+__device__ __forceinline__ uint32_t max_xor16_u32(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+  return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
+}
+__device__ __forceinline__ uint32_t max_xor32_u32(uint32_t v) {
+  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
+}
+
 // Block order for causal work whose cost grows with the query tile.
 // Workgroups are dispatched in index order, round-robin over the 8 XCDs
 // (block i starts on XCD i % 8).  Index order here is: tiles longest first,

@@ -124,6 +124,20 @@ hipError_t launch_staged_attn(const float* scores, int64_t ld, const float* thr,
                               int HQ, int DQ, float scale, float* out, void* ws, int64_t ws_bytes,
                               hipStream_t stream);
 
+// The same attention computed densely on MFMA tiles with fp32 probabilities
+// (dense_attn.hip): DQ = DV in {64, 128}.
+// Needs a workspace of dense_attn_workspace bytes, 16-byte aligned.
+bool dense_attn_supported(int dtype, int64_t T, int HQ, int DQ, int DV);
+int64_t dense_attn_workspace(int dtype, int64_t B, int64_t T, int HQ, int D);
+// The kernel expected to be fastest for a shape whose queries select about
+// top_k keys (0: unknown): what launch_sparse_attn picks, the dense kernel, or
+// the per-query gathers.
+enum class AttnPick { kThreshold = 0, kDense = 1, kGather = 2 };
+AttnPick pick_sparse_attn(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int64_t top_k);
+hipError_t launch_dense_attn(const float* scores, int64_t ld, const float* thr, const void* Q,
+                             const void* K, const void* V, int dtype, int64_t B, int64_t T, int HQ,
+                             int D, float scale, float* out, void* ws, hipStream_t stream);
+
 // Fused forward for T <= kFusedMaxT.
 constexpr int64_t kFusedMaxT = 2048;
 hipError_t launch_fused(const void* qi, const void* ki, const void* wi, const void* Q,

@@ -452,36 +452,6 @@ __global__ __launch_bounds__((64 * qtile_waves<Tag, DI, NQ>())) void indexer_qti
 // 2^+-60, w outside [2^-40, 2^60]), is summed in plain fp32 from memory
 // instead: the split would turn inf into inf - inf.
 // ---------------------------------------------------------------------------
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-
-// x, y (scaled) as two f16 pieces each, packed in pairs.
-__device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32_t& l) {
-  const f16x2 hv = __builtin_convertvector((f32x2{x, y}), f16x2);
-  const f16x2 lv =
-      __builtin_convertvector((f32x2{x - static_cast<float>(hv[0]), y - static_cast<float>(hv[1])}), f16x2);
-  h = __builtin_bit_cast(uint32_t, hv);
-  l = __builtin_bit_cast(uint32_t, lv);
-}
-// Scale exponent of a row whose largest magnitude has these bits (sign
-// cleared): x * 2^sh puts it in [2^14, 2^15); 0 for a row of zeros.
-__device__ __forceinline__ bool split_scale(uint32_t maxbits, int& sh) {
-  const int e = static_cast<int>(maxbits >> 23);
-  sh = maxbits == 0u ? 0 : 141 - e;
-  return maxbits == 0u || (e >= 127 - 60 && e <= 127 + 60);
-}
-__device__ __forceinline__ float pow2f(int e) {  // 2^e, -126 <= e <= 127
-  return __uint_as_float(static_cast<uint32_t>(e + 127) << 23);
-}
-__device__ __forceinline__ uint32_t max_xor16_u32(uint32_t v) {
-  const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-  return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
-}
-__device__ __forceinline__ uint32_t max_xor32_u32(uint32_t v) {
-  const auto r = __builtin_amdgcn_permlane32_swap(v, v, false, false);
-  return max(static_cast<uint32_t>(r[0]), static_cast<uint32_t>(r[1]));
-}
-
 template <int DI>
 size_t split_lds_bytes(QTileShape sh) {
   // both q pieces, w, and the inverse q scales

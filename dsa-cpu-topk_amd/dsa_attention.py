@@ -76,13 +76,16 @@ def _attn_inputs(Q, K, V):
 
 def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
                          out: torch.Tensor | None = None, tiled: bool = False,
-                         kernel: str | None = None) -> torch.Tensor:
+                         kernel: str | None = None, top_k: int = 0) -> torch.Tensor:
     """Sparse attention for any T given scores [B,T,T] fp32 and threshold
     [B,T,1] (or [B,T]); only entries s <= t of each score row are read.
 
     The library picks the kernel: per-query gathers; dense-masked MFMA tiles
-    for T >= 4096 with 16-bit Q/K/V and DQ = DV in {64, 128}; K/V staged
-    through LDS for fp32 rows of HQ*DQ = 512 at T >= 3072 when the batch
+    for T >= 4096 with 16-bit Q/K/V and DQ = DV in {64, 128}; dense-masked
+    MFMA tiles with fp32 probabilities for other shapes of DQ = DV in {64,
+    128} where they are expected to be faster (dsa_sparse_attn_pick; top_k, the
+    keys each query is expected to select, helps that rule and changes nothing
+    else); K/V staged through LDS for fp32 rows of HQ*DQ = 512 at T >= 3072 when the batch
     gives at least one 64-query tile per compute unit (with a workspace
     from the caching allocator, so that long key ranges split over several
     blocks; dsa_sparse_attn_workspace_bytes gives its size).  Where it would
@@ -90,8 +93,10 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
     (dsa_selection_mask, 1 bit per (query, key) instead of a 4-byte score
     read once per head) and the tile kernel reads that (dsa_sparse_attn_mask):
     the same output, bit for bit.
-    kernel="tiled" (or tiled=True) / "staged" / "mask" runs that kernel at
-    any T (AssertionError for shapes it does not cover)."""
+    kernel="tiled" (or tiled=True) / "staged" / "mask" / "dense" / "gather" runs that
+    kernel at any T (AssertionError for shapes it does not cover); "staged"
+    is the dense one where the library would otherwise have staged (T >= 3072)
+    and now takes it."""
     L.require_gpu(scores, threshold, Q, K, V)
     B, T, _ = scores.shape
     HQ, DQ = Q.shape[-2], Q.shape[-1]
@@ -106,20 +111,34 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
         out = torch.empty(B, T, HQ, DV, device=Q.device, dtype=torch.float32)
     if tiled:
         kernel = "tiled"
-    assert kernel in (None, "tiled", "staged", "mask"), f"unknown kernel {kernel!r}"
+    assert kernel in (None, "tiled", "staged", "mask", "dense", "gather"), f"unknown kernel {kernel!r}"
     if kernel is None and L.lib().dsa_sparse_attn_uses_mask(L.dtype_code(dt), T, HQ, DQ, DV):
         kernel = "mask"
     if kernel == "mask":
         return _sparse_attention_mask(scores, thr, Q, K, V, out)
+    code = L.dtype_code(dt)
+    if kernel is None or (kernel == "staged" and T >= 3072):
+        with torch.cuda.device(Q.device):
+            kernel = {0: kernel, 1: "dense", 2: "gather"}[
+                L.lib().dsa_sparse_attn_pick(code, B, T, HQ, DQ, DV, int(top_k))]
+    if kernel == "dense":
+        nws = L.lib().dsa_sparse_attn_dense_workspace_bytes(code, B, T, HQ, DQ, DV)
+        ws = torch.empty(max(nws, 16), device=Q.device, dtype=torch.uint8)
+        L.check(L.lib().dsa_sparse_attn_dense(
+            scores.data_ptr(), T, thr.data_ptr(), Q.data_ptr(), K.data_ptr(), V.data_ptr(), code,
+            B, T, HQ, DQ, DV, 1.0 / math.sqrt(DQ), out.data_ptr(), ws.data_ptr(), nws,
+            L.stream_ptr(Q.device)), "sparse_attention")
+        return out
     args = (scores.data_ptr(), T, thr.data_ptr(), Q.data_ptr(), K.data_ptr(), V.data_ptr(),
-            L.dtype_code(dt), B, T, HQ, DQ, DV, 1.0 / math.sqrt(DQ), out.data_ptr())
+            code, B, T, HQ, DQ, DV, 1.0 / math.sqrt(DQ), out.data_ptr())
     if kernel == "tiled":
         rc = L.lib().dsa_sparse_attn_threshold_tiled(*args, L.stream_ptr(Q.device))
+    elif kernel == "gather":
+        rc = L.lib().dsa_sparse_attn_gather(*args, L.stream_ptr(Q.device))
     else:
         staged = kernel == "staged"
         with torch.cuda.device(Q.device):
-            nws = L.lib().dsa_sparse_attn_workspace_bytes(int(staged), L.dtype_code(dt), B, T, HQ,
-                                                          DQ, DV, T)
+            nws = L.lib().dsa_sparse_attn_workspace_bytes(int(staged), code, B, T, HQ, DQ, DV, T)
         ws = torch.empty(max(nws, 0), device=Q.device, dtype=torch.uint8) if nws > 0 else None
         fn = (L.lib().dsa_sparse_attn_threshold_staged_ws if staged
               else L.lib().dsa_sparse_attn_threshold_ws)
@@ -189,7 +208,7 @@ def dsa_split_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
         _, mask = topk_threshold_mask(scores, k)
         return sparse_attention_from_mask(mask, Q, K, V)
     thr = topk_threshold(scores, k, causal=True)
-    return sparse_attention_hip(scores, thr, Q, K, V)
+    return sparse_attention_hip(scores, thr, Q, K, V, top_k=k)
 
 
 def dsa_fused_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:

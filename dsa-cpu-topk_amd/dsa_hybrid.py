@@ -107,7 +107,7 @@ def _finish(ctx: HybridContext, blocks, k: int, causal: bool, nthreads: int, Q, 
         ev.synchronize()
         _host_select(ctx, r0, r1, k, causal, nthreads)
     ctx.thr_gpu.copy_(ctx.thr_cpu, non_blocking=True)
-    return sparse_attention_hip(ctx.scores_gpu, ctx.thr_gpu, Q, K, V, out=out)
+    return sparse_attention_hip(ctx.scores_gpu, ctx.thr_gpu, Q, K, V, out=out, top_k=k)
 
 
 def dsa_hybrid_cpu_topk(q_idx, k_idx, w_idx, Q, K, V, top_k: int,

@@ -92,7 +92,7 @@ class DSAStreamPipeline:
             self.attention_stream.wait_event(ready)
             topk_threshold_into(self.scores[slot], self.k, self.thr[slot], causal=True)
             out = torch.empty(B, T, Q.shape[2], V.shape[3], device=self.device)
-            sparse_attention_hip(self.scores[slot], self.thr[slot], Q, K, V, out=out)
+            sparse_attention_hip(self.scores[slot], self.thr[slot], Q, K, V, out=out, top_k=self.k)
             done = torch.cuda.Event()
             done.record(self.attention_stream)
         self._done[slot] = done
@@ -167,7 +167,7 @@ class DSAStreamGraph:
             q_idx, k_idx, w_idx, Q, K, V = bt
             indexer_scores_hip(q_idx, k_idx, w_idx, write_upper=False, out=self.scores)
             topk_threshold_into(self.scores, self.k, self.thr, causal=True)
-            sparse_attention_hip(self.scores, self.thr, Q, K, V, out=out)
+            sparse_attention_hip(self.scores, self.thr, Q, K, V, out=out, top_k=self.k)
 
     def replay(self) -> None:
         self.graph.replay()
@@ -206,7 +206,7 @@ def dsa_attention_stream(batches, top_k: int, depth: int | None = None):
         assert scores.shape == (B, T, T), "dsa_attention_stream: batches must share one shape"
         indexer_scores_hip(q_idx, k_idx, w_idx, write_upper=False, out=scores)
         topk_threshold_into(scores, k, thr, causal=True)
-        outs.append(sparse_attention_hip(scores, thr, Q, K, V))
+        outs.append(sparse_attention_hip(scores, thr, Q, K, V, top_k=k))
     if dev is not None:
         torch.cuda.synchronize(dev)
     return outs

@@ -336,6 +336,41 @@ int dsa_sparse_attn_mask_noalloc(const float* scores, int64_t ld, const float* t
 int dsa_sparse_attn_uses_mask(int dtype, int64_t T, int HQ, int DQ, int DV);
 
 /*
+ * The attention of dsa_sparse_attn_threshold (same sel and O, fp32
+ * probabilities and sums for every input type) computed densely on MFMA
+ * tiles under a selection bitmask: 128 queries of one head share every K/V
+ * tile, fp32 operands and the probabilities are split into 16-bit pieces
+ * whose products are exact.  Tiles the pieces cannot carry (non-finite K, V or
+ * results, values beyond 2^+-60) are gathered per query instead, decided on the
+ * device.
+ *   dsa_sparse_attn_dense_workspace_bytes: the workspace it needs (device
+ *     memory of the stream's device, 16-byte aligned, used by no other work
+ *     until the launches complete, contents on entry free); 0 for shapes it
+ *     does not cover.  Pure function of the arguments.
+ *   dsa_sparse_attn_gather: the per-query gathers alone, whatever kernel
+ *     dsa_sparse_attn_threshold would take.
+ *   dsa_sparse_attn_pick: the entry expected to be fastest -- 0
+ *     dsa_sparse_attn_threshold_ws, 1 dsa_sparse_attn_dense, 2
+ *     dsa_sparse_attn_gather; top_k: keys a query is expected to select, 0 if
+ *     unknown.  Needs the device (its compute-unit count).
+ * Constraints (dense): DQ = DV in {64, 128}; T <= 2^20; and those of
+ *   dsa_sparse_attn_threshold.  A workspace below the needed size is refused
+ *   (DSA_EINVAL).
+ * Replaces: _sparse_attn_kernel + sparse_attention_with_threshold_triton,
+ *           reference dsa_attention.py:234-324.
+ */
+int64_t dsa_sparse_attn_dense_workspace_bytes(int dtype, int64_t B, int64_t T, int HQ, int DQ,
+                                              int DV);
+int dsa_sparse_attn_pick(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int64_t top_k);
+int dsa_sparse_attn_gather(const float* scores, int64_t ld, const float* thr, const void* Q,
+                           const void* K, const void* V, int dtype, int64_t B, int64_t T, int HQ,
+                           int DQ, int DV, float scale, float* out, void* stream);
+int dsa_sparse_attn_dense(const float* scores, int64_t ld, const float* thr, const void* Q,
+                          const void* K, const void* V, int dtype, int64_t B, int64_t T, int HQ,
+                          int DQ, int DV, float scale, float* out, void* workspace,
+                          int64_t workspace_bytes, void* stream);
+
+/*
  * Fused DSA forward for T <= 2048: indexer -> per-row radix select ->
  * sparse attention in one kernel; the score rows live in LDS only.
  * Same result as dsa_indexer_scores + dsa_topk_threshold(k = min(top_k,T),

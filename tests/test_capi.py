@@ -423,3 +423,35 @@ def test_staged_entry_score_limit():
     a = list(ok)
     a[7] = 0
     assert f(*a) == L.DSA_OK
+
+
+def test_sparse_attn_dense_entries_check_arguments():
+    """dsa_sparse_attn_dense and dsa_sparse_attn_gather validate before any
+    HIP call; the workspace query covers DQ = DV in {64, 128} only."""
+    f = L.lib().dsa_sparse_attn_dense
+    ws = L.lib().dsa_sparse_attn_dense_workspace_bytes
+    need = ws(L.DSA_F32, 2, 512, 8, 64, 64)
+    assert need > 2 * 512 * 8 * 8 + 4 * 2 * 512 * 8 * 64 * 2
+    assert 0 < ws(L.DSA_BF16, 2, 512, 8, 64, 64) < need
+    for bad in ((L.DSA_F32, 2, 512, 8, 32, 32), (L.DSA_F32, 2, 512, 8, 64, 128),
+                (L.DSA_FP8, 2, 512, 8, 64, 64), (L.DSA_F32, 0, 512, 8, 64, 64),
+                (L.DSA_F32, 1, (1 << 20) + 1, 1, 64, 64)):
+        assert ws(*bad) == 0
+
+    def call(fn, extra, **kw):
+        a = [FAKE, 512, FAKE, FAKE, FAKE, FAKE, L.DSA_F32, 2, 512, 8, 64, 64, 0.125, FAKE, *extra, None]
+        for i, v in kw.items():
+            a[int(i[1:])] = v
+        return _rc(fn, *a)
+
+    assert call(f, (FAKE, need - 1))[0] == L.DSA_EINVAL
+    assert call(f, (None, need))[0] == L.DSA_EINVAL
+    assert call(f, (FAKE, -1))[0] == L.DSA_EINVAL
+    assert call(f, (FAKE, need), a10=32, a11=32)[0] == L.DSA_EUNSUPPORTED
+    assert call(f, (FAKE, need), a7=0)[0] == L.DSA_OK
+    g = L.lib().dsa_sparse_attn_gather
+    for fn, extra in ((f, (FAKE, need)), (g, ())):
+        assert call(fn, extra, a1=256)[0] == L.DSA_EINVAL           # ld < T
+        assert call(fn, extra, a12=float("nan"))[0] == L.DSA_EINVAL
+        assert call(fn, extra, a0=None)[0] == L.DSA_EINVAL
+        assert call(fn, extra, a9=3)[0] == L.DSA_EINVAL             # HQ not a power of two

@@ -1,0 +1,141 @@
+"""GPU: the dense MFMA attention with fp32 probabilities (kernel="dense") --
+tile edges, both block forms, non-finite and wide-range operands -- against
+the float64 oracle and the per-query gathers."""
+from __future__ import annotations
+
+import math
+
+import pytest
+import torch
+
+import _dsa_lib as L
+from dsa_attention import sparse_attention_hip
+from helpers import say
+from oracle import dsa_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+F32, BF, HF = torch.float32, torch.bfloat16, torch.float16
+
+
+def case(T, HQ, D, k, dtype, B=1, seed=0):
+    _, _, _, Q, K, V = O.make_inputs(B, T, 1, 1, HQ, D, D, dtype=dtype, seed0=seed)
+    g = torch.Generator().manual_seed(seed + 5)
+    s = torch.randn(B, T, T, generator=g)
+    s = torch.where(torch.rand(B, T, T, generator=g) < 0.1, 0.0, s)
+    masked = s.masked_fill(~torch.ones(T, T, dtype=torch.bool).tril(), -math.inf)
+    return s, O.topk_threshold(masked, min(k, T)), Q, K, V
+
+
+def bound(Q, K, V, T):
+    """Elementwise bound on the difference of two fp32 evaluations: a logit
+    is off by at most 16 * 2^-24 |q||k| scale (products to 2^-22, sums) and
+    exp2's argument by 2^-24 of its size (<= 64), a probability by that
+    relative to itself, numerator and normaliser both; the sums over the
+    keys add (T/32 + 8) * 2^-24."""
+    D = Q.shape[-1]
+    lg = float(Q.double().norm(dim=-1).max() * K.double().norm(dim=-1).max()) / math.sqrt(D)
+    return (2 * (16 * lg + 64) + T / 32 + 8) * 2.0 ** -24 * float(V.double().abs().max())
+
+
+@pytest.mark.parametrize("dtype", [F32, BF, HF])
+@pytest.mark.parametrize("T,HQ,D,k", [(1, 1, 64, 1), (31, 2, 128, 5), (63, 4, 64, 9), (64, 1, 128, 8),
+                                      (65, 8, 64, 64), (127, 2, 64, 20), (128, 2, 128, 30),
+                                      (129, 4, 64, 129), (200, 1, 128, 16), (257, 2, 64, 3),
+                                      (333, 16, 128, 40), (333, 32, 64, 70)])
+def test_dense_edges(dev, T, HQ, D, k, dtype):
+    """Remainders of the key and query tiles, one to several tiles, every key
+    selected, rows that no wave's tile holds; two key groups per block."""
+    say(f"dense T={T} HQ={HQ} D={D} k={k} {dtype}")
+    s, thr, Q, K, V = case(T, HQ, D, k, dtype, B=2, seed=T)
+    out = sparse_attention_hip(*(x.to(dev) for x in (s, thr, Q, K, V)), kernel="dense").cpu()
+    want = O.sparse_attn_threshold(s, thr, Q, K, V)
+    err = float((out.double() - want).abs().max())
+    assert err <= bound(Q, K, V, T), err
+
+
+@pytest.mark.parametrize("dtype,HQ,D", [(F32, 16, 64), (F32, 8, 128), (BF, 16, 64), (HF, 8, 128)])
+def test_dense_many_blocks(dev, dtype, HQ, D):
+    """More than two blocks per compute unit: one key group per block.  All
+    rows against the gathers, which the oracle tests cover."""
+    T, k = 2200, 150
+    B = 2 * 256 * 128 // (HQ * T) + 1
+    say(f"dense many blocks B={B} T={T} HQ={HQ} D={D} {dtype}")
+    g = torch.Generator(device=dev).manual_seed(3)
+    s = torch.randn(B, T, T, generator=g, device=dev)
+    tril = torch.ones(T, T, dtype=torch.bool, device=dev).tril()
+    thr = s.masked_fill(~tril, -math.inf).topk(k, dim=-1).values[..., -1:].contiguous()
+    Q, K, V = (torch.randn(B, T, HQ, D, generator=g, device=dev).to(dtype) for _ in range(3))
+    a = sparse_attention_hip(s, thr, Q, K, V, kernel="dense")
+    b = sparse_attention_hip(s, thr, Q, K, V, kernel="gather")
+    torch.cuda.synchronize()
+    assert float((a - b).abs().max()) <= 2 * bound(Q, K, V, T)
+
+
+@pytest.mark.parametrize("dtype,D", [(F32, 64), (F32, 128), (BF, 64), (HF, 128)])
+def test_dense_nonfinite(dev, dtype, D):
+    """inf and NaN in Q, K and V, selected and not, and rows that select
+    nothing: what the gathers give, NaN for NaN."""
+    T, HQ, k = 400, 2, 12
+    s, thr, Q, K, V = case(T, HQ, D, k, dtype, B=2, seed=9)
+    thr[0, 7], thr[0, 300] = math.nan, math.inf
+    for x, at, v in ((K, (0, 70, 0, 3), math.inf), (K, (0, 71, 1, 0), -math.inf),
+                     (K, (0, 90, 0, 5), math.nan), (V, (0, 150, 1, 2), math.inf),
+                     (V, (0, 151, 0, 9), math.nan), (Q, (0, 200, 0, 1), math.inf),
+                     (Q, (0, 201, 1, 1), math.nan)):
+        x[at] = v
+    args = tuple(x.to(dev) for x in (s, thr, Q, K, V))
+    a = sparse_attention_hip(*args, kernel="dense").cpu()
+    b = sparse_attention_hip(*args, kernel="gather").cpu()
+    assert torch.equal(torch.isnan(a), torch.isnan(b))
+    assert torch.equal(torch.isinf(a), torch.isinf(b))
+    fin = torch.isfinite(b)
+    clean = [torch.nan_to_num(x.float(), 0, 0, 0) for x in (Q, K, V)]
+    assert float((a - b)[fin].abs().max()) <= 2 * bound(*clean, T)
+    assert bool(torch.isfinite(a[1]).all())
+
+
+@pytest.mark.parametrize("span", [4, 9, 30, 70])
+def test_dense_fp32_ranges(dev, span):
+    """fp32 operands of very different magnitude: V tiles on one, on two
+    neighbouring and on far-apart scales (the last gathered), Q and K rows
+    scaled against each other, rows of zeros, and rows beyond the scales."""
+    T, HQ, D, k = 300, 2, 64, 25
+    s, thr, Q, K, V = case(T, HQ, D, k, F32, seed=span)
+    say(f"dense ranges span={span}")
+    V = V.clone()
+    V[:, 100:200] *= 2.0 ** -span
+    V[:, 10] = 0.0
+    K = K.clone()
+    K[:, 130:140] *= 2.0 ** -span
+    K[:, 20] = 0.0
+    Q = Q * 2.0 ** min(span, 40)
+    K = K * 2.0 ** -min(span, 40)
+    Q[:, 33] = 0.0
+    out = sparse_attention_hip(*(x.to(dev) for x in (s, thr, Q, K, V)), kernel="dense").cpu()
+    want = O.sparse_attn_threshold(s, thr, Q, K, V)
+    # rows that selected keys of 100..199 only would need the bound of those
+    assert float((out.double() - want).abs().max()) <= bound(Q, K, V, T)
+
+
+def test_dense_arguments(dev):
+    x = torch.zeros(1, 64, 2, 32, device=dev)
+    s, t = torch.zeros(1, 64, 64, device=dev), torch.zeros(1, 64, 1, device=dev)
+    with pytest.raises(L.DSAUnsupported):
+        sparse_attention_hip(s, t, x, x, x, kernel="dense")
+
+
+@pytest.mark.parametrize("B,T,k,HQ,D,dtype", [(8, 1024, 64, 8, 64, F32), (2, 2048, 256, 16, 128, HF)])
+def test_split_forward_takes_it(dev, B, T, k, HQ, D, dtype):
+    """The split forward at shapes the rule gives to the dense kernel equals
+    its stages run apart."""
+    from dsa_attention import dsa_split_hip
+    from lightning_indexer import indexer_scores_hip
+    from topk_threshold import topk_threshold
+
+    assert L.lib().dsa_sparse_attn_pick(L.dtype_code(dtype), B, T, HQ, D, D, k) == 1
+    ins = tuple(x.to(dev) for x in O.make_inputs(B, T, 4, 32, HQ, D, D, dtype=dtype))
+    sc = indexer_scores_hip(*ins[:3], write_upper=False)
+    thr = topk_threshold(sc, k, causal=True)
+    want = sparse_attention_hip(sc, thr, *ins[3:], kernel="dense")
+    assert torch.equal(dsa_split_hip(*ins, k), want)
