@@ -13,6 +13,7 @@ Python asserts raise; positive status (HIP runtime failure) -> RuntimeError.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 
@@ -60,6 +61,10 @@ _SIGNATURES = {
                                _I),
     "dsa_sparse_attn_dense": ([_P, _I64, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _F, _P, _P,
                                _I64, _P], _I),
+    "dsa_forward_uses_split": ([_I, _I64, _I64, _I, _I, _I, _I, _I, _I], _I),
+    "dsa_split_workspace_bytes": ([_I, _I64, _I64, _I, _I, _I, _I], _I64),
+    "dsa_split_forward": ([_P, _P, _P, _I, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _I, _I, _I, _F,
+                           _P, _P, _I64, _P], _I),
     "dsa_fused_forward": ([_P, _P, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _I, _I, _I, _F,
                            _P, _P], _I),
     "dsa_selection_mask": ([_P, _I64, _P, _I64, _I64, _P, _I64, _P], _I),
@@ -127,16 +132,15 @@ def check(rc: int, what: str) -> None:
     raise RuntimeError(f"{what}: {msg}")
 
 
+_DTYPE_CODES = {torch.float32: DSA_F32, torch.bfloat16: DSA_BF16, torch.float16: DSA_F16,
+                torch.float8_e4m3fn: DSA_FP8}
+
+
 def dtype_code(t: torch.dtype) -> int:
-    if t == torch.float32:
-        return DSA_F32
-    if t == torch.bfloat16:
-        return DSA_BF16
-    if t == torch.float16:
-        return DSA_F16
-    if t == torch.float8_e4m3fn:
-        return DSA_FP8
-    raise AssertionError(f"unsupported dtype {t}")
+    code = _DTYPE_CODES.get(t)
+    if code is None:
+        raise AssertionError(f"unsupported dtype {t}")
+    return code
 
 
 def common_dtype(*xs: torch.Tensor) -> torch.dtype:
@@ -144,9 +148,12 @@ def common_dtype(*xs: torch.Tensor) -> torch.dtype:
     their shared dtype if it is fp32/bf16/fp16, otherwise fp32 (the reference
     upcasts every load to fp32: dsa_attention.py:125-129)."""
     d = xs[0].dtype
-    if all(x.dtype == d for x in xs) and d in (torch.float32, torch.bfloat16, torch.float16):
-        return d
-    return torch.float32
+    if d is not torch.float32 and d is not torch.bfloat16 and d is not torch.float16:
+        return torch.float32
+    for x in xs:
+        if x.dtype is not d:
+            return torch.float32
+    return d
 
 
 def prep(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
@@ -159,8 +166,33 @@ def prep(x: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     return x
 
 
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """`with` block in which `device` is the current GPU (nothing to enter
+    when it already is, or when no index is given)."""
+    if device.index is None or device.index == torch.cuda.current_device():
+        return _NO_SWITCH
+    return torch.cuda.device(device)
+
+
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream of `device`, as the pointer the C entries take."""
+    i = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
+
+
+def ready_ptrs(dtype: torch.dtype, xs) -> list | None:
+    """The data pointers of `xs`, or None if one of them is not what `prep`
+    would return unchanged (dtype, contiguous, 16-byte aligned)."""
+    ptrs = []
+    for x in xs:
+        p = x.data_ptr()
+        if x.dtype is not dtype or p & 15 or not x.is_contiguous():
+            return None
+        ptrs.append(p)
+    return ptrs
 
 
 def require_gpu(*xs: torch.Tensor) -> None:

@@ -79,6 +79,26 @@ int check_attn(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, const vo
   return DSA_OK;
 }
 
+// Q, K, V and out of the bitmask tile kernel (any HQ from 1 to 1024).
+int check_tile_attn(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, const void* Q,
+                    const void* K, const void* V, const float* out, const char* who) {
+  if (!dtype_ok(dtype)) return fail(DSA_EINVAL, "%s: unknown dtype %d", who, dtype);
+  if (B < 0 || T < 0) return fail(DSA_EINVAL, "%s: negative size", who);
+  if (T > kMaxElems) return fail(DSA_EINVAL, "%s: T=%lld too large", who, (long long)T);
+  if (HQ < 1 || HQ > 1024) return fail(DSA_EINVAL, "%s: HQ=%d outside [1,1024]", who, HQ);
+  if (dtype == DSA_F32 || DQ != DV || (DQ != 64 && DQ != 128))
+    return fail(DSA_EUNSUPPORTED, "%s: needs bf16/fp16 and DQ = DV in {64,128} (dtype %d DQ=%d DV=%d)", who, dtype, DQ, DV);
+  if (T * HQ * static_cast<int64_t>(DQ) * 2 > (int64_t{1} << 32) - 1)
+    return fail(DSA_EINVAL, "%s: T*HQ*D = %lld 16-bit elements must be < 4 GiB", who,
+                (long long)(T * HQ * static_cast<int64_t>(DQ)));
+  if (B * T == 0) return DSA_OK;
+  if (!Q || !K || !V || !out) return fail(DSA_EINVAL, "%s: null pointer", who);
+  if (!aligned16(Q) || !aligned16(K) || !aligned16(V) || !aligned16(out))
+    return fail(DSA_EINVAL, "%s: Q/K/V/out must be 16-byte aligned", who);
+  if (B * T * HQ * static_cast<int64_t>(DQ) > (int64_t{1} << 40)) return fail(DSA_EINVAL, "%s: Q too large", who);
+  return DSA_OK;
+}
+
 }  // namespace
 
 extern "C" {
@@ -252,26 +272,16 @@ int dsa_selection_mask(const float* scores, int64_t ld, const float* thr, int64_
 int dsa_sparse_attn_mask(const uint64_t* mask, int64_t ldm, const void* Q, const void* K,
                          const void* V, int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV,
                          float scale, float* out, void* stream) {
-  if (!dtype_ok(dtype)) return fail(DSA_EINVAL, "sparse_attn_mask: unknown dtype %d", dtype);
-  if (B < 0 || T < 0) return fail(DSA_EINVAL, "sparse_attn_mask: negative size");
-  if (T > kMaxElems) return fail(DSA_EINVAL, "sparse_attn_mask: T=%lld too large", (long long)T);
-  if (HQ < 1 || HQ > 1024) return fail(DSA_EINVAL, "sparse_attn_mask: HQ=%d outside [1,1024]", HQ);
+  const int rc = check_tile_attn(dtype, B, T, HQ, DQ, DV, Q, K, V, out, "sparse_attn_mask");
+  if (rc != DSA_OK) return rc;
   if (!std::isfinite(scale)) return fail(DSA_EINVAL, "sparse_attn_mask: scale must be finite");
-  if (dtype == DSA_F32 || dtype == DSA_FP8 || DQ != DV || (DQ != 64 && DQ != 128))
-    return fail(DSA_EUNSUPPORTED, "sparse_attn_mask: needs bf16/fp16 and DQ = DV in {64,128} (dtype %d DQ=%d DV=%d)", dtype, DQ, DV);
   if (ldm < (T + 63) / 64)
     return fail(DSA_EINVAL, "sparse_attn_mask: ldm=%lld < ceil(T/64)=%lld", (long long)ldm, (long long)((T + 63) / 64));
   // 128 mask rows are addressed with 32-bit byte offsets
   if (ldm > (int64_t{1} << 21) - 1) return fail(DSA_EINVAL, "sparse_attn_mask: ldm=%lld too large", (long long)ldm);
-  if (T * HQ * static_cast<int64_t>(DQ) * 2 > (int64_t{1} << 32) - 1)
-    return fail(DSA_EINVAL, "sparse_attn_mask: T*HQ*D = %lld 16-bit elements must be < 4 GiB",
-                (long long)(T * HQ * static_cast<int64_t>(DQ)));
   if (B * T == 0) return DSA_OK;
-  if (!mask || !Q || !K || !V || !out) return fail(DSA_EINVAL, "sparse_attn_mask: null pointer");
+  if (!mask) return fail(DSA_EINVAL, "sparse_attn_mask: null pointer");
   if ((reinterpret_cast<uintptr_t>(mask) & 7u) != 0) return fail(DSA_EINVAL, "sparse_attn_mask: mask must be 8-byte aligned");
-  if (!aligned16(Q) || !aligned16(K) || !aligned16(V) || !aligned16(out))
-    return fail(DSA_EINVAL, "sparse_attn_mask: Q/K/V/out must be 16-byte aligned");
-  if (B * T * HQ * static_cast<int64_t>(DQ) > (int64_t{1} << 40)) return fail(DSA_EINVAL, "sparse_attn_mask: Q too large");
   return hip_status(dsa::launch_tile_attn_mask(mask, ldm, Q, K, V, dtype, B, T, HQ, DQ, scale, out,
                                                static_cast<hipStream_t>(stream)),
                     "dsa_sparse_attn_mask");
@@ -384,6 +394,43 @@ int dsa_sparse_attn_dense(const float* scores, int64_t ld, const float* thr, con
   return hip_status(dsa::launch_dense_attn(scores, ld, thr, Q, K, V, dtype, B, T, HQ, DQ, scale, out,
                                            workspace, static_cast<hipStream_t>(stream)),
                     "dsa_sparse_attn_dense");
+}
+
+int64_t dsa_split_workspace_bytes(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int top_k) {
+  if (!dtype_ok(dtype) || B <= 0 || T <= 0 || T > kMaxElems || B * T > kMaxElems || top_k < 1) return 0;
+  if (!dsa::sparse_attn_uses_tiles(dtype, T, HQ, DQ, DV) && !dsa::sparse_attn_supported(dtype, HQ, DQ, DV))
+    return 0;
+  return dsa::split_workspace(dtype, B, T, HQ, DQ, DV, top_k < T ? top_k : T);
+}
+
+int dsa_forward_uses_split(int dtype, int64_t B, int64_t T, int HI, int DI, int HQ, int DQ, int DV,
+                           int top_k) {
+  if (!dtype_ok(dtype) || B <= 0 || T <= 0 || HI < 1 || DI < 1 || HQ < 1 || DQ < 1 || DV < 1 || top_k < 1)
+    return 0;
+  return T > dsa::kFusedMaxT || dsa::forward_uses_split(dtype, B, T, HI, DI, HQ, DQ, DV, top_k) ? 1 : 0;
+}
+
+int dsa_split_forward(const void* q_idx, const void* k_idx, const void* w_idx, int idx_dtype,
+                      const void* Q, const void* K, const void* V, int dtype, int64_t B, int64_t T,
+                      int HI, int DI, int HQ, int DQ, int DV, int top_k, float scale, float* out,
+                      void* workspace, int64_t workspace_bytes, void* stream) {
+  if (top_k < 1) return fail(DSA_EINVAL, "split: top_k must be >= 1 (got %d)", top_k);
+  int rc = check_indexer(q_idx, k_idx, w_idx, idx_dtype, B, T, HI, DI, static_cast<float*>(workspace), T);
+  if (rc != DSA_OK) return rc;
+  rc = dsa::sparse_attn_uses_tiles(dtype, T, HQ, DQ, DV)
+           ? check_tile_attn(dtype, B, T, HQ, DQ, DV, Q, K, V, out, "split")
+           : check_attn(dtype, B, T, HQ, DQ, DV, Q, K, V, out, "split");
+  if (rc != DSA_OK) return rc;
+  if (!std::isfinite(scale)) return fail(DSA_EINVAL, "split: scale must be finite");
+  if (B * T == 0) return DSA_OK;
+  if (B * T > kMaxElems) return fail(DSA_EINVAL, "split: B*T=%lld rows >= 2^31", (long long)(B * T));
+  const int k = top_k < T ? top_k : static_cast<int>(T);
+  const int64_t need = dsa::split_workspace(dtype, B, T, HQ, DQ, DV, k);
+  if (!aligned16(workspace) || workspace_bytes < need)
+    return fail(DSA_EINVAL, "split: needs a 16-byte aligned workspace of %lld bytes (got %lld)", (long long)need, (long long)workspace_bytes);
+  return hip_status(dsa::launch_split(q_idx, k_idx, w_idx, idx_dtype, Q, K, V, dtype, B, T, HI, DI, HQ,
+                                      DQ, DV, k, scale, out, workspace, static_cast<hipStream_t>(stream)),
+                    "dsa_split_forward");
 }
 
 int dsa_fused_forward(const void* q_idx, const void* k_idx, const void* w_idx, const void* Q,

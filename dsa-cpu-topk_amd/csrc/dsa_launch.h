@@ -138,6 +138,19 @@ hipError_t launch_dense_attn(const float* scores, int64_t ld, const float* thr, 
                              const void* K, const void* V, int dtype, int64_t B, int64_t T, int HQ,
                              int D, float scale, float* out, void* ws, hipStream_t stream);
 
+// The split forward (indexer, select of the k-th largest, attention) on one
+// stream, over a 16-byte aligned workspace of split_workspace bytes.  idx_dtype
+// is the indexer inputs' type (3: fp8 with fp32 weights), dtype Q, K and V's.
+int64_t split_workspace(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int64_t k);
+hipError_t launch_split(const void* qi, const void* ki, const void* wi, int idx_dtype, const void* Q,
+                        const void* K, const void* V, int dtype, int64_t B, int64_t T, int HI, int DI,
+                        int HQ, int DQ, int DV, int k, float scale, float* out, void* ws,
+                        hipStream_t stream);
+
+// Whether launch_split is expected to be faster than launch_fused.
+bool forward_uses_split(int dtype, int64_t B, int64_t T, int HI, int DI, int HQ, int DQ, int DV,
+                        int64_t k);
+
 // Fused forward for T <= kFusedMaxT.
 constexpr int64_t kFusedMaxT = 2048;
 hipError_t launch_fused(const void* qi, const void* ki, const void* wi, const void* Q,

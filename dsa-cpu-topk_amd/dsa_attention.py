@@ -25,8 +25,8 @@ import math
 import torch
 
 import _dsa_lib as L
-from lightning_indexer import indexer_scores_hip, indexer_scores_torch
-from topk_threshold import topk_threshold, topk_threshold_mask
+from lightning_indexer import indexer_scores_hip, indexer_scores_torch  # noqa: F401
+from topk_threshold import topk_threshold, topk_threshold_mask  # noqa: F401
 
 
 # ---------------------------------------------------------------------------
@@ -118,7 +118,7 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
         return _sparse_attention_mask(scores, thr, Q, K, V, out)
     code = L.dtype_code(dt)
     if kernel is None or (kernel == "staged" and T >= 3072):
-        with torch.cuda.device(Q.device):
+        with L.on_device(Q.device):
             kernel = {0: kernel, 1: "dense", 2: "gather"}[
                 L.lib().dsa_sparse_attn_pick(code, B, T, HQ, DQ, DV, int(top_k))]
     if kernel == "dense":
@@ -137,7 +137,7 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
         rc = L.lib().dsa_sparse_attn_gather(*args, L.stream_ptr(Q.device))
     else:
         staged = kernel == "staged"
-        with torch.cuda.device(Q.device):
+        with L.on_device(Q.device):
             nws = L.lib().dsa_sparse_attn_workspace_bytes(int(staged), code, B, T, HQ, DQ, DV, T)
         ws = torch.empty(max(nws, 0), device=Q.device, dtype=torch.uint8) if nws > 0 else None
         fn = (L.lib().dsa_sparse_attn_threshold_staged_ws if staged
@@ -194,21 +194,41 @@ def _sparse_attention_mask(scores, thr, Q, K, V, out):
 
 def dsa_split_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
     """Split forward for any T: indexer (causal half only) -> causal
-    radix-select of the min(top_k,T)-th largest -> sparse attention.  Where
-    the attention runs on tiles from a selection bitmask, the select writes
-    that bitmask in its own pass over the scores (topk_threshold_mask): the
-    same output as the three steps apart, bit for bit."""
+    radix-select of the min(top_k,T)-th largest -> sparse attention, as one
+    call of the library (dsa_split_forward) over one workspace.  Where the
+    attention runs on tiles from a selection bitmask, the select writes that
+    bitmask in its own pass over the scores (topk_threshold_mask).  The same
+    output as the three steps apart, bit for bit."""
+    L.require_gpu(q_idx, k_idx, w_idx, Q, K, V)
     B, T, HQ, DQ = Q.shape
     DV = V.shape[-1]
-    scores = indexer_scores_hip(q_idx, k_idx, w_idx, write_upper=False)
-    k = min(top_k, T)
-    L.require_gpu(Q, K, V)
-    dt = L.common_dtype(Q, K, V)
-    if L.lib().dsa_sparse_attn_uses_mask(L.dtype_code(dt), T, HQ, DQ, DV):
-        _, mask = topk_threshold_mask(scores, k)
-        return sparse_attention_from_mask(mask, Q, K, V)
-    thr = topk_threshold(scores, k, causal=True)
-    return sparse_attention_hip(scores, thr, Q, K, V, top_k=k)
+    _, _, HI, DI = q_idx.shape
+    assert q_idx.shape == (B, T, HI, DI), f"q shape {tuple(q_idx.shape)} != {(B, T, HI, DI)}"
+    assert k_idx.shape == (B, T, DI), f"k shape {tuple(k_idx.shape)} != {(B, T, DI)}"
+    assert w_idx.shape == (B, T, HI), f"w shape {tuple(w_idx.shape)} != {(B, T, HI)}"
+    assert K.shape == (B, T, HQ, DQ) and V.shape == (B, T, HQ, DV), "K/V shape"
+    k = min(int(top_k), T)
+    if k <= 0:
+        raise RuntimeError("k must be > 0")
+    f8 = torch.float8_e4m3fn
+    if q_idx.dtype == f8 and k_idx.dtype == f8:
+        it = f8
+        q_idx, k_idx, w_idx = L.prep(q_idx, f8), L.prep(k_idx, f8), L.prep(w_idx, torch.float32)
+    else:
+        it = L.common_dtype(q_idx, k_idx, w_idx)
+        q_idx, k_idx, w_idx = L.prep(q_idx, it), L.prep(k_idx, it), L.prep(w_idx, it)
+    dt, Q, K, V = _attn_inputs(Q, K, V)
+    code = L.dtype_code(dt)
+    out = torch.empty(B, T, HQ, DV, device=Q.device, dtype=torch.float32)
+    with L.on_device(Q.device):
+        nws = L.lib().dsa_split_workspace_bytes(code, B, T, HQ, DQ, DV, k)
+        ws = torch.empty(max(nws, 16), device=Q.device, dtype=torch.uint8)
+        rc = L.lib().dsa_split_forward(
+            q_idx.data_ptr(), k_idx.data_ptr(), w_idx.data_ptr(), L.dtype_code(it), Q.data_ptr(),
+            K.data_ptr(), V.data_ptr(), code, B, T, HI, DI, HQ, DQ, DV, k, 1.0 / math.sqrt(DQ),
+            out.data_ptr(), ws.data_ptr(), nws, L.stream_ptr(Q.device))
+    L.check(rc, "dsa_split")
+    return out
 
 
 def dsa_fused_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
@@ -220,21 +240,41 @@ def dsa_fused_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
     DV = V.shape[-1]
     assert k_idx.shape == (B, T, DI) and w_idx.shape == (B, T, HI), "indexer input shapes"
     assert K.shape == (B, T, HQ, DQ) and V.shape == (B, T, HQ, DV), "K/V shapes"
-    dt = L.common_dtype(q_idx, k_idx, w_idx, Q, K, V)
-    q_idx, k_idx, w_idx, Q, K, V = (L.prep(x, dt) for x in (q_idx, k_idx, w_idx, Q, K, V))
-    out = torch.empty(B, T, HQ, DV, device=Q.device, dtype=torch.float32)
-    rc = L.lib().dsa_fused_forward(
-        q_idx.data_ptr(), k_idx.data_ptr(), w_idx.data_ptr(), Q.data_ptr(), K.data_ptr(),
-        V.data_ptr(), L.dtype_code(dt), B, T, HI, DI, HQ, DQ, DV, int(top_k),
-        1.0 / math.sqrt(DQ), out.data_ptr(), L.stream_ptr(Q.device))
-    L.check(rc, "dsa_fused")
+    xs = (q_idx, k_idx, w_idx, Q, K, V)
+    dt = L.common_dtype(*xs)
+    ptrs = L.ready_ptrs(dt, xs)
+    if ptrs is None:
+        xs = tuple(L.prep(x, dt) for x in xs)
+        ptrs = [x.data_ptr() for x in xs]
+    device = Q.device
+    out = torch.empty((B, T, HQ, DV), device=device, dtype=torch.float32)
+    rc = L.lib().dsa_fused_forward(*ptrs, L.dtype_code(dt), B, T, HI, DI, HQ, DQ, DV, int(top_k),
+                                   1.0 / math.sqrt(DQ), out.data_ptr(), L.stream_ptr(device))
+    if rc != L.DSA_OK:
+        L.check(rc, "dsa_fused")
     return out
 
 
+def _split_is_faster(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> bool:
+    """The library's rule, for inputs of one type on one GPU (the fused kernel
+    takes mixed ones in fp32)."""
+    B, T, HQ, DQ = Q.shape
+    if T < 200 or (T < 512 and q_idx.shape[3] < 128):
+        return False  # never by that rule; such calls are launch-bound, so asking it counts
+    dt = Q.dtype
+    if not Q.is_cuda or dt not in (torch.float32, torch.bfloat16, torch.float16) or \
+            any(x.dtype != dt for x in (q_idx, k_idx, w_idx, K, V)):
+        return False
+    with L.on_device(Q.device):
+        return bool(L.lib().dsa_forward_uses_split(L.dtype_code(dt), B, T, q_idx.shape[2],
+                                                   q_idx.shape[3], HQ, DQ, V.shape[-1], int(top_k)))
+
+
 def dsa_forward_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
-    """Forward for any shape: the fused kernel where one exists (T <= 2048),
-    else the split kernels.  Both are gfx950 HIP; nothing runs on the CPU."""
-    if Q.shape[1] <= L.lib().dsa_fused_max_T():
+    """Forward for any shape: the fused kernel where one exists (T <= 2048)
+    and is not expected to be slower (dsa_forward_uses_split), else the split
+    kernels.  Both are gfx950 HIP; nothing runs on the CPU."""
+    if Q.shape[1] <= L.lib().dsa_fused_max_T() and not _split_is_faster(q_idx, k_idx, w_idx, Q, K, V, top_k):
         try:
             return dsa_fused_hip(q_idx, k_idx, w_idx, Q, K, V, top_k)
         except L.DSAUnsupported:
@@ -254,8 +294,8 @@ def dsa_attention_triton(q_idx, k_idx, w_idx, Q, K, V, top_k: int,
     B, T, HQ, DQ = Q.shape
     DV = V.shape[-1]
     HI, DI = q_idx.shape[2], q_idx.shape[3]
-    _assert_pow2([("T", T), ("HI", HI), ("DI", DI), ("HQ", HQ), ("DQ", DQ), ("DV", DV),
-                  ("BLOCK_S", BLOCK_S), ("top_k", top_k)])
+    _assert_pow2((("T", T), ("HI", HI), ("DI", DI), ("HQ", HQ), ("DQ", DQ), ("DV", DV),
+                  ("BLOCK_S", BLOCK_S), ("top_k", top_k)))
     assert T % BLOCK_S == 0, "T must be divisible by BLOCK_S"
     assert top_k <= T
     return dsa_forward_hip(q_idx, k_idx, w_idx, Q, K, V, top_k)

@@ -371,6 +371,27 @@ int dsa_sparse_attn_dense(const float* scores, int64_t ld, const float* thr, con
                           int64_t workspace_bytes, void* stream);
 
 /*
+ * The split DSA forward in one call: dsa_indexer_scores (write_upper 0), the
+ * causal select of the min(top_k, T)-th largest, and the attention entry that
+ * dsa_sparse_attn_pick names (the bitmask pair where dsa_sparse_attn_uses_mask
+ * is 1) -- the same kernels, so the same result bit for bit.
+ * dtype is Q, K and V's; idx_dtype q_idx, k_idx and w_idx's (DSA_FP8: fp32 w).
+ * workspace: device memory of the stream's device of
+ *   dsa_split_workspace_bytes (scores, thresholds, and what the attention
+ *   needs), 16-byte aligned, used by no other work until the launches complete.
+ * Replaces: dsa_attention_split_triton, reference dsa_attention.py:327-345.
+ */
+/* 1 where dsa_split_forward is expected to be faster than dsa_fused_forward
+ * (every T the latter refuses included).  Needs the device. */
+int dsa_forward_uses_split(int dtype, int64_t B, int64_t T, int HI, int DI, int HQ, int DQ, int DV,
+                           int top_k);
+int64_t dsa_split_workspace_bytes(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int top_k);
+int dsa_split_forward(const void* q_idx, const void* k_idx, const void* w_idx, int idx_dtype,
+                      const void* Q, const void* K, const void* V, int dtype, int64_t B, int64_t T,
+                      int HI, int DI, int HQ, int DQ, int DV, int top_k, float scale, float* out,
+                      void* workspace, int64_t workspace_bytes, void* stream);
+
+/*
  * Fused DSA forward for T <= 2048: indexer -> per-row radix select ->
  * sparse attention in one kernel; the score rows live in LDS only.
  * Same result as dsa_indexer_scores + dsa_topk_threshold(k = min(top_k,T),

@@ -455,3 +455,32 @@ def test_sparse_attn_dense_entries_check_arguments():
         assert call(fn, extra, a12=float("nan"))[0] == L.DSA_EINVAL
         assert call(fn, extra, a0=None)[0] == L.DSA_EINVAL
         assert call(fn, extra, a9=3)[0] == L.DSA_EINVAL             # HQ not a power of two
+
+
+def test_split_forward_entry_checks_arguments():
+    """dsa_split_forward validates its stages' arguments before any HIP call,
+    and takes what the stages take: any head count on the bitmask tiles."""
+    f = L.lib().dsa_split_forward
+    ws = L.lib().dsa_split_workspace_bytes
+    need = ws(L.DSA_F32, 2, 256, 4, 32, 32, 16)
+    assert need >= 2 * 256 * 256 * 4 + 2 * 256 * 4
+    assert ws(L.DSA_BF16, 1, 4096, 3, 128, 128, 64) >= 4096 * 4096 * 4 + 4096 * 64 * 8
+    assert ws(L.DSA_F32, 2, 256, 3, 32, 32, 16) == 0
+    base = [FAKE] * 3 + [L.DSA_F32] + [FAKE] * 3 + [L.DSA_F32, 2, 256, 4, 32, 4, 32, 32, 16, 0.1, FAKE,
+                                                    FAKE, need, None]
+
+    def call(**kw):
+        a = list(base)
+        for i, v in kw.items():
+            a[int(i[1:])] = v
+        return _rc(f, *a)[0]
+
+    assert call(a15=0) == L.DSA_EINVAL                       # top_k
+    assert call(a3=7) == L.DSA_EINVAL                        # indexer dtype
+    assert call(a11=24) == L.DSA_EUNSUPPORTED                # DI
+    assert call(a12=3) == L.DSA_EINVAL                       # HQ on the gathers
+    assert call(a16=float("inf")) == L.DSA_EINVAL
+    assert call(a19=need - 1) == L.DSA_EINVAL
+    assert call(a18=None) == L.DSA_EINVAL
+    assert call(a8=0) == L.DSA_OK
+    assert call(a7=L.DSA_BF16, a8=0, a9=4096, a12=3, a13=128, a14=128) == L.DSA_OK

@@ -139,3 +139,22 @@ def test_split_forward_takes_it(dev, B, T, k, HQ, D, dtype):
     thr = topk_threshold(sc, k, causal=True)
     want = sparse_attention_hip(sc, thr, *ins[3:], kernel="dense")
     assert torch.equal(dsa_split_hip(*ins, k), want)
+
+
+@pytest.mark.parametrize("B,T,k,HI,DI,HQ,D,dtype,split", [
+    (4, 512, 32, 64, 128, 4, 128, BF, 1), (2, 1024, 64, 8, 64, 8, 64, F32, 1),
+    (3, 950, 40, 16, 128, 4, 64, BF, 1), (2, 1500, 16, 4, 32, 4, 32, F32, 0),
+    (16, 512, 32, 4, 32, 4, 32, F32, 0), (2, 100, 9, 8, 128, 4, 32, BF, 0)])
+def test_forward_picks_split_or_fused(dev, B, T, k, HI, DI, HQ, D, dtype, split):
+    """Either side of the forward's rule gives the same attention: the other
+    form's output up to fp32 rounding, rows whose selection differs by a
+    near-tie apart (at most a handful)."""
+    import dsa_attention as DA
+
+    ins = tuple(x.to(dev) for x in O.make_inputs(B, T, HI, DI, HQ, D, D, dtype=dtype, seed0=T))
+    assert DA._split_is_faster(*ins, k) == bool(split)
+    got = DA.dsa_forward_hip(*ins, k)
+    assert torch.equal(got, (DA.dsa_split_hip if split else DA.dsa_fused_hip)(*ins, k))
+    other = (DA.dsa_fused_hip if split else DA.dsa_split_hip)(*ins, k)
+    off = (got - other).abs().amax(dim=(-1, -2)) > 2 * bound(*(x.cpu() for x in ins[3:]), T)
+    assert int(off.sum()) <= max(2, B * T // 1000)
