@@ -66,6 +66,27 @@ struct SelectArgs {
   int64_t ldm = 0;
 };
 
+// Four consecutive scores in one global_load_dwordx4, which needs 4-byte
+// alignment only: rows of any length and stride load 16 bytes per lane (at an
+// odd stride a wave's 1 KiB touches 9 cache lines instead of 8).  (Rows that were
+// not 16-byte granular took dword loads and the block kernels before: 96539
+// rows of 81, k = 12, 94.7 -> 36.1 us; 4000 of 20001, k = 300, 163 -> 59; 16384
+// of 3001, k = 128, 49.8 -> 40.7.)  The kernels' RAGGED instances do so; where
+// length, stride and base are 16-byte granular no row needs edge_row, whose
+// test alone costs the one-wave kernel 4% (config 2 standalone 174 -> 181 us).
+typedef float f32x4_u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ float4 load_f4(const char* p) {
+  const f32x4_u f = *reinterpret_cast<const f32x4_u*>(p);
+  return make_float4(f[0], f[1], f[2], f[3]);
+}
+// Whether the last group of four of a row (entries (nv - 1) & ~3 .. + 3) runs
+// past the end of the score array: the last row, and the rows before it that
+// end within three entries of that.  Such a row loads entry by entry, or
+// shifts its last group back inside.
+__device__ __forceinline__ bool edge_row(const SelectArgs& a, int64_t row, int64_t nv) {
+  return row * a.ld + ((nv + 3) & ~int64_t{3}) > (a.rows - 1) * a.ld + a.n;
+}
+
 // Row r of the 1-D causal order: q = r / nb (rows longest first), r % nb
 // the batch element; 32-bit arithmetic when the grid allows it (r is
 // wave-uniform, so this is scalar work).
@@ -382,7 +403,7 @@ __device__ __forceinline__ void load_keys4(const float* __restrict__ src, int64_
                                            int64_t nvalid, uint32_t (&kk)[4]) {
   if (VEC) {
     if (pos < nvalid) {
-      const float4 f = *reinterpret_cast<const float4*>(src + pos);
+      const float4 f = load_f4(reinterpret_cast<const char*>(src + pos));
       kk[0] = float_to_key(f.x);
       kk[1] = (pos + 1 < nvalid) ? float_to_key(f.y) : kKeyNone;
       kk[2] = (pos + 2 < nvalid) ? float_to_key(f.z) : kKeyNone;
@@ -402,7 +423,7 @@ __device__ __forceinline__ void load_keys4(const float* __restrict__ src, int64_
 // ---------------------------------------------------------------------------
 // Keys plus ~30 working registers fit 64 VGPRs up to V = 32: blocks of up to
 // 512 threads ask for 8 waves per SIMD there, so that four rows share a CU.
-template <int NT, int V, int P1, bool VEC>
+template <int NT, int V, int P1, bool RAGGED>
 __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_kernel(SelectArgs a) {
   static_assert(V % 4 == 0 && NT % kWave == 0 && NT <= 1024, "block shape");
   static_assert(P1 == 11 || P1 == 12, "first digit width");
@@ -446,13 +467,13 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_k
     // so each load takes one offset register against the scalar base
     const char* row_bytes = reinterpret_cast<const char*>(src);
     float raw[V];
-    if constexpr (VEC) {
+    if (!RAGGED || !edge_row(a, row, nvalid)) {
       const int last4 = (nv - 1) & ~3;
 #pragma unroll
       for (int j = 0; j < NCH; ++j) {
         const int pos = (j * NT + tid) * 4;
         const uint32_t off = static_cast<uint32_t>(min(pos, last4)) * 4u;
-        const float4 f = *reinterpret_cast<const float4*>(row_bytes + off);
+        const float4 f = load_f4(row_bytes + off);
         raw[4 * j] = f.x;
         raw[4 * j + 1] = f.y;
         raw[4 * j + 2] = f.z;
@@ -729,16 +750,18 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_k
 // Exact k-th largest key of the nvalid entries at src by three radix passes
 // that each re-read the row; krem is left at the rank of the wanted key among
 // the keys equal to it.  hist: kBins words of LDS.
-template <int NT, bool VEC>
+// edge: edge_row.
+template <int NT>
 __device__ __forceinline__ uint32_t stream_select(const float* __restrict__ src, int64_t nvalid,
                                                   int k, uint32_t* hist, uint32_t* wsum,
-                                                  uint32_t* info, uint32_t& krem) {
+                                                  uint32_t* info, uint32_t& krem, bool edge) {
   const int tid = threadIdx.x;
   const int64_t nchunks = (nvalid + 4 * NT - 1) / (4 * NT);
   auto visit = [&](auto&& f) {
     for (int64_t j = 0; j < nchunks; ++j) {
       uint32_t kk[4];
-      load_keys4<VEC>(src, (j * NT + tid) * 4, nvalid, kk);
+      if (edge) load_keys4<false>(src, (j * NT + tid) * 4, nvalid, kk);
+      else load_keys4<true>(src, (j * NT + tid) * 4, nvalid, kk);
 #pragma unroll
       for (int c = 0; c < 4; ++c) f(kk[c]);
     }
@@ -752,7 +775,7 @@ __device__ __forceinline__ uint32_t stream_select(const float* __restrict__ src,
   return found ? thr_key : prefix;
 }
 
-template <int NT, bool VEC>
+template <int NT>
 __global__ __launch_bounds__(NT) void topk_stream_kernel(SelectArgs a) {
   __shared__ uint32_t hist[kBins];
   __shared__ uint32_t wsum[NT / kWave];
@@ -768,13 +791,15 @@ __global__ __launch_bounds__(NT) void topk_stream_kernel(SelectArgs a) {
   }
   const float* __restrict__ src = a.scores + row * a.ld;
   uint32_t krem;
-  const uint32_t thr_key = stream_select<NT, VEC>(src, nvalid, k, hist, wsum, info, krem);
+  const bool edge = edge_row(a, row, nvalid);
+  const uint32_t thr_key = stream_select<NT>(src, nvalid, k, hist, wsum, info, krem, edge);
   if (tid == 0) a.thr[row] = key_to_float(thr_key);
   if (a.idx != nullptr) {
     const int64_t nchunks = (nvalid + 4 * NT - 1) / (4 * NT);
     emit_indices<NT>(a.idx + row * static_cast<int64_t>(k), nchunks, thr_key, krem, wsum,
                      [&](int64_t j, uint32_t(&kk)[4]) {
-                       load_keys4<VEC>(src, (j * NT + tid) * 4, nvalid, kk);
+                       if (edge) load_keys4<false>(src, (j * NT + tid) * 4, nvalid, kk);
+                       else load_keys4<true>(src, (j * NT + tid) * 4, nvalid, kk);
                      });
   }
 }
@@ -827,7 +852,7 @@ constexpr int kFinGather = 64;   // kept values of one finishing bin ranked in r
 // Eight blocks per CU (at most 64 VGPRs; the LDS columns allow eight): at
 // config 4 thresholds 101 -> 98 us, with indices 156 -> 152, the bitmask
 // 129 -> 127 against six (the bitmask and index forms spill a few SGPRs).
-template <int NT, bool IDX, bool MASK = false>
+template <int NT, bool RAGGED, bool IDX, bool MASK = false>
 __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
   // IDX: exactly-k indices; MASK: the selection bitmask (a.mask), both from
   // the row's flag bitmap below.
@@ -871,10 +896,23 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
   const int last4 = (nv - 1) & ~3;
   const int nc = (nv + CH - 1) / CH;
   const bool whole = nc <= 4;
-  // Clamped float4 load of chunk j: no load behind a branch.
+  // Clamped float4 load of chunk j: no load behind a branch.  An edge row is
+  // clamped to its last four entries instead (nv >= 4: longer rows only), and
+  // the thread whose group starts at last4 shifts what it got into place
+  // (settle) once it has arrived.
+  const bool edge = RAGGED && edge_row(a, row, nvalid);
+  const int lim4 = edge ? nv - 4 : last4;
   auto load4 = [&](int j) -> float4 {
-    const uint32_t off = static_cast<uint32_t>(min((j * NT + tid) * 4, last4)) * 4u;
-    return *reinterpret_cast<const float4*>(row_bytes + off);
+    const uint32_t off = static_cast<uint32_t>(min((j * NT + tid) * 4, lim4)) * 4u;
+    return load_f4(row_bytes + off);
+  };
+  auto settle = [&](float4& f, int j) {
+    if (edge && (j * NT + tid) * 4 == last4) {
+      const int m = nv - last4;  // 1 .. 4 entries
+      if (m == 1) f.x = f.w;
+      if (m == 2) f = make_float4(f.z, f.w, 0.f, 0.f);
+      if (m == 3) f = make_float4(f.y, f.z, f.w, 0.f);
+    }
   };
   auto sample_chunk = [&](int s) { return whole ? s : (s * nc) / 4; };
   // Sample entry i of this thread lies inside the row (always, unless whole).
@@ -887,6 +925,7 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
     for (int s = 0; s < 4; ++s) f[s] = load4(sample_chunk(s));
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
+      settle(f[s], sample_chunk(s));
       sv[4 * s] = f[s].x;
       sv[4 * s + 1] = f[s].y;
       sv[4 * s + 2] = f[s].z;
@@ -1050,6 +1089,7 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
       }
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
+        settle(cur[q], jc[q]);
         const float fv[4] = {cur[q].x, cur[q].y, cur[q].z, cur[q].w};
         if (4 * it + q < ns && room()) {  // else a repeated load past the last chunk
           Took r[4];
@@ -1376,14 +1416,15 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
     return;
   }
   uint32_t krem;
-  const uint32_t tk = stream_select<NT, true>(src, nvalid, k, lds, wsum, info, krem);
+  const uint32_t tk = stream_select<NT>(src, nvalid, k, lds, wsum, info, krem, edge);
   if (tid == 0) a.thr[row] = key_to_float(tk);
   if (!IDX && a.mask != nullptr) emit_mask_row<NT>(a, row, nv - 1, key_to_float(tk));
   if constexpr (IDX) {
     const int64_t nchunks = (nvalid + 4 * NT - 1) / (4 * NT);
     emit_indices<NT>(a.idx + row * static_cast<int64_t>(k), nchunks, tk, krem, wsum,
                      [&](int64_t j, uint32_t(&kk)[4]) {
-                       load_keys4<true>(src, (j * NT + tid) * 4, nvalid, kk);
+                       if (edge) load_keys4<false>(src, (j * NT + tid) * 4, nvalid, kk);
+                       else load_keys4<true>(src, (j * NT + tid) * 4, nvalid, kk);
                      });
   }
 }
@@ -1404,7 +1445,7 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
 // value costs one min/max, one fma + med3 + convert for its bin (kept, 8 bits
 // each, for the gather) and one LDS add (config 2 standalone: 222 -> 177 us,
 // 60 -> 75% of HBM peak).
-template <int V>
+template <int V, bool RAGGED>
 __global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wave_kernel(
     SelectArgs a) {
   static_assert(V % 4 == 0 && V >= 4 && V <= 64, "values per lane");
@@ -1436,17 +1477,28 @@ __global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wav
   const int nv = static_cast<int>(nvalid);  // <= 64*V
   const int nch = (nv + 4 * kWave - 1) / (4 * kWave);  // chunks holding valid entries
   float v[V];
+  const bool edge = RAGGED && edge_row(a, row, nvalid);  // wave-uniform
   {
     const char* rb = reinterpret_cast<const char*>(a.scores + row * a.ld);
-    const int last4 = (nv - 1) & ~3;
+    if (!edge) {
+      const int last4 = (nv - 1) & ~3;
 #pragma unroll
-    for (int j = 0; j < NCH; ++j) {
-      const uint32_t off = static_cast<uint32_t>(min((j * kWave + lane) * 4, last4)) * 4u;
-      const float4 f = *reinterpret_cast<const float4*>(rb + off);
-      v[4 * j] = f.x;
-      v[4 * j + 1] = f.y;
-      v[4 * j + 2] = f.z;
-      v[4 * j + 3] = f.w;
+      for (int j = 0; j < NCH; ++j) {
+        const uint32_t off = static_cast<uint32_t>(min((j * kWave + lane) * 4, last4)) * 4u;
+        const float4 f = load_f4(rb + off);
+        v[4 * j] = f.x;
+        v[4 * j + 1] = f.y;
+        v[4 * j + 2] = f.z;
+        v[4 * j + 3] = f.w;
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < NCH; ++j)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const uint32_t off = static_cast<uint32_t>(min((j * kWave + lane) * 4 + c, nv - 1)) * 4u;
+          v[4 * j + c] = *reinterpret_cast<const float*>(rb + off);
+        }
     }
   }
   // f(x, i) for every valid entry (i: its register index).
@@ -1626,9 +1678,15 @@ __global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wav
         }
         for (int j = 0; j < nch; ++j) {
           const int p0 = (j * kWave + lane) * 4;
-          const uint32_t off = static_cast<uint32_t>(min(p0, last4)) * 4u;
-          const float4 q4 = *reinterpret_cast<const float4*>(rb + off);
-          const float xs[4] = {q4.x, q4.y, q4.z, q4.w};
+          float xs[4];
+          if (!edge) {
+            const float4 q4 = load_f4(rb + static_cast<uint32_t>(min(p0, last4)) * 4u);
+            xs[0] = q4.x; xs[1] = q4.y; xs[2] = q4.z; xs[3] = q4.w;
+          } else {
+  #pragma unroll
+            for (int c = 0; c < 4; ++c)
+              xs[c] = *reinterpret_cast<const float*>(rb + static_cast<uint32_t>(min(p0 + c, nv - 1)) * 4u);
+          }
   #pragma unroll
           for (int c = 0; c < 4; ++c)
             if (p0 + c < nv) f(xs[c], 4 * j + c);
@@ -1671,15 +1729,21 @@ __global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wav
   if (lane == 0) a.thr[row] = key_to_float(tk);
 }
 
+// Rows whose length, stride and base are not all 16-byte granular.
+bool ragged(const SelectArgs& a) {
+  return a.n % 4 != 0 || a.ld % 4 != 0 || (reinterpret_cast<uintptr_t>(a.scores) & 15u) != 0;
+}
+
 template <int V>
 hipError_t launch_wave(const SelectArgs& a, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((a.rows + 3) / 4));
-  hipLaunchKernelGGL((topk_wave_kernel<V>), grid, dim3(256), 0, stream, a);
+  if (ragged(a)) hipLaunchKernelGGL((topk_wave_kernel<V, true>), grid, dim3(256), 0, stream, a);
+  else hipLaunchKernelGGL((topk_wave_kernel<V, false>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
 template <int NT, int V, int P1>
-hipError_t launch_reg(const SelectArgs& a, bool vec, hipStream_t stream) {
+hipError_t launch_reg(const SelectArgs& a, hipStream_t stream) {
   // Causal rows: a 2-D grid (batch element, row) whose blocks need no
   // division to find their row (register rows are at most 32768 long, so
   // causal_T fits the grid's y range).
@@ -1687,10 +1751,8 @@ hipError_t launch_reg(const SelectArgs& a, bool vec, hipStream_t stream) {
   const bool two_d = a.causal_T > 1 && a.causal_T <= 65535 && nb <= 0x7fffffff;
   const dim3 grid = two_d ? dim3(static_cast<unsigned>(nb), static_cast<unsigned>(a.causal_T))
                           : dim3(static_cast<unsigned>(a.rows));
-  if (vec)
-    hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, true>), grid, dim3(NT), 0, stream, a);
-  else
-    hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, false>), grid, dim3(NT), 0, stream, a);
+  if (ragged(a)) hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, true>), grid, dim3(NT), 0, stream, a);
+  else hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, false>), grid, dim3(NT), 0, stream, a);
   return hipGetLastError();
 }
 
@@ -1707,21 +1769,19 @@ bool bracket_fits(int64_t cap, int k) {
   return (2.0 * delta + 1.0) / frac <= 0.5 * kCandCap;
 }
 
+template <bool IDX, bool MASK>
 hipError_t launch_bracket(const SelectArgs& a, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(a.rows));
-  if (a.idx != nullptr)
-    hipLaunchKernelGGL((topk_bracket_kernel<256, true>), grid, dim3(256), 0, stream, a);
+  if (ragged(a))
+    hipLaunchKernelGGL((topk_bracket_kernel<256, true, IDX, MASK>), grid, dim3(256), 0, stream, a);
   else
-    hipLaunchKernelGGL((topk_bracket_kernel<256, false>), grid, dim3(256), 0, stream, a);
+    hipLaunchKernelGGL((topk_bracket_kernel<256, false, IDX, MASK>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
-hipError_t launch_stream(const SelectArgs& a, bool vec, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(a.rows));
-  if (vec)
-    hipLaunchKernelGGL((topk_stream_kernel<1024, true>), grid, dim3(1024), 0, stream, a);
-  else
-    hipLaunchKernelGGL((topk_stream_kernel<1024, false>), grid, dim3(1024), 0, stream, a);
+hipError_t launch_stream(const SelectArgs& a, hipStream_t stream) {
+  hipLaunchKernelGGL((topk_stream_kernel<1024>), dim3(static_cast<unsigned>(a.rows)), dim3(1024), 0,
+                     stream, a);
   return hipGetLastError();
 }
 
@@ -1732,10 +1792,6 @@ hipError_t launch_topk(const float* scores, int64_t rows, int64_t n, int64_t ld,
   if (rows == 0) return hipSuccess;
   SelectArgs a{scores, rows, n, ld, k, causal_T, thr, idx, causal_T > 0 ? rows / causal_T : 0};
   const int64_t cap = causal_T > 0 ? (causal_T < n ? causal_T : n) : n;
-  // float4 loads stay inside [0, n) of every row only when n, ld and the base
-  // are all 16-byte granular.
-  const bool vec = (n % 4 == 0) && (ld % 4 == 0) &&
-                   ((reinterpret_cast<uintptr_t>(scores) & 15u) == 0);
   // Rows above 8K entries use a 12-bit first digit: hot digits of real
   // score rows spread over twice the bins (fewer same-address LDS atomics)
   // and the chosen digit leaves half the candidates.
@@ -1745,30 +1801,28 @@ hipError_t launch_topk(const float* scores, int64_t rows, int64_t n, int64_t ld,
   // leave 4 waves per SIMD and the block kernel is faster: 43 vs 45 us).
   // With indices: rows of at most 16 chunks (the per-thread position masks
   // are 64 bits).
-  if (vec && bracket_fits(cap, k) && (idx == nullptr || cap <= kBracketIdxMaxN))
-    return launch_bracket(a, stream);
-  if (idx == nullptr && vec && cap <= 2048) {
+  if (bracket_fits(cap, k) && (idx == nullptr || cap <= kBracketIdxMaxN))
+    return idx != nullptr ? launch_bracket<true, false>(a, stream) : launch_bracket<false, false>(a, stream);
+  if (idx == nullptr && cap <= 2048) {
     if (cap <= 512) return launch_wave<8>(a, stream);
     if (cap <= 1024) return launch_wave<16>(a, stream);
     return launch_wave<32>(a, stream);
   }
-  if (cap <= 512) return launch_reg<128, 4, 11>(a, vec, stream);
-  if (cap <= 1024) return launch_reg<128, 8, 11>(a, vec, stream);
-  if (cap <= 2048) return launch_reg<256, 8, 11>(a, vec, stream);
-  if (cap <= 4096) return launch_reg<256, 16, 11>(a, vec, stream);
-  if (cap <= 8192) return launch_reg<512, 16, 11>(a, vec, stream);
-  if (cap <= 16384) return launch_reg<512, 32, 12>(a, vec, stream);
-  if (cap <= 32768) return launch_reg<1024, 32, 12>(a, vec, stream);
-  return launch_stream(a, vec, stream);
+  if (cap <= 512) return launch_reg<128, 4, 11>(a, stream);
+  if (cap <= 1024) return launch_reg<128, 8, 11>(a, stream);
+  if (cap <= 2048) return launch_reg<256, 8, 11>(a, stream);
+  if (cap <= 4096) return launch_reg<256, 16, 11>(a, stream);
+  if (cap <= 8192) return launch_reg<512, 16, 11>(a, stream);
+  if (cap <= 16384) return launch_reg<512, 32, 12>(a, stream);
+  if (cap <= 32768) return launch_reg<1024, 32, 12>(a, stream);
+  return launch_stream(a, stream);
 }
 
 hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t ld, int k,
                             float* thr, uint64_t* mask, int64_t ldm, hipStream_t stream) {
   if (B == 0 || T == 0) return hipSuccess;
   const int64_t rows = B * T;
-  const bool vec = (T % 4 == 0) && (ld % 4 == 0) &&
-                   ((reinterpret_cast<uintptr_t>(scores) & 15u) == 0);
-  if (vec && bracket_fits(T, k)) {
+  if (bracket_fits(T, k)) {
     // The rows the bracket kernel would select anyway: it writes each row's
     // bitmask words as soon as it has the threshold (config 4: the mask
     // kernel's second 537 MB read of the scores goes).  Rows of up to 16
@@ -1777,13 +1831,8 @@ hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t l
     SelectArgs a{scores, rows, T, ld, k, T, thr, nullptr, B};
     a.mask = mask;
     a.ldm = ldm;
-    if (T <= kBracketIdxMaxN)
-      hipLaunchKernelGGL((topk_bracket_kernel<256, false, true>), dim3(static_cast<unsigned>(rows)),
-                         dim3(256), 0, stream, a);
-    else
-      hipLaunchKernelGGL((topk_bracket_kernel<256, false>), dim3(static_cast<unsigned>(rows)),
-                         dim3(256), 0, stream, a);
-    return hipGetLastError();
+    return T <= kBracketIdxMaxN ? launch_bracket<false, true>(a, stream)
+                                : launch_bracket<false, false>(a, stream);
   }
   const hipError_t e = launch_topk(scores, rows, T, ld, k, T, thr, nullptr, stream);
   if (e != hipSuccess) return e;

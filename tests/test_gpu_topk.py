@@ -438,3 +438,59 @@ def test_causal_c4_shape_properties(dev):
     sub = sub.masked_fill(torch.arange(T)[None, :] > torch.tensor(rows)[:, None], float("-inf"))
     assert torch.equal(thr[0, rows].cpu(), O.topk_threshold(sub, k))
     assert np.array_equal(idx[0, rows].cpu().numpy(), O.select_indices(sub.numpy(), k))
+
+
+@pytest.mark.parametrize("n", [1, 2, 3, 5, 63, 255, 511, 513, 1023, 1025, 2047, 2049, 4095, 4097, 4098,
+                               4099, 5001, 8195, 16383, 20001, 40003])
+def test_rows_of_any_length_stride_and_alignment(dev, n):
+    """Rows load 16 bytes per lane at any 4-byte alignment; the last rows of
+    the array, whose last group of four would run past its end, load entry by
+    entry or shift that group.  Lengths of every remainder around each
+    kernel's limit, strides and base offsets of 0 to 3 entries, thresholds
+    and indices, bit for bit against torch.topk (whose index order for ties
+    does not matter here: distinct values)."""
+    import _dsa_lib as L
+
+    rows = 5
+    g = torch.Generator().manual_seed(n)
+    for pad, off in ((0, 0), (1, 1), (3, 2), (2, 3)):
+        ld = n + pad
+        x = torch.randn(rows, n, generator=g)
+        flat = torch.full((off + (rows - 1) * ld + n,), float("nan"))
+        view = flat[off:].as_strided((rows, n), (ld, 1))
+        view.copy_(x)
+        buf = flat.to(dev)
+        for k in sorted({1, max(1, n // 3), n}):
+            thr = torch.empty(rows, device=dev)
+            idx = torch.empty(rows, k, device=dev, dtype=torch.int32)
+            want = x.topk(k, dim=-1)
+            for ip in (None, idx.data_ptr()):
+                rc = L.lib().dsa_topk_threshold(buf.data_ptr() + 4 * off, rows, n, ld, k, 0,
+                                                thr.data_ptr(), ip, L.stream_ptr(torch.device(dev)))
+                assert rc == 0
+                assert torch.equal(thr.cpu(), want.values[:, -1]), (pad, off, k, ip is None)
+            assert torch.equal(idx.cpu().long(), want.indices.sort(-1).values), (pad, off, k)
+
+
+@pytest.mark.parametrize("T,k", [(4097, 300), (4099, 64), (6001, 1000), (3001, 100), (701, 30)])
+def test_ragged_causal_masks_and_indices(dev, T, k):
+    """Odd T: thresholds, the bitmask the select writes (against the two
+    launches) and indices, garbage above the diagonal."""
+    from dsa_attention import selection_mask
+
+    g = torch.Generator(device=dev).manual_seed(T)
+    s = torch.randn(2, T, T, generator=g, device=dev)
+    tril = torch.ones(T, T, dtype=torch.bool, device=dev).tril()
+    full = s.masked_fill(~tril, float("-inf"))
+    s = s.masked_fill(~tril, float("nan"))
+    want = full.topk(k, dim=-1)
+    thr, mask = topk_threshold_mask(s, k)
+    assert torch.equal(thr, want.values[..., -1:])
+    W = (T + 63) // 64
+    written = (torch.arange(W, device=dev)[None, :] <= (torch.arange(T, device=dev)[:, None] | 127) // 64)
+    ref = selection_mask(s, thr)
+    assert torch.equal(mask[:, written], ref[:, written])
+    thr2, idx = topk_indices(s, k, causal=True)
+    assert torch.equal(thr2, thr)
+    rows = torch.arange(T, device=dev) + 1 >= k
+    assert torch.equal(idx[:, rows].long(), want.indices[:, rows].sort(-1).values)
