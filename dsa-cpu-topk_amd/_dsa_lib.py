@@ -44,6 +44,7 @@ _SIGNATURES = {
     "dsa_indexer_scores_fp8_scaled": ([_P, _P, _P, _P, _P, _I64, _I64, _I, _I, _P, _I64, _I, _P],
                                       _I),
     "dsa_topk_threshold": ([_P, _I64, _I64, _I64, _I, _I64, _P, _P, _P], _I),
+    "dsa_topk_member": ([_P, _I64, _I64, _I64, _I, _P, _P, _P], _I),
     "dsa_sparse_attn_threshold": ([_P, _I64, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _F,
                                    _P, _P], _I),
     "dsa_sparse_attn_threshold_tiled": ([_P, _I64, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I,

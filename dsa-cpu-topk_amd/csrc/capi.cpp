@@ -176,6 +176,18 @@ int dsa_topk_threshold(const float* scores, int64_t rows, int64_t n, int64_t ld,
                     "dsa_topk_threshold");
 }
 
+int dsa_topk_member(const float* scores, int64_t rows, int64_t n, int64_t ld, int k, float* thr,
+                    uint8_t* member, void* stream) {
+  if (rows < 0 || n < 0) return fail(DSA_EINVAL, "topk_member: negative size rows=%lld n=%lld", (long long)rows, (long long)n);
+  if (k <= 0 || k > n) return fail(DSA_EINVAL, "topk_member: k=%d outside [1, N=%lld]", k, (long long)n);
+  if (n > kMaxElems / 4 || rows > kMaxElems) return fail(DSA_EINVAL, "topk_member: rows=%lld of N=%lld too large", (long long)rows, (long long)n);
+  if (ld < n) return fail(DSA_EINVAL, "topk_member: ld=%lld < N=%lld", (long long)ld, (long long)n);
+  if (rows == 0) return DSA_OK;
+  if (!scores || !thr || !member) return fail(DSA_EINVAL, "topk_member: null pointer");
+  return hip_status(dsa::launch_topk_member(scores, rows, n, ld, k, thr, member, static_cast<hipStream_t>(stream)),
+                    "dsa_topk_member");
+}
+
 int dsa_topk_threshold_mask(const float* scores, int64_t B, int64_t T, int64_t ld, int k,
                             float* thr, uint64_t* mask, int64_t ldm, void* stream) {
   if (B < 0 || T < 0) return fail(DSA_EINVAL, "topk_mask: negative size B=%lld T=%lld", (long long)B, (long long)T);

@@ -11,6 +11,10 @@ namespace dsa {
 // Radix-select: thr[r] = k-th largest of row r, optional exactly-k indices.
 hipError_t launch_topk(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
                        int64_t causal_T, float* thr, int32_t* idx, hipStream_t stream);
+// Thresholds and, per entry, one byte: whether it is among the row's k largest
+// (the lowest indices first among equals); rows of n bytes.
+hipError_t launch_topk_member(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
+                              float* thr, uint8_t* member, hipStream_t stream);
 // Causal thresholds of a [B,T,T] score matrix plus the rows' selection
 // bitmask (what launch_selection_mask writes), in one pass over the scores
 // where the bracket kernel serves the rows; otherwise the two launches.

@@ -423,8 +423,9 @@ __device__ __forceinline__ void load_keys4(const float* __restrict__ src, int64_
 // ---------------------------------------------------------------------------
 // Keys plus ~30 working registers fit 64 VGPRs up to V = 32: blocks of up to
 // 512 threads ask for 8 waves per SIMD there, so that four rows share a CU.
-template <int NT, int V, int P1, bool RAGGED>
-__global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_kernel(SelectArgs a) {
+// NEG (threshold only): rows that hold -inf in number, masked score rows.
+template <int NT, int V, int P1, bool RAGGED, bool NEG = false>
+__global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void topk_reg_kernel(SelectArgs a) {
   static_assert(V % 4 == 0 && NT % kWave == 0 && NT <= 1024, "block shape");
   static_assert(P1 == 11 || P1 == 12, "first digit width");
   constexpr int NCH = V / 4;
@@ -438,7 +439,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_k
   __shared__ uint32_t cand[CAP];
   __shared__ uint32_t wsum[NT / kWave];
   __shared__ uint32_t info[4];
-  __shared__ uint32_t ncand;
+  __shared__ uint32_t ncand, ninf;
   __shared__ float red[3 * (NT / kWave)];
 
   const int tid = threadIdx.x;
@@ -537,6 +538,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_k
   uint32_t thr_key = 0, krem = 0;
   bool keys_in_regs = false, done = false;
   if (tid == 0) ncand = 0u;
+  if (NEG && tid == 0) ninf = 0u;
   // Rows of up to 16 values per thread search by value bins first; longer
   // register rows (32 per thread) have no registers to spare for it and go
   // straight to the radix passes.
@@ -567,9 +569,19 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_k
     }
   };
   block_range();
+  // -inf queues at one counter of a histogram, entry by entry.  Under NEG it
+  // is counted from the registers: a row with fewer than k entries above it
+  // has it as the k-th largest, and any other row is binned without it.
+  const bool neg = NEG && !(lo > -__builtin_huge_valf());
   if (!(lo > -__builtin_huge_valf()) || !(hi < __builtin_huge_valf())) {
     // An infinite value (block-uniform, rare): the finite range instead.
     block_sync_lds();  // every wave has read red
+    if (neg) {
+      uint32_t ni = 0;
+      visit_vals([&](float x, int) { ni += x == -__builtin_huge_valf() ? 1u : 0u; });
+      ni = wave_inclusive_sum(ni);
+      if (lane == kWave - 1) atomicAdd(&ninf, ni);  // published by block_range
+    }
     lo = __builtin_huge_valf();
     hi = -__builtin_huge_valf();
     visit_vals([&](float x, int) {
@@ -578,6 +590,10 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_k
       hi = fmaxf(hi, fin ? x : -__builtin_huge_valf());
     });
     block_range();
+    if (neg && static_cast<uint32_t>(k) > static_cast<uint32_t>(nv) - ninf) {
+      if (tid == 0) a.thr[row] = -__builtin_huge_valf();
+      return;
+    }
   }
   // Stage 2: NBV bins linear in value between lo and hi.  Bins follow the
   // data's density, so the histogram's ds_adds rarely collide, and the bin
@@ -607,8 +623,9 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512) ? 8 : 4) void topk_reg_k
 #pragma unroll
   for (int i = 0; i < V / 2; ++i) bp[i] = 0u;
   visit_vals([&](float x, int i) {
-    const uint32_t c = bin_of(x);
-    atomicAdd(&hist[c], 1u);
+    uint32_t c = bin_of(x);
+    if (neg && x == -__builtin_huge_valf()) c = 0xffffu;  // no bin
+    else atomicAdd(&hist[c], 1u);
     bp[i >> 1] |= c << (16 * (i & 1));
   });
   auto bin_at = [&](int i) __attribute__((always_inline)) {
@@ -852,7 +869,7 @@ constexpr int kFinGather = 64;   // kept values of one finishing bin ranked in r
 // Eight blocks per CU (at most 64 VGPRs; the LDS columns allow eight): at
 // config 4 thresholds 101 -> 98 us, with indices 156 -> 152, the bitmask
 // 129 -> 127 against six (the bitmask and index forms spill a few SGPRs).
-template <int NT, bool RAGGED, bool IDX, bool MASK = false>
+template <int NT, bool RAGGED, bool IDX, bool MASK = false, bool NEG = false>  // NEG: as in topk_reg_kernel
 __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
   // IDX: exactly-k indices; MASK: the selection bitmask (a.mask), both from
   // the row's flag bitmap below.
@@ -979,6 +996,7 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
     reinterpret_cast<uint4*>(lds)[q * NT + tid] = make_uint4(0u, 0u, 0u, 0u);
   float vmin, vmax;
   block_range(false, vmin, vmax);
+  const bool neg = NEG && !(vmin > -__builtin_huge_valf());  // the sample may hold -inf
   if (!(vmax < __builtin_huge_valf()) || !(vmin > -__builtin_huge_valf())) {
     block_sync_lds();  // every wave has read wext
     block_range(true, vmin, vmax);
@@ -990,7 +1008,17 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
     scale = 0.0f;
     vmin = 0.0f;
   }
-  if (whole) {
+  if (neg) {  // -inf is counted apart and added to its bin, 0, once per wave
+    uint32_t ni = 0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      if (!sample_in(i)) continue;
+      if (sv[i] == -__builtin_huge_valf()) ++ni;
+      else atomicAdd(&lds[value_bin(sv[i], vmin, scale, kBrBins - 1)], 1u);
+    }
+    ni = wave_inclusive_sum(ni);
+    if (lane == kWave - 1 && ni != 0u) atomicAdd(&lds[0], ni);
+  } else if (whole) {
 #pragma unroll
     for (int i = 0; i < 16; ++i)
       if (sample_in(i)) atomicAdd(&lds[value_bin(sv[i], vmin, scale, kBrBins - 1)], 1u);
@@ -1415,8 +1443,30 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
     }
     return;
   }
-  uint32_t krem;
-  const uint32_t tk = stream_select<NT>(src, nvalid, k, lds, wsum, info, krem, edge);
+  uint32_t krem = 0;
+  uint32_t tk = float_to_key(-__builtin_huge_valf());
+  bool short_row = false;
+  if (neg) {
+    // A masked row with fewer than k entries above -inf: one counting pass
+    // instead of three radix passes that queue at one digit.
+    uint32_t n = 0;
+    for (int j = 0; j < nc; ++j) {
+      float4 f = load4(j);
+      settle(f, j);
+      const float fv[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+        n += ((j * NT + tid) * 4 + c < nv && fv[c] != -__builtin_huge_valf()) ? 1u : 0u;
+    }
+    uint32_t over;
+    block_sync_lds();  // earlier reads of wsum are done
+    block_exclusive_sum<NT>(n, wsum, over);
+    if (static_cast<uint32_t>(k) > over) {
+      krem = static_cast<uint32_t>(k) - over;
+      short_row = true;
+    }
+  }
+  if (!short_row) tk = stream_select<NT>(src, nvalid, k, lds, wsum, info, krem, edge);
   if (tid == 0) a.thr[row] = key_to_float(tk);
   if (!IDX && a.mask != nullptr) emit_mask_row<NT>(a, row, nv - 1, key_to_float(tk));
   if constexpr (IDX) {
@@ -1445,8 +1495,8 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
 // value costs one min/max, one fma + med3 + convert for its bin (kept, 8 bits
 // each, for the gather) and one LDS add (config 2 standalone: 222 -> 177 us,
 // 60 -> 75% of HBM peak).
-template <int V, bool RAGGED>
-__global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wave_kernel(
+template <int V, bool RAGGED, bool NEG = false>  // NEG: as in topk_reg_kernel
+__global__ __launch_bounds__(256, V <= 16 ? (NEG ? 6 : 8) : (V <= 32 ? (NEG ? 5 : 6) : 4)) void topk_wave_kernel(
     SelectArgs a) {
   static_assert(V % 4 == 0 && V >= 4 && V <= 64, "values per lane");
   constexpr int NCH = V / 4;  // float4 chunks per lane; chunk j covers 256 entries
@@ -1579,6 +1629,16 @@ __global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wav
   });
   lo = wave_extreme_f32<false>(lo);
   hi = wave_extreme_f32<true>(hi);
+  const bool neg = NEG && !(lo > -__builtin_huge_valf());
+  if (neg) {
+    uint32_t above = 0;
+    visit([&](float x, int) { above += x == -__builtin_huge_valf() ? 0u : 1u; });
+    above = wave_read_lane(wave_inclusive_sum(above), kWave - 1);
+    if (static_cast<uint32_t>(k) > above) {
+      if (lane == 0) a.thr[row] = -__builtin_huge_valf();
+      return;
+    }
+  }
   if (!(lo > -__builtin_huge_valf()) || !(hi < __builtin_huge_valf())) {
     lo = __builtin_huge_valf();
     hi = -__builtin_huge_valf();
@@ -1613,11 +1673,21 @@ __global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wav
   uint32_t bp[V / 4];
 #pragma unroll
   for (int i = 0; i < V / 4; ++i) bp[i] = 0u;
+  [[maybe_unused]] uint32_t nbot = 0;  // -inf entries of this lane
   visit([&](float x, int i) {
     const uint32_t c = bin_of(x);
-    atomicAdd(&hist[c], 1u);
+    if constexpr (NEG) {
+      if (x == -__builtin_huge_valf()) ++nbot;
+      else atomicAdd(&hist[c], 1u);
+    } else {
+      atomicAdd(&hist[c], 1u);
+    }
     bp[i >> 2] |= c << (8 * (i & 3));
   });
+  if constexpr (NEG) {  // bin 255 keeps them, added once
+    nbot = wave_inclusive_sum(nbot);
+    if (lane == kWave - 1) atomicAdd(&hist[255], nbot);
+  }
   wave_lds_sync();
   uint32_t bsel, brank, bcnt;
   pick_top(static_cast<uint32_t>(k), bsel, brank, bcnt);
@@ -1729,21 +1799,131 @@ __global__ __launch_bounds__(256, V <= 16 ? 8 : (V <= 32 ? 6 : 4)) void topk_wav
   if (lane == 0) a.thr[row] = key_to_float(tk);
 }
 
+// ---------------------------------------------------------------------------
+// Membership of each entry in its row's top k, one byte each, from the row's
+// k-th largest: entries above it, and the lowest-index ones equal to it up to
+// k.  One wave per row: a first pass counts the entries above and equal (4 per
+// lane and step, 4 steps' loads in flight), a second one, from the cache,
+// writes the bytes; only rows that take part of their equal entries rank them.
+// HBM-bound: the row read, n bytes written (two [4096, 4096] matrices with the
+// -inf triangle, k = 256: 27 us, and 34 for the thresholds before it; 138 us
+// as indices scattered into a zeroed mask).
+// ---------------------------------------------------------------------------
+// U: steps of 256 entries a lane holds at once (REG: the whole row, read once).
+// In the key order (NaN the largest value, -0 = +0) an entry is above the
+// threshold if !(x <= th), at or above it if !(x < th).  Two rewrites of what
+// was loaded keep that true everywhere: positions past the row read as -inf
+// (below any threshold but -inf, which every entry of the row reaches), and
+// under a NaN threshold NaNs as +inf against +inf, the rest as -inf.
+template <int U, bool REG>
+__global__ __launch_bounds__(256) void member_kernel(SelectArgs a, uint8_t* __restrict__ member) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  if (row >= a.rows) return;  // whole waves
+  const int n = static_cast<int>(a.n);
+  constexpr float kInf = __builtin_huge_valf();
+  const float thr = a.thr[row];
+  const bool tn = thr != thr;
+  const float th = tn ? kInf : thr;
+  const char* rb = reinterpret_cast<const char*>(a.scores + row * a.ld);
+  uint8_t* out = member + row * a.n;
+  const bool edge = edge_row(a, row, n);
+  constexpr int CH = 4 * kWave;  // entries per step
+  const int last4 = (n - 1) & ~3;
+  float x[U][4];
+  auto load = [&](int s) {
+    if (!edge) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const float4 f = load_f4(rb + static_cast<uint32_t>(min(s + u * CH + 4 * lane, last4)) * 4u);
+        x[u][0] = f.x; x[u][1] = f.y; x[u][2] = f.z; x[u][3] = f.w;
+      }
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          x[u][c] = *reinterpret_cast<const float*>(rb + static_cast<uint32_t>(min(s + u * CH + 4 * lane + c, n - 1)) * 4u);
+    }
+    if (tn) {
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[u][c] = x[u][c] != x[u][c] ? kInf : -kInf;
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+      if (s + (u + 1) * CH > n) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) x[u][c] = s + u * CH + 4 * lane + c < n ? x[u][c] : -kInf;
+      }
+  };
+  uint32_t gt = 0, ge = 0;
+  for (int s = 0; s < n; s += U * CH) {
+    load(s);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        gt += !(x[u][c] <= th) ? 1u : 0u;
+        ge += !(x[u][c] < th) ? 1u : 0u;
+      }
+  }
+  gt = wave_read_lane(wave_inclusive_sum(gt), kWave - 1);
+  ge = wave_read_lane(wave_inclusive_sum(ge), kWave - 1);
+  if (th == -kInf) ge = static_cast<uint32_t>(n);
+  const uint32_t need = static_cast<uint32_t>(a.k) - gt;  // equal entries to take
+  const bool all = ge - gt == need;
+  uint32_t before = 0;  // equal entries of earlier steps
+  for (int s = 0; s < n; s += U * CH) {
+    if constexpr (!REG) load(s);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s + u * CH >= n) break;
+      const int p0 = s + u * CH + 4 * lane;
+      uint32_t w = 0;
+      if (all) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) w |= !(x[u][c] < th) ? 1u << (8 * c) : 0u;
+      } else {
+        uint32_t eq = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) eq += (p0 + c < n && x[u][c] == th) ? 1u : 0u;
+        const uint32_t incl = wave_inclusive_sum(eq);
+        uint32_t rank = before + incl - eq;
+        before += wave_read_lane(incl, kWave - 1);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if (x[u][c] == th) w |= rank++ < need ? 1u << (8 * c) : 0u;
+          else w |= !(x[u][c] < th) ? 1u << (8 * c) : 0u;
+        }
+      }
+      if (p0 + 4 <= n) {
+        __builtin_memcpy(out + p0, &w, 4);  // any byte alignment
+      } else {
+        for (int c = 0; c < 4; ++c)
+          if (p0 + c < n) out[p0 + c] = static_cast<uint8_t>(w >> (8 * c));
+      }
+    }
+  }
+}
+
 // Rows whose length, stride and base are not all 16-byte granular.
 bool ragged(const SelectArgs& a) {
   return a.n % 4 != 0 || a.ld % 4 != 0 || (reinterpret_cast<uintptr_t>(a.scores) & 15u) != 0;
 }
 
 template <int V>
-hipError_t launch_wave(const SelectArgs& a, hipStream_t stream) {
+hipError_t launch_wave(const SelectArgs& a, bool neg, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((a.rows + 3) / 4));
-  if (ragged(a)) hipLaunchKernelGGL((topk_wave_kernel<V, true>), grid, dim3(256), 0, stream, a);
+  if (neg) hipLaunchKernelGGL((topk_wave_kernel<V, true, true>), grid, dim3(256), 0, stream, a);
+  else if (ragged(a)) hipLaunchKernelGGL((topk_wave_kernel<V, true>), grid, dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((topk_wave_kernel<V, false>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
 template <int NT, int V, int P1>
-hipError_t launch_reg(const SelectArgs& a, hipStream_t stream) {
+hipError_t launch_reg(const SelectArgs& a, bool neg, hipStream_t stream) {
   // Causal rows: a 2-D grid (batch element, row) whose blocks need no
   // division to find their row (register rows are at most 32768 long, so
   // causal_T fits the grid's y range).
@@ -1751,6 +1931,12 @@ hipError_t launch_reg(const SelectArgs& a, hipStream_t stream) {
   const bool two_d = a.causal_T > 1 && a.causal_T <= 65535 && nb <= 0x7fffffff;
   const dim3 grid = two_d ? dim3(static_cast<unsigned>(nb), static_cast<unsigned>(a.causal_T))
                           : dim3(static_cast<unsigned>(a.rows));
+  if constexpr (V <= 16) {
+    if (neg) {
+      hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, true, true>), grid, dim3(NT), 0, stream, a);
+      return hipGetLastError();
+    }
+  }
   if (ragged(a)) hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, true>), grid, dim3(NT), 0, stream, a);
   else hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, false>), grid, dim3(NT), 0, stream, a);
   return hipGetLastError();
@@ -1770,9 +1956,11 @@ bool bracket_fits(int64_t cap, int k) {
 }
 
 template <bool IDX, bool MASK>
-hipError_t launch_bracket(const SelectArgs& a, hipStream_t stream) {
+hipError_t launch_bracket(const SelectArgs& a, bool neg, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(a.rows));
-  if (ragged(a))
+  if (!IDX && !MASK && neg)
+    hipLaunchKernelGGL((topk_bracket_kernel<256, true, false, false, true>), grid, dim3(256), 0, stream, a);
+  else if (ragged(a))
     hipLaunchKernelGGL((topk_bracket_kernel<256, true, IDX, MASK>), grid, dim3(256), 0, stream, a);
   else
     hipLaunchKernelGGL((topk_bracket_kernel<256, false, IDX, MASK>), grid, dim3(256), 0, stream, a);
@@ -1785,10 +1973,13 @@ hipError_t launch_stream(const SelectArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-}  // namespace
-
-hipError_t launch_topk(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
-                       int64_t causal_T, float* thr, int32_t* idx, hipStream_t stream) {
+// neg: the rows may hold -inf in number (thresholds of masked score rows: two
+// [4096, 4096] matrices with the -inf triangle, k = 256: 72 -> 35 us; six of
+// 1800, k = 150: 101 -> 33).  The kernels that count it apart are instances of
+// their own, for any alignment: in the plain ones the test costs rows without
+// -inf up to a quarter (spilled registers: 16384 x 4096, 45 -> 56 us).
+hipError_t launch_select(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
+                         int64_t causal_T, float* thr, int32_t* idx, bool neg, hipStream_t stream) {
   if (rows == 0) return hipSuccess;
   SelectArgs a{scores, rows, n, ld, k, causal_T, thr, idx, causal_T > 0 ? rows / causal_T : 0};
   const int64_t cap = causal_T > 0 ? (causal_T < n ? causal_T : n) : n;
@@ -1802,20 +1993,42 @@ hipError_t launch_topk(const float* scores, int64_t rows, int64_t n, int64_t ld,
   // With indices: rows of at most 16 chunks (the per-thread position masks
   // are 64 bits).
   if (bracket_fits(cap, k) && (idx == nullptr || cap <= kBracketIdxMaxN))
-    return idx != nullptr ? launch_bracket<true, false>(a, stream) : launch_bracket<false, false>(a, stream);
+    return idx != nullptr ? launch_bracket<true, false>(a, false, stream)
+                          : launch_bracket<false, false>(a, neg, stream);
   if (idx == nullptr && cap <= 2048) {
-    if (cap <= 512) return launch_wave<8>(a, stream);
-    if (cap <= 1024) return launch_wave<16>(a, stream);
-    return launch_wave<32>(a, stream);
+    if (cap <= 512) return launch_wave<8>(a, neg, stream);
+    if (cap <= 1024) return launch_wave<16>(a, neg, stream);
+    return launch_wave<32>(a, neg, stream);
   }
-  if (cap <= 512) return launch_reg<128, 4, 11>(a, stream);
-  if (cap <= 1024) return launch_reg<128, 8, 11>(a, stream);
-  if (cap <= 2048) return launch_reg<256, 8, 11>(a, stream);
-  if (cap <= 4096) return launch_reg<256, 16, 11>(a, stream);
-  if (cap <= 8192) return launch_reg<512, 16, 11>(a, stream);
-  if (cap <= 16384) return launch_reg<512, 32, 12>(a, stream);
-  if (cap <= 32768) return launch_reg<1024, 32, 12>(a, stream);
+  if (cap <= 512) return launch_reg<128, 4, 11>(a, neg, stream);
+  if (cap <= 1024) return launch_reg<128, 8, 11>(a, neg, stream);
+  if (cap <= 2048) return launch_reg<256, 8, 11>(a, neg, stream);
+  if (cap <= 4096) return launch_reg<256, 16, 11>(a, neg, stream);
+  if (cap <= 8192) return launch_reg<512, 16, 11>(a, neg, stream);
+  if (cap <= 16384) return launch_reg<512, 32, 12>(a, neg, stream);
+  if (cap <= 32768) return launch_reg<1024, 32, 12>(a, neg, stream);
   return launch_stream(a, stream);
+}
+
+}  // namespace
+
+hipError_t launch_topk(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
+                       int64_t causal_T, float* thr, int32_t* idx, hipStream_t stream) {
+  return launch_select(scores, rows, n, ld, k, causal_T, thr, idx, false, stream);
+}
+
+hipError_t launch_topk_member(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
+                              float* thr, uint8_t* member, hipStream_t stream) {
+  if (rows == 0) return hipSuccess;
+  const hipError_t e = launch_select(scores, rows, n, ld, k, 0, thr, nullptr, true, stream);
+  if (e != hipSuccess) return e;
+  const SelectArgs a{scores, rows, n, ld, k, 0, thr, nullptr, 0};
+  const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
+  if (n <= 1024) hipLaunchKernelGGL((member_kernel<4, true>), grid, dim3(256), 0, stream, a, member);
+  else if (n <= 2048) hipLaunchKernelGGL((member_kernel<8, true>), grid, dim3(256), 0, stream, a, member);
+  else if (n <= 4096) hipLaunchKernelGGL((member_kernel<16, true>), grid, dim3(256), 0, stream, a, member);
+  else hipLaunchKernelGGL((member_kernel<8, false>), grid, dim3(256), 0, stream, a, member);
+  return hipGetLastError();
 }
 
 hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t ld, int k,
@@ -1831,8 +2044,8 @@ hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t l
     SelectArgs a{scores, rows, T, ld, k, T, thr, nullptr, B};
     a.mask = mask;
     a.ldm = ldm;
-    return T <= kBracketIdxMaxN ? launch_bracket<false, true>(a, stream)
-                                : launch_bracket<false, false>(a, stream);
+    return T <= kBracketIdxMaxN ? launch_bracket<false, true>(a, false, stream)
+                                : launch_bracket<false, false>(a, false, stream);
   }
   const hipError_t e = launch_topk(scores, rows, T, ld, k, T, thr, nullptr, stream);
   if (e != hipSuccess) return e;

@@ -267,15 +267,12 @@ def indexer_triton(h, W_Q, W_K, W_W, num_heads, head_dim, **kw):
 def topk_mask(scores: torch.Tensor, k: int) -> torch.Tensor:
     """Boolean [B,T,T] mask of the top-k key positions of every query row.
 
-    Built from the radix-select's exactly-k index set: the lowest index wins
+    The radix-select's exactly-k set: the lowest index wins
     ties, so the mask is deterministic (the reference took torch.topk's
     indices, whose tie order is unspecified).  GPU tensors only.
     """
-    from topk_threshold import topk_indices
+    from topk_threshold import topk_member
 
     L.require_gpu(scores)
     B, T, _ = scores.shape
-    _, idx = topk_indices(scores, min(k, T))
-    mask = torch.zeros_like(scores, dtype=torch.bool)
-    mask.scatter_(-1, idx.long(), True)
-    return mask
+    return topk_member(scores, min(k, T))

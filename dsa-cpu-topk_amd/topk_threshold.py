@@ -138,6 +138,23 @@ def topk_threshold_mask(scores: torch.Tensor, k: int, thr: torch.Tensor | None =
     return thr, mask
 
 
+def topk_member(scores: torch.Tensor, k: int) -> torch.Tensor:
+    """Boolean mask, shaped as `scores` (GPU): the k positions of every row
+    that topk_indices lists."""
+    N = _check(scores, k)
+    L.require_gpu(scores)
+    rows = scores.numel() // N
+    thr = torch.empty(rows, device=scores.device, dtype=torch.float32)
+    member = torch.empty(scores.shape, device=scores.device, dtype=torch.bool)
+    if rows:
+        rc = L.lib().dsa_topk_member(scores.data_ptr(), rows, N, N, int(k), thr.data_ptr(),
+                                     member.data_ptr(), L.stream_ptr(scores.device))
+        if rc != L.DSA_OK:
+            msg = L.lib().dsa_last_error().decode(errors="replace")
+            raise RuntimeError(f"topk_member: {msg}")
+    return member
+
+
 def topk_indices(scores: torch.Tensor, k: int, causal: bool = False):
     """(threshold [...,1] fp32, indices [...,k] int32).
 

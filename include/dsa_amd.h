@@ -134,6 +134,16 @@ int dsa_topk_threshold(const float* scores, int64_t rows, int64_t n, int64_t ld,
                        void* stream);
 
 /*
+ * The k-th largest of each row (thr) and its top-k set as one byte per entry:
+ * member[r*n + j] = 1 for every entry above thr[r] and the lowest-index ones
+ * equal to it up to k in all, else 0 (the set dsa_topk_threshold's idx lists).
+ * Rows of n < 2^29 entries, ld >= n.
+ * Replaces: topk_mask, reference lightning_indexer.py:137-144.
+ */
+int dsa_topk_member(const float* scores, int64_t rows, int64_t n, int64_t ld, int k, float* thr,
+                    uint8_t* member, void* stream);
+
+/*
  * Sparse attention restricted to keys whose indexer score passes a threshold.
  *   sel(b,t,s) = (s <= t) && (scores[b,t,s] >= thr[b*T+t])   (ties kept)
  *   O[b,t,h,:] = sum_{s in sel} softmax_s(<Q[b,t,h],K[b,s,h]> * scale) V[b,s,h,:]

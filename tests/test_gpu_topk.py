@@ -494,3 +494,28 @@ def test_ragged_causal_masks_and_indices(dev, T, k):
     assert torch.equal(thr2, thr)
     rows = torch.arange(T, device=dev) + 1 >= k
     assert torch.equal(idx[:, rows].long(), want.indices[:, rows].sort(-1).values)
+
+
+@pytest.mark.parametrize("n,k", [(1, 1), (3, 2), (63, 5), (256, 256), (1023, 40), (1025, 1), (3001, 700),
+                                 (4099, 300), (5000, 4999), (16388, 9000)])
+def test_topk_member_bytes(dev, n, k):
+    """The top-k set as bytes equals the listed indices: distinct values,
+    heavy ties (part of the equal entries taken), -inf tails with more and with
+    fewer than k entries before them, NaN and +inf."""
+    from topk_threshold import topk_member
+
+    g = torch.Generator().manual_seed(n)
+    x = torch.randn(9, n, generator=g)
+    x[1] = torch.randint(0, 3, (n,), generator=g).float()
+    x[2] = 1.0
+    x[3, n // 2:] = float("-inf")
+    x[4, ::3] = float("nan")
+    x[5] = float("nan")
+    x[6, ::2] = float("inf")
+    x[7] = torch.where(torch.rand(n, generator=g) < 0.5, 0.0, -0.0)
+    x[8, k // 2:] = float("-inf")
+    x = x.to(dev)
+    got = topk_member(x, k)
+    _, idx = topk_indices(x, k)
+    want = torch.zeros(9, n, dtype=torch.bool, device=dev).scatter_(-1, idx.long(), True)
+    assert torch.equal(got, want)
