@@ -64,6 +64,8 @@ struct SelectArgs {
   // per row; null: none.
   uint64_t* mask = nullptr;
   int64_t ldm = 0;
+  // MEM instances and member_kernel: one byte per entry, n per row.
+  uint8_t* member = nullptr;
 };
 
 // Four consecutive scores in one global_load_dwordx4, which needs 4-byte
@@ -288,6 +290,118 @@ __device__ __forceinline__ bool radix_pass(Visit&& visit, uint32_t* hist, uint32
   return false;
 }
 
+// Membership of each entry in its row's top k, one byte each: entries above
+// the row's k-th largest, and the lowest-index ones equal to it up to k.
+
+// Bytes p .. p + 3 of a row of n, from the flags in w's bytes.
+__device__ __forceinline__ void store_members(uint8_t* out, int p, int n, uint32_t w) {
+  if (p + 4 <= n) {
+    __builtin_memcpy(out + p, &w, 4);  // any byte alignment
+  } else {
+    for (int c = 0; c < 4; ++c)
+      if (p + c < n) out[p + c] = static_cast<uint8_t>(w >> (8 * c));
+  }
+}
+
+// By a block, from the row's keys in registers (chunk j: positions
+// (j*NT + tid)*4 .. +3; kKeyNone past the row).  Only a row that takes part of
+// its equal entries ranks them.
+template <int NT, int NCH>
+__device__ __forceinline__ void emit_members(uint8_t* out, int n, const uint32_t (&key)[4 * NCH],
+                                             uint32_t thr_key, uint32_t krem, uint32_t* wsum) {
+  const int tid = threadIdx.x;
+  uint32_t neq = 0, tot;
+#pragma unroll
+  for (int i = 0; i < 4 * NCH; ++i) neq += (key[i] == thr_key) ? 1u : 0u;
+  block_exclusive_sum<NT>(neq, wsum, tot);
+  const bool all = tot == krem;
+  uint32_t run = 0;  // equal entries of earlier chunks
+#pragma unroll
+  for (int j = 0; j < NCH; ++j) {
+    if (j * NT * 4 < n) {
+      uint32_t w = 0;
+      if (all) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) w |= (key[4 * j + c] >= thr_key) ? 1u << (8 * c) : 0u;
+      } else {
+        uint32_t eq = 0;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) eq += (key[4 * j + c] == thr_key) ? 1u : 0u;
+        uint32_t rank = run + block_exclusive_sum<NT>(eq, wsum, tot);
+        run += tot;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          if (key[4 * j + c] == thr_key) w |= rank++ < krem ? 1u << (8 * c) : 0u;
+          else w |= (key[4 * j + c] > thr_key) ? 1u << (8 * c) : 0u;
+        }
+      }
+      store_members(out, (j * NT + tid) * 4, n, w);
+    }
+  }
+}
+
+// By a wave, four entries per lane and step, as floats.  In the key order (NaN
+// the largest value, -0 = +0) an entry is above the threshold if !(x <= th), at
+// or above it if !(x < th).  Two rewrites of what was loaded keep that true
+// everywhere: positions past the row read as -inf (below any threshold but
+// -inf, which every entry of the row reaches), and under a NaN threshold NaNs
+// as +inf against +inf, the rest as -inf.
+struct MemberWave {
+  int n;
+  bool nan_thr;
+  float th;
+  uint32_t gt = 0, ge = 0;  // entries above, at or above the threshold
+  uint32_t need = 0, before = 0;
+  bool all = false;
+  __device__ __forceinline__ MemberWave(int n, float thr)
+      : n(n), nan_thr(thr != thr), th(thr != thr ? __builtin_huge_valf() : thr) {}
+  // A step's entries, from position p0 on (4 per lane; step: its first).
+  __device__ __forceinline__ void rewrite(float (&x)[4], int p0, int step) const {
+    if (nan_thr) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[c] = x[c] != x[c] ? __builtin_huge_valf() : -__builtin_huge_valf();
+    }
+    if (step + 4 * kWave > n) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[c] = p0 + c < n ? x[c] : -__builtin_huge_valf();
+    }
+  }
+  __device__ __forceinline__ void count(const float (&x)[4]) {
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      gt += !(x[c] <= th) ? 1u : 0u;
+      ge += !(x[c] < th) ? 1u : 0u;
+    }
+  }
+  __device__ __forceinline__ void counted(int k) {
+    gt = wave_read_lane(wave_inclusive_sum(gt), kWave - 1);
+    ge = wave_read_lane(wave_inclusive_sum(ge), kWave - 1);
+    if (th == -__builtin_huge_valf()) ge = static_cast<uint32_t>(n);
+    need = static_cast<uint32_t>(k) - gt;  // equal entries to take
+    all = ge - gt == need;
+  }
+  __device__ __forceinline__ void write(uint8_t* out, const float (&x)[4], int p0) {
+    uint32_t w = 0;
+    if (all) {
+#pragma unroll
+      for (int c = 0; c < 4; ++c) w |= !(x[c] < th) ? 1u << (8 * c) : 0u;
+    } else {
+      uint32_t eq = 0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) eq += (p0 + c < n && x[c] == th) ? 1u : 0u;
+      const uint32_t incl = wave_inclusive_sum(eq);
+      uint32_t rank = before + incl - eq;
+      before += wave_read_lane(incl, kWave - 1);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        if (x[c] == th) w |= rank++ < need ? 1u << (8 * c) : 0u;
+        else w |= !(x[c] < th) ? 1u << (8 * c) : 0u;
+      }
+    }
+    store_members(out, p0, n, w);
+  }
+};
+
 // Writes the exactly-k index set of a row whose keys `chunk(j, kk)` yields
 // chunk by chunk (chunk j covers positions (j*NT + tid)*4 .. +3), in
 // ascending index order.  Position of a selected element =
@@ -423,9 +537,10 @@ __device__ __forceinline__ void load_keys4(const float* __restrict__ src, int64_
 // ---------------------------------------------------------------------------
 // Keys plus ~30 working registers fit 64 VGPRs up to V = 32: blocks of up to
 // 512 threads ask for 8 waves per SIMD there, so that four rows share a CU.
-// NEG (threshold only): rows that hold -inf in number, masked score rows.
-template <int NT, int V, int P1, bool RAGGED, bool NEG = false>
-__global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void topk_reg_kernel(SelectArgs a) {
+// MEM (no indices): the row's member bytes too, for rows that may hold -inf in
+// number (masked score rows).
+template <int NT, int V, int P1, bool RAGGED, bool MEM = false>
+__global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void topk_reg_kernel(SelectArgs a) {
   static_assert(V % 4 == 0 && NT % kWave == 0 && NT <= 1024, "block shape");
   static_assert(P1 == 11 || P1 == 12, "first digit width");
   constexpr int NCH = V / 4;
@@ -538,7 +653,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void to
   uint32_t thr_key = 0, krem = 0;
   bool keys_in_regs = false, done = false;
   if (tid == 0) ncand = 0u;
-  if (NEG && tid == 0) ninf = 0u;
+  if (MEM && tid == 0) ninf = 0u;
   // Rows of up to 16 values per thread search by value bins first; longer
   // register rows (32 per thread) have no registers to spare for it and go
   // straight to the radix passes.
@@ -569,10 +684,10 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void to
     }
   };
   block_range();
-  // -inf queues at one counter of a histogram, entry by entry.  Under NEG it
+  // -inf queues at one counter of a histogram, entry by entry.  Under MEM it
   // is counted from the registers: a row with fewer than k entries above it
   // has it as the k-th largest, and any other row is binned without it.
-  const bool neg = NEG && !(lo > -__builtin_huge_valf());
+  const bool neg = MEM && !(lo > -__builtin_huge_valf());
   if (!(lo > -__builtin_huge_valf()) || !(hi < __builtin_huge_valf())) {
     // An infinite value (block-uniform, rare): the finite range instead.
     block_sync_lds();  // every wave has read red
@@ -590,9 +705,15 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void to
       hi = fmaxf(hi, fin ? x : -__builtin_huge_valf());
     });
     block_range();
-    if (neg && static_cast<uint32_t>(k) > static_cast<uint32_t>(nv) - ninf) {
-      if (tid == 0) a.thr[row] = -__builtin_huge_valf();
-      return;
+    if constexpr (MEM) {
+      const uint32_t above = static_cast<uint32_t>(nv) - ninf;
+      if (neg && static_cast<uint32_t>(k) > above) {
+        if (tid == 0) a.thr[row] = -__builtin_huge_valf();
+        to_keys();
+        emit_members<NT, NCH>(a.member + row * a.n, nv, key, float_to_key(-__builtin_huge_valf()),
+                              static_cast<uint32_t>(k) - above, wsum);
+        return;
+      }
     }
   }
   // Stage 2: NBV bins linear in value between lo and hi.  Bins follow the
@@ -644,7 +765,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void to
     block_sync_lds();
     // Threshold only: the other waves exit now, so their registers take the
     // next rows' loads.
-    if (a.idx == nullptr && tid >= kWave) return;
+    if (!MEM && a.idx == nullptr && tid >= kWave) return;
     if (tid < kWave) {
       uint32_t tk, ngt;
       if (bcnt <= static_cast<uint32_t>(kWave)) {
@@ -665,7 +786,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void to
         for (uint32_t i = lane; i < bcnt; i += kWave) g += (cand[i] > tk) ? 1u : 0u;
         ngt = wave_read_lane(wave_inclusive_sum(g), kWave - 1);
       }
-      if (a.idx == nullptr) {
+      if (!MEM && a.idx == nullptr) {
         if (tid == 0) a.thr[row] = key_to_float(tk);
         return;
       }
@@ -722,7 +843,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void to
         });
         block_sync_lds();
         const uint32_t n_c = cnt;
-        if (a.idx == nullptr) {
+        if (!MEM && a.idx == nullptr) {
           if (tid >= kWave) return;
           const uint32_t tk = wave_select_cand(cand, n_c, prefix, S1, krem, hist);
           if (tid == 0) a.thr[row] = key_to_float(tk);
@@ -746,7 +867,10 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !NEG) ? 8 : 4) void to
   }
   if (tid == 0) a.thr[row] = key_to_float(thr_key);
 
-  if (a.idx != nullptr) {
+  if constexpr (MEM) {
+    if (!keys_in_regs) to_keys();
+    emit_members<NT, NCH>(a.member + row * a.n, nv, key, thr_key, krem, wsum);
+  } else if (a.idx != nullptr) {
     if (!keys_in_regs) to_keys();
     int32_t* out = a.idx + row * static_cast<int64_t>(k);
     emit_indices<NT>(out, nch, thr_key, krem, wsum, [&](int64_t j, uint32_t(&kk)[4]) {
@@ -869,7 +993,7 @@ constexpr int kFinGather = 64;   // kept values of one finishing bin ranked in r
 // Eight blocks per CU (at most 64 VGPRs; the LDS columns allow eight): at
 // config 4 thresholds 101 -> 98 us, with indices 156 -> 152, the bitmask
 // 129 -> 127 against six (the bitmask and index forms spill a few SGPRs).
-template <int NT, bool RAGGED, bool IDX, bool MASK = false, bool NEG = false>  // NEG: as in topk_reg_kernel
+template <int NT, bool RAGGED, bool IDX, bool MASK = false, bool NEG = false>  // NEG: rows that may hold -inf in number
 __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
   // IDX: exactly-k indices; MASK: the selection bitmask (a.mask), both from
   // the row's flag bitmap below.
@@ -1495,8 +1619,8 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
 // value costs one min/max, one fma + med3 + convert for its bin (kept, 8 bits
 // each, for the gather) and one LDS add (config 2 standalone: 222 -> 177 us,
 // 60 -> 75% of HBM peak).
-template <int V, bool RAGGED, bool NEG = false>  // NEG: as in topk_reg_kernel
-__global__ __launch_bounds__(256, V <= 16 ? (NEG ? 6 : 8) : (V <= 32 ? (NEG ? 5 : 6) : 4)) void topk_wave_kernel(
+template <int V, bool RAGGED, bool MEM = false>  // MEM: as in topk_reg_kernel
+__global__ __launch_bounds__(256, V <= 16 ? (MEM ? 6 : 8) : (V <= 32 ? (MEM ? 5 : 6) : 4)) void topk_wave_kernel(
     SelectArgs a) {
   static_assert(V % 4 == 0 && V >= 4 && V <= 64, "values per lane");
   constexpr int NCH = V / 4;  // float4 chunks per lane; chunk j covers 256 entries
@@ -1620,6 +1744,21 @@ __global__ __launch_bounds__(256, V <= 16 ? (NEG ? 6 : 8) : (V <= 32 ? (NEG ? 5 
     rank = wave_read_lane(rank, src);
     cnt = wave_read_lane(cnt, src);
   };
+  [[maybe_unused]] auto members = [&](float thr) __attribute__((always_inline)) {
+    MemberWave m(nv, thr);
+    auto step = [&](int j, auto&& f) __attribute__((always_inline)) {
+      float x[4] = {v[4 * j], v[4 * j + 1], v[4 * j + 2], v[4 * j + 3]};
+      m.rewrite(x, (j * kWave + lane) * 4, j * kWave * 4);
+      f(x);
+    };
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+      if (j < nch) step(j, [&](const float(&x)[4]) { m.count(x); });
+    m.counted(k);
+#pragma unroll
+    for (int j = 0; j < NCH; ++j)
+      if (j < nch) step(j, [&](const float(&x)[4]) { m.write(a.member + row * a.n, x, (j * kWave + lane) * 4); });
+  };
   // The row's min and max (fminf / fmaxf ignore NaN); a row holding an
   // infinite value (wave-uniform, rare) takes its finite range instead.
   float lo = __builtin_huge_valf(), hi = -__builtin_huge_valf();
@@ -1629,13 +1768,14 @@ __global__ __launch_bounds__(256, V <= 16 ? (NEG ? 6 : 8) : (V <= 32 ? (NEG ? 5 
   });
   lo = wave_extreme_f32<false>(lo);
   hi = wave_extreme_f32<true>(hi);
-  const bool neg = NEG && !(lo > -__builtin_huge_valf());
+  const bool neg = MEM && !(lo > -__builtin_huge_valf());
   if (neg) {
     uint32_t above = 0;
     visit([&](float x, int) { above += x == -__builtin_huge_valf() ? 0u : 1u; });
     above = wave_read_lane(wave_inclusive_sum(above), kWave - 1);
     if (static_cast<uint32_t>(k) > above) {
       if (lane == 0) a.thr[row] = -__builtin_huge_valf();
+      if constexpr (MEM) members(-__builtin_huge_valf());
       return;
     }
   }
@@ -1676,7 +1816,7 @@ __global__ __launch_bounds__(256, V <= 16 ? (NEG ? 6 : 8) : (V <= 32 ? (NEG ? 5 
   [[maybe_unused]] uint32_t nbot = 0;  // -inf entries of this lane
   visit([&](float x, int i) {
     const uint32_t c = bin_of(x);
-    if constexpr (NEG) {
+    if constexpr (MEM) {
       if (x == -__builtin_huge_valf()) ++nbot;
       else atomicAdd(&hist[c], 1u);
     } else {
@@ -1684,7 +1824,7 @@ __global__ __launch_bounds__(256, V <= 16 ? (NEG ? 6 : 8) : (V <= 32 ? (NEG ? 5 
     }
     bp[i >> 2] |= c << (8 * (i & 3));
   });
-  if constexpr (NEG) {  // bin 255 keeps them, added once
+  if constexpr (MEM) {  // bin 255 keeps them, added once
     nbot = wave_inclusive_sum(nbot);
     if (lane == kWave - 1) atomicAdd(&hist[255], nbot);
   }
@@ -1797,115 +1937,55 @@ __global__ __launch_bounds__(256, V <= 16 ? (NEG ? 6 : 8) : (V <= 32 ? (NEG ? 5 
     }
   }
   if (lane == 0) a.thr[row] = key_to_float(tk);
+  if constexpr (MEM) members(key_to_float(tk));
 }
 
 // ---------------------------------------------------------------------------
-// Membership of each entry in its row's top k, one byte each, from the row's
-// k-th largest: entries above it, and the lowest-index ones equal to it up to
-// k.  One wave per row: a first pass counts the entries above and equal (4 per
-// lane and step, 4 steps' loads in flight), a second one, from the cache,
-// writes the bytes; only rows that take part of their equal entries rank them.
-// HBM-bound: the row read, n bytes written (two [4096, 4096] matrices with the
-// -inf triangle, k = 256: 27 us, and 34 for the thresholds before it; 138 us
-// as indices scattered into a zeroed mask).
+// Member bytes from the thresholds, for the rows whose select does not hold
+// them in registers.  One wave per row: a first pass counts the entries above
+// and equal, a second one, from the cache, writes the bytes; 8 loads of 16
+// bytes per lane in flight.  HBM-bound: the row read, n bytes written (two
+// [8000, 8000] matrices with the -inf triangle, k = 1000: 166 us).
 // ---------------------------------------------------------------------------
-// U: steps of 256 entries a lane holds at once (REG: the whole row, read once).
-// In the key order (NaN the largest value, -0 = +0) an entry is above the
-// threshold if !(x <= th), at or above it if !(x < th).  Two rewrites of what
-// was loaded keep that true everywhere: positions past the row read as -inf
-// (below any threshold but -inf, which every entry of the row reaches), and
-// under a NaN threshold NaNs as +inf against +inf, the rest as -inf.
-template <int U, bool REG>
-__global__ __launch_bounds__(256) void member_kernel(SelectArgs a, uint8_t* __restrict__ member) {
+__global__ __launch_bounds__(256) void member_kernel(SelectArgs a) {
+  constexpr int U = 8;           // steps in flight
+  constexpr int CH = 4 * kWave;  // entries per step
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t row = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (row >= a.rows) return;  // whole waves
   const int n = static_cast<int>(a.n);
-  constexpr float kInf = __builtin_huge_valf();
-  const float thr = a.thr[row];
-  const bool tn = thr != thr;
-  const float th = tn ? kInf : thr;
   const char* rb = reinterpret_cast<const char*>(a.scores + row * a.ld);
-  uint8_t* out = member + row * a.n;
   const bool edge = edge_row(a, row, n);
-  constexpr int CH = 4 * kWave;  // entries per step
   const int last4 = (n - 1) & ~3;
-  float x[U][4];
-  auto load = [&](int s) {
-    if (!edge) {
+  MemberWave m(n, a.thr[row]);
+  auto steps = [&](auto&& f) __attribute__((always_inline)) {  // f(x, p0) for every step of the row
+    for (int s = 0; s < n; s += U * CH) {
+      float x[U][4];
+      if (!edge) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const float4 f = load_f4(rb + static_cast<uint32_t>(min(s + u * CH + 4 * lane, last4)) * 4u);
-        x[u][0] = f.x; x[u][1] = f.y; x[u][2] = f.z; x[u][3] = f.w;
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-          x[u][c] = *reinterpret_cast<const float*>(rb + static_cast<uint32_t>(min(s + u * CH + 4 * lane + c, n - 1)) * 4u);
-    }
-    if (tn) {
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) x[u][c] = x[u][c] != x[u][c] ? kInf : -kInf;
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-      if (s + (u + 1) * CH > n) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) x[u][c] = s + u * CH + 4 * lane + c < n ? x[u][c] : -kInf;
-      }
-  };
-  uint32_t gt = 0, ge = 0;
-  for (int s = 0; s < n; s += U * CH) {
-    load(s);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        gt += !(x[u][c] <= th) ? 1u : 0u;
-        ge += !(x[u][c] < th) ? 1u : 0u;
-      }
-  }
-  gt = wave_read_lane(wave_inclusive_sum(gt), kWave - 1);
-  ge = wave_read_lane(wave_inclusive_sum(ge), kWave - 1);
-  if (th == -kInf) ge = static_cast<uint32_t>(n);
-  const uint32_t need = static_cast<uint32_t>(a.k) - gt;  // equal entries to take
-  const bool all = ge - gt == need;
-  uint32_t before = 0;  // equal entries of earlier steps
-  for (int s = 0; s < n; s += U * CH) {
-    if constexpr (!REG) load(s);
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      if (s + u * CH >= n) break;
-      const int p0 = s + u * CH + 4 * lane;
-      uint32_t w = 0;
-      if (all) {
-#pragma unroll
-        for (int c = 0; c < 4; ++c) w |= !(x[u][c] < th) ? 1u << (8 * c) : 0u;
-      } else {
-        uint32_t eq = 0;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) eq += (p0 + c < n && x[u][c] == th) ? 1u : 0u;
-        const uint32_t incl = wave_inclusive_sum(eq);
-        uint32_t rank = before + incl - eq;
-        before += wave_read_lane(incl, kWave - 1);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          if (x[u][c] == th) w |= rank++ < need ? 1u << (8 * c) : 0u;
-          else w |= !(x[u][c] < th) ? 1u << (8 * c) : 0u;
+        for (int u = 0; u < U; ++u) {
+          const float4 q = load_f4(rb + static_cast<uint32_t>(min(s + u * CH + 4 * lane, last4)) * 4u);
+          x[u][0] = q.x; x[u][1] = q.y; x[u][2] = q.z; x[u][3] = q.w;
         }
-      }
-      if (p0 + 4 <= n) {
-        __builtin_memcpy(out + p0, &w, 4);  // any byte alignment
       } else {
-        for (int c = 0; c < 4; ++c)
-          if (p0 + c < n) out[p0 + c] = static_cast<uint8_t>(w >> (8 * c));
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            x[u][c] = *reinterpret_cast<const float*>(
+                rb + static_cast<uint32_t>(min(s + u * CH + 4 * lane + c, n - 1)) * 4u);
       }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (s + u * CH < n) {
+          m.rewrite(x[u], s + u * CH + 4 * lane, s + u * CH);
+          f(x[u], s + u * CH + 4 * lane);
+        }
     }
-  }
+  };
+  steps([&](const float(&x)[4], int) { m.count(x); });
+  m.counted(a.k);
+  steps([&](const float(&x)[4], int p0) { m.write(a.member + row * a.n, x, p0); });
 }
 
 // Rows whose length, stride and base are not all 16-byte granular.
@@ -1914,16 +1994,16 @@ bool ragged(const SelectArgs& a) {
 }
 
 template <int V>
-hipError_t launch_wave(const SelectArgs& a, bool neg, hipStream_t stream) {
+hipError_t launch_wave(const SelectArgs& a, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((a.rows + 3) / 4));
-  if (neg) hipLaunchKernelGGL((topk_wave_kernel<V, true, true>), grid, dim3(256), 0, stream, a);
+  if (a.member != nullptr) hipLaunchKernelGGL((topk_wave_kernel<V, true, true>), grid, dim3(256), 0, stream, a);
   else if (ragged(a)) hipLaunchKernelGGL((topk_wave_kernel<V, true>), grid, dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((topk_wave_kernel<V, false>), grid, dim3(256), 0, stream, a);
   return hipGetLastError();
 }
 
 template <int NT, int V, int P1>
-hipError_t launch_reg(const SelectArgs& a, bool neg, hipStream_t stream) {
+hipError_t launch_reg(const SelectArgs& a, hipStream_t stream) {
   // Causal rows: a 2-D grid (batch element, row) whose blocks need no
   // division to find their row (register rows are at most 32768 long, so
   // causal_T fits the grid's y range).
@@ -1932,7 +2012,7 @@ hipError_t launch_reg(const SelectArgs& a, bool neg, hipStream_t stream) {
   const dim3 grid = two_d ? dim3(static_cast<unsigned>(nb), static_cast<unsigned>(a.causal_T))
                           : dim3(static_cast<unsigned>(a.rows));
   if constexpr (V <= 16) {
-    if (neg) {
+    if (a.member != nullptr) {
       hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, true, true>), grid, dim3(NT), 0, stream, a);
       return hipGetLastError();
     }
@@ -1956,9 +2036,9 @@ bool bracket_fits(int64_t cap, int k) {
 }
 
 template <bool IDX, bool MASK>
-hipError_t launch_bracket(const SelectArgs& a, bool neg, hipStream_t stream) {
+hipError_t launch_bracket(const SelectArgs& a, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>(a.rows));
-  if (!IDX && !MASK && neg)
+  if (!IDX && !MASK && a.member != nullptr)
     hipLaunchKernelGGL((topk_bracket_kernel<256, true, false, false, true>), grid, dim3(256), 0, stream, a);
   else if (ragged(a))
     hipLaunchKernelGGL((topk_bracket_kernel<256, true, IDX, MASK>), grid, dim3(256), 0, stream, a);
@@ -1973,15 +2053,26 @@ hipError_t launch_stream(const SelectArgs& a, hipStream_t stream) {
   return hipGetLastError();
 }
 
-// neg: the rows may hold -inf in number (thresholds of masked score rows: two
-// [4096, 4096] matrices with the -inf triangle, k = 256: 72 -> 35 us; six of
-// 1800, k = 150: 101 -> 33).  The kernels that count it apart are instances of
-// their own, for any alignment: in the plain ones the test costs rows without
-// -inf up to a quarter (spilled registers: 16384 x 4096, 45 -> 56 us).
+hipError_t launch_member(const SelectArgs& a, hipStream_t stream) {
+  hipLaunchKernelGGL(member_kernel, dim3(static_cast<unsigned>((a.rows + 3) / 4)), dim3(256), 0, stream, a);
+  return hipGetLastError();
+}
+
+// member: also the top-k sets as bytes (no indices, whole rows), for rows that
+// may hold -inf in number: masked score rows, where counting it one by one in
+// a histogram takes longer than the rest of the select (thresholds of two
+// [4096, 4096] matrices with the -inf triangle, k = 256: 72 -> 35 us without).
+// Rows of up to 8192 that a wave or a block holds in registers write the bytes
+// from there (MEM instances, any alignment: 45 us for both against
+// 35 + 27 through member_kernel); longer ones, and the bracket kernel's, take
+// member_kernel.  The plain instances stay without it: the test and what it
+// keeps alive cost rows without -inf up to a quarter (16384 x 4096: 45 -> 56 us).
 hipError_t launch_select(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
-                         int64_t causal_T, float* thr, int32_t* idx, bool neg, hipStream_t stream) {
+                         int64_t causal_T, float* thr, int32_t* idx, uint8_t* member,
+                         hipStream_t stream) {
   if (rows == 0) return hipSuccess;
   SelectArgs a{scores, rows, n, ld, k, causal_T, thr, idx, causal_T > 0 ? rows / causal_T : 0};
+  a.member = member;
   const int64_t cap = causal_T > 0 ? (causal_T < n ? causal_T : n) : n;
   // Rows above 8K entries use a 12-bit first digit: hot digits of real
   // score rows spread over twice the bins (fewer same-address LDS atomics)
@@ -1992,43 +2083,37 @@ hipError_t launch_select(const float* scores, int64_t rows, int64_t n, int64_t l
   // leave 4 waves per SIMD and the block kernel is faster: 43 vs 45 us).
   // With indices: rows of at most 16 chunks (the per-thread position masks
   // are 64 bits).
-  if (bracket_fits(cap, k) && (idx == nullptr || cap <= kBracketIdxMaxN))
-    return idx != nullptr ? launch_bracket<true, false>(a, false, stream)
-                          : launch_bracket<false, false>(a, neg, stream);
-  if (idx == nullptr && cap <= 2048) {
-    if (cap <= 512) return launch_wave<8>(a, neg, stream);
-    if (cap <= 1024) return launch_wave<16>(a, neg, stream);
-    return launch_wave<32>(a, neg, stream);
+  if (bracket_fits(cap, k) && (idx == nullptr || cap <= kBracketIdxMaxN)) {
+    const hipError_t e = idx != nullptr ? launch_bracket<true, false>(a, stream)
+                                        : launch_bracket<false, false>(a, stream);
+    return e == hipSuccess && member != nullptr ? launch_member(a, stream) : e;
   }
-  if (cap <= 512) return launch_reg<128, 4, 11>(a, neg, stream);
-  if (cap <= 1024) return launch_reg<128, 8, 11>(a, neg, stream);
-  if (cap <= 2048) return launch_reg<256, 8, 11>(a, neg, stream);
-  if (cap <= 4096) return launch_reg<256, 16, 11>(a, neg, stream);
-  if (cap <= 8192) return launch_reg<512, 16, 11>(a, neg, stream);
-  if (cap <= 16384) return launch_reg<512, 32, 12>(a, neg, stream);
-  if (cap <= 32768) return launch_reg<1024, 32, 12>(a, neg, stream);
-  return launch_stream(a, stream);
+  if (idx == nullptr && cap <= 2048) {
+    if (cap <= 512) return launch_wave<8>(a, stream);
+    if (cap <= 1024) return launch_wave<16>(a, stream);
+    return launch_wave<32>(a, stream);
+  }
+  if (cap <= 512) return launch_reg<128, 4, 11>(a, stream);
+  if (cap <= 1024) return launch_reg<128, 8, 11>(a, stream);
+  if (cap <= 2048) return launch_reg<256, 8, 11>(a, stream);
+  if (cap <= 4096) return launch_reg<256, 16, 11>(a, stream);
+  if (cap <= 8192) return launch_reg<512, 16, 11>(a, stream);
+  const hipError_t e = cap <= 16384   ? launch_reg<512, 32, 12>(a, stream)
+                       : cap <= 32768 ? launch_reg<1024, 32, 12>(a, stream)
+                                      : launch_stream(a, stream);
+  return e == hipSuccess && member != nullptr ? launch_member(a, stream) : e;
 }
 
 }  // namespace
 
 hipError_t launch_topk(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
                        int64_t causal_T, float* thr, int32_t* idx, hipStream_t stream) {
-  return launch_select(scores, rows, n, ld, k, causal_T, thr, idx, false, stream);
+  return launch_select(scores, rows, n, ld, k, causal_T, thr, idx, nullptr, stream);
 }
 
 hipError_t launch_topk_member(const float* scores, int64_t rows, int64_t n, int64_t ld, int k,
                               float* thr, uint8_t* member, hipStream_t stream) {
-  if (rows == 0) return hipSuccess;
-  const hipError_t e = launch_select(scores, rows, n, ld, k, 0, thr, nullptr, true, stream);
-  if (e != hipSuccess) return e;
-  const SelectArgs a{scores, rows, n, ld, k, 0, thr, nullptr, 0};
-  const dim3 grid(static_cast<unsigned>((rows + 3) / 4));
-  if (n <= 1024) hipLaunchKernelGGL((member_kernel<4, true>), grid, dim3(256), 0, stream, a, member);
-  else if (n <= 2048) hipLaunchKernelGGL((member_kernel<8, true>), grid, dim3(256), 0, stream, a, member);
-  else if (n <= 4096) hipLaunchKernelGGL((member_kernel<16, true>), grid, dim3(256), 0, stream, a, member);
-  else hipLaunchKernelGGL((member_kernel<8, false>), grid, dim3(256), 0, stream, a, member);
-  return hipGetLastError();
+  return launch_select(scores, rows, n, ld, k, 0, thr, nullptr, member, stream);
 }
 
 hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t ld, int k,
@@ -2044,8 +2129,8 @@ hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t l
     SelectArgs a{scores, rows, T, ld, k, T, thr, nullptr, B};
     a.mask = mask;
     a.ldm = ldm;
-    return T <= kBracketIdxMaxN ? launch_bracket<false, true>(a, false, stream)
-                                : launch_bracket<false, false>(a, false, stream);
+    return T <= kBracketIdxMaxN ? launch_bracket<false, true>(a, stream)
+                                : launch_bracket<false, false>(a, stream);
   }
   const hipError_t e = launch_topk(scores, rows, T, ld, k, T, thr, nullptr, stream);
   if (e != hipSuccess) return e;
