@@ -272,9 +272,14 @@ def _split_is_faster(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> bool:
 
 def dsa_forward_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
     """Forward for any shape: the fused kernel where one exists (T <= 2048)
-    and is not expected to be slower (dsa_forward_uses_split), else the split
-    kernels.  Both are gfx950 HIP; nothing runs on the CPU."""
-    if Q.shape[1] <= L.lib().dsa_fused_max_T() and not _split_is_faster(q_idx, k_idx, w_idx, Q, K, V, top_k):
+    and is not expected to be slower (dsa_forward_uses_split) or the split
+    workspace does not fit, else the split kernels.  Both are gfx950 HIP; nothing runs on the CPU."""
+    if Q.shape[1] <= L.lib().dsa_fused_max_T():
+        if _split_is_faster(q_idx, k_idx, w_idx, Q, K, V, top_k):
+            try:
+                return dsa_split_hip(q_idx, k_idx, w_idx, Q, K, V, top_k)
+            except (torch.OutOfMemoryError, L.DSAUnsupported):
+                pass  # the fused kernel keeps no [B, T, T] scores in HBM
         try:
             return dsa_fused_hip(q_idx, k_idx, w_idx, Q, K, V, top_k)
         except L.DSAUnsupported:

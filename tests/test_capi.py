@@ -484,3 +484,22 @@ def test_split_forward_entry_checks_arguments():
     assert call(a18=None) == L.DSA_EINVAL
     assert call(a8=0) == L.DSA_OK
     assert call(a7=L.DSA_BF16, a8=0, a9=4096, a12=3, a13=128, a14=128) == L.DSA_OK
+
+
+@pytest.mark.parametrize("error", [torch.OutOfMemoryError, L.DSAUnsupported])
+def test_forward_takes_fused_where_the_split_workspace_does_not_fit(monkeypatch, error):
+    """A call that the rule gives to the split forward still runs where the
+    [B, T, T] workspace cannot be had; past the fused kernel's T it raises."""
+    import dsa_attention as DA
+
+    def split(*a):
+        raise error("no workspace")
+
+    monkeypatch.setattr(DA, "_split_is_faster", lambda *a: True)
+    monkeypatch.setattr(DA, "dsa_split_hip", split)
+    monkeypatch.setattr(DA, "dsa_fused_hip", lambda *a: "fused")
+    x = torch.empty(1, L.lib().dsa_fused_max_T(), 1, 64)
+    assert DA.dsa_forward_hip(x, x, x, x, x, x, 4) == "fused"
+    x = torch.empty(1, x.shape[1] + 1, 1, 64)
+    with pytest.raises(error):
+        DA.dsa_forward_hip(x, x, x, x, x, x, 4)
