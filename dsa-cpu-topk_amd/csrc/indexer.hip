@@ -449,8 +449,9 @@ __global__ __launch_bounds__((64 * qtile_waves<Tag, DI, NQ>())) void indexer_qti
 // Positive scales leave the ReLU: q's inverse is folded into w, k's multiplies
 // each finished score.  A super-block whose q rows, w rows or k rows hold a
 // non-finite value, or a scale too far out for that folding (rows beyond
-// 2^+-60, w outside [2^-40, 2^60]), is summed in plain fp32 from memory
-// instead: the split would turn inf into inf - inf.
+// 2^+-60, w outside [2^-40, 2^30]), is summed in plain fp32 from memory
+// instead: the split would turn inf into inf - inf.  Before k's scale is undone
+// a sum is at most |w||q| 2^15 DI HI < 2^30 2^61 2^15 2^18, a finite float.
 // ---------------------------------------------------------------------------
 template <int DI>
 size_t split_lds_bytes(QTileShape sh) {
@@ -544,7 +545,7 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
       const int t = t0 + tl;
       const float wv = (t < T && h < HI) ? w[static_cast<int64_t>(t) * a.ldw + h] : 0.f;
       const uint32_t wb = __float_as_uint(wv) & 0x7fffffffu;
-      if (wb != 0u && (wb < (127u - 40u) << 23 || wb > (127u + 60u) << 23)) qbad = 1u;
+      if (wb != 0u && (wb < (127u - 40u) << 23 || wb > (127u + 30u) << 23)) qbad = 1u;
       const int at = ((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3);
       wf[at] = wv * qs[at];
     }

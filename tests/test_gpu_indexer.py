@@ -387,3 +387,19 @@ def test_fp32_pieces_nonfinite_rows(dev):
     assert bool(((out.double() - ref).abs()[fin] <= 1e-4 + 1e-4 * ref.abs()[fin]).all())
     # 64-query rows away from the planted queries, keys before the planted keys
     assert torch.equal(out[0, :32], clean[0, :32])
+
+
+def test_fp32_pieces_large_weights_times_large_rows(dev):
+    """A finite score of large q rows and weights and small k rows stays
+    finite (k's scale is undone last; the product before it would pass fp32's
+    range, so such weights take the plain fp32 sum: DI + HI + 2 roundings)."""
+    T, HI, DI = 70, 8, 64
+    q, k, w, *_ = O.make_inputs(1, T, HI, DI, 1, 1, 1, seed0=11)
+    q, k, w = q * 2.0 ** 56, k * 2.0 ** -40, w * 2.0 ** 55
+    out = indexer_scores_hip(q.to(dev), k.to(dev), w.to(dev)).cpu()
+    ref = O.indexer_scores(q, k, w)
+    l1 = torch.einsum("bth,bths->bts", w.double().abs(),
+                      torch.einsum("bthd,bsd->bths", q.double().abs(), k.double().abs()))
+    causal = torch.ones(T, T, dtype=torch.bool).tril()
+    bound = (DI + HI + 2) * 2.0 ** -24 * l1
+    assert bool(((out.double() - ref).abs() <= bound)[:, causal].all())
