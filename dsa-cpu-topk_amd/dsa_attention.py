@@ -95,8 +95,8 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
     the same output, bit for bit.
     kernel="tiled" (or tiled=True) / "staged" / "mask" / "dense" / "gather" runs that
     kernel at any T (AssertionError for shapes it does not cover); "staged"
-    is the dense one where the library would otherwise have staged (T >= 3072)
-    and now takes it."""
+    is the dense one for the shapes of the staged kernel that the library gives
+    to the dense one (T >= 3072)."""
     L.require_gpu(scores, threshold, Q, K, V)
     B, T, _ = scores.shape
     HQ, DQ = Q.shape[-2], Q.shape[-1]
@@ -118,9 +118,11 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
         return _sparse_attention_mask(scores, thr, Q, K, V, out)
     code = L.dtype_code(dt)
     if kernel is None or (kernel == "staged" and T >= 3072):
+        # a forced staged kernel: top_k 0, the rule that takes staged shapes only
+        k = int(top_k) if kernel is None else 0
         with L.on_device(Q.device):
             kernel = {0: kernel, 1: "dense", 2: "gather"}[
-                L.lib().dsa_sparse_attn_pick(code, B, T, HQ, DQ, DV, int(top_k))]
+                L.lib().dsa_sparse_attn_pick(code, B, T, HQ, DQ, DV, k)]
     if kernel == "dense":
         nws = L.lib().dsa_sparse_attn_dense_workspace_bytes(code, B, T, HQ, DQ, DV)
         ws = torch.empty(max(nws, 16), device=Q.device, dtype=torch.uint8)

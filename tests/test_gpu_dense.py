@@ -158,3 +158,12 @@ def test_forward_picks_split_or_fused(dev, B, T, k, HI, DI, HQ, D, dtype, split)
     other = (DA.dsa_fused_hip if split else DA.dsa_split_hip)(*ins, k)
     off = (got - other).abs().amax(dim=(-1, -2)) > 2 * bound(*(x.cpu() for x in ins[3:]), T)
     assert int(off.sum()) <= max(2, B * T // 1000)
+
+
+def test_forced_staged_refuses_what_it_refused(dev):
+    """A staged kernel asked for by name stays refused for other shapes,
+    whatever top_k says of the dense kernel."""
+    x = torch.zeros(1, 3072, 4, 64, device=dev, dtype=BF)
+    s, t = torch.zeros(1, 3072, 3072, device=dev), torch.zeros(1, 3072, 1, device=dev)
+    with pytest.raises(L.DSAUnsupported):
+        sparse_attention_hip(s, t, x, x, x, kernel="staged", top_k=3072)
