@@ -25,8 +25,8 @@ import math
 import torch
 
 import _dsa_lib as L
-from lightning_indexer import indexer_scores_hip, indexer_scores_torch  # noqa: F401
-from topk_threshold import topk_threshold, topk_threshold_mask  # noqa: F401
+from lightning_indexer import indexer_scores_hip, indexer_scores_torch
+from topk_threshold import topk_threshold, topk_threshold_mask
 
 
 # ---------------------------------------------------------------------------
@@ -96,7 +96,8 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
     kernel="tiled" (or tiled=True) / "staged" / "mask" / "dense" / "gather" runs that
     kernel at any T (AssertionError for shapes it does not cover); "staged"
     is the dense one for the shapes of the staged kernel that the library gives
-    to the dense one (T >= 3072)."""
+    to the dense one (T >= 3072).  Where the dense kernel's workspace does not
+    fit, a call that did not ask for it by name takes one of the others."""
     L.require_gpu(scores, threshold, Q, K, V)
     B, T, _ = scores.shape
     HQ, DQ = Q.shape[-2], Q.shape[-1]
@@ -121,11 +122,20 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
         # a forced staged kernel: top_k 0, the rule that takes staged shapes only
         k = int(top_k) if kernel is None else 0
         with L.on_device(Q.device):
-            kernel = {0: kernel, 1: "dense", 2: "gather"}[
+            picked = {0: kernel, 1: "dense", 2: "gather"}[
                 L.lib().dsa_sparse_attn_pick(code, B, T, HQ, DQ, DV, k)]
-    if kernel == "dense":
+    else:
+        picked = kernel
+    if picked == "dense":
         nws = L.lib().dsa_sparse_attn_dense_workspace_bytes(code, B, T, HQ, DQ, DV)
-        ws = torch.empty(max(nws, 16), device=Q.device, dtype=torch.uint8)
+        try:
+            ws = torch.empty(max(nws, 16), device=Q.device, dtype=torch.uint8)
+        except torch.OutOfMemoryError:
+            if kernel == "dense":
+                raise
+            picked = kernel  # the other kernels need little or no workspace
+    kernel = picked
+    if kernel == "dense":
         L.check(L.lib().dsa_sparse_attn_dense(
             scores.data_ptr(), T, thr.data_ptr(), Q.data_ptr(), K.data_ptr(), V.data_ptr(), code,
             B, T, HQ, DQ, DV, 1.0 / math.sqrt(DQ), out.data_ptr(), ws.data_ptr(), nws,
@@ -224,7 +234,20 @@ def dsa_split_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
     out = torch.empty(B, T, HQ, DV, device=Q.device, dtype=torch.float32)
     with L.on_device(Q.device):
         nws = L.lib().dsa_split_workspace_bytes(code, B, T, HQ, DQ, DV, k)
-        ws = torch.empty(max(nws, 16), device=Q.device, dtype=torch.uint8)
+        try:
+            ws = torch.empty(max(nws, 16), device=Q.device, dtype=torch.uint8)
+        except torch.OutOfMemoryError:
+            ws = None
+        if ws is None:
+            # The stages apart take the same scores, but not in one piece, and
+            # do without the dense kernel's workspace.
+            scores = indexer_scores_hip(q_idx, k_idx, w_idx, write_upper=False)
+            if L.lib().dsa_sparse_attn_uses_mask(code, T, HQ, DQ, DV):
+                _, mask = topk_threshold_mask(scores, k)
+                del scores
+                return sparse_attention_from_mask(mask, Q, K, V, out=out)
+            return sparse_attention_hip(scores, topk_threshold(scores, k, causal=True), Q, K, V,
+                                        out=out, top_k=k)
         rc = L.lib().dsa_split_forward(
             q_idx.data_ptr(), k_idx.data_ptr(), w_idx.data_ptr(), L.dtype_code(it), Q.data_ptr(),
             K.data_ptr(), V.data_ptr(), code, B, T, HI, DI, HQ, DQ, DV, k, 1.0 / math.sqrt(DQ),

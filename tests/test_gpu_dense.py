@@ -160,6 +160,35 @@ def test_forward_picks_split_or_fused(dev, B, T, k, HI, DI, HQ, D, dtype, split)
     assert int(off.sum()) <= max(2, B * T // 1000)
 
 
+@pytest.mark.parametrize("B,T,k,HQ,D,dtype", [(2, 2048, 256, 16, 128, HF), (1, 4200, 300, 4, 64, BF)])
+def test_forward_without_its_workspace(dev, monkeypatch, B, T, k, HQ, D, dtype):
+    """Where the split forward's workspace and the dense kernel's cannot be
+    had, the stages run apart on the kernels that need none; a dense kernel
+    asked for by name raises."""
+    from dsa_attention import dsa_split_hip, selection_mask, sparse_attention_from_mask
+    from lightning_indexer import indexer_scores_hip
+    from topk_threshold import topk_threshold
+
+    ins = tuple(x.to(dev) for x in O.make_inputs(B, T, 4, 32, HQ, D, D, dtype=dtype))
+    sc = indexer_scores_hip(*ins[:3], write_upper=False)
+    thr = topk_threshold(sc, k, causal=True)
+    if L.lib().dsa_sparse_attn_uses_mask(L.dtype_code(dtype), T, HQ, D, D):
+        want = sparse_attention_from_mask(selection_mask(sc, thr), *ins[3:])
+    else:
+        want = sparse_attention_hip(sc, thr, *ins[3:], kernel="gather")
+    empty = torch.empty
+
+    def no_workspace(*a, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no workspace")
+        return empty(*a, **kw)
+
+    monkeypatch.setattr(torch, "empty", no_workspace)
+    assert torch.equal(dsa_split_hip(*ins, k), want)
+    with pytest.raises(torch.OutOfMemoryError):
+        sparse_attention_hip(sc, thr, *ins[3:], kernel="dense")
+
+
 def test_forced_staged_refuses_what_it_refused(dev):
     """A staged kernel asked for by name stays refused for other shapes,
     whatever top_k says of the dense kernel."""
