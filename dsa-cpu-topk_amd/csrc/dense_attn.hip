@@ -84,7 +84,8 @@ __device__ __forceinline__ bool split_scale_v(uint32_t maxbits, int& sh) {
 // magnitude (held in registers between the maximum and the conversion), and
 // record that magnitude.
 //
-// The others write the selection bitmask: one wave per row, rows longest first, each causal score read once (nontemporal, 16 loads
+// The others (none if the select has written the mask: scores null) write the
+// selection bitmask: one wave per row, rows longest first, each causal score read once (nontemporal, 16 loads
 // in flight per lane), as selection_mask_kernel (tile_attn.hip) does.
 // ---------------------------------------------------------------------------
 struct PrepareArgs {
@@ -885,7 +886,8 @@ hipError_t dispatch_redo(const RedoArgs& a, int E, hipStream_t stream) {
 template <int D>
 hipError_t launch_prepare(PrepareArgs a, hipStream_t stream) {
   a.nconv = D > 0 ? static_cast<uint32_t>(a.B * ((a.T + 63) / 64) * a.HQ) : 0u;
-  const int64_t nblk = a.nconv + (a.B * a.T + 3) / 4;
+  const int64_t nblk = a.nconv + (a.scores != nullptr ? (a.B * a.T + 3) / 4 : 0);
+  if (nblk == 0) return hipSuccess;
   hipLaunchKernelGGL((prepare_kernel<D>), dim3(static_cast<unsigned>(nblk)), dim3(256), 0, stream, a);
   return hipGetLastError();
 }

@@ -130,7 +130,8 @@ hipError_t launch_staged_attn(const float* scores, int64_t ld, const float* thr,
 
 // The same attention computed densely on MFMA tiles with fp32 probabilities
 // (dense_attn.hip): DQ = DV in {64, 128}.
-// Needs a workspace of dense_attn_workspace bytes, 16-byte aligned.
+// Needs a workspace of dense_attn_workspace bytes, 16-byte aligned, which begins
+// with the selection bitmask ([B*T][ceil(T/64)] words; scores null: already there).
 bool dense_attn_supported(int dtype, int64_t T, int HQ, int DQ, int DV);
 int64_t dense_attn_workspace(int dtype, int64_t B, int64_t T, int HQ, int D);
 // The kernel expected to be fastest for a shape whose queries select about

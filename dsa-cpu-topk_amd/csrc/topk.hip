@@ -59,9 +59,9 @@ struct SelectArgs {
   float* thr;
   int32_t* idx;
   int64_t nbatch;  // rows / causal_T in causal mode (set by the host)
-  // Causal rows only, threshold-only bracket kernel: also the row's
-  // selection bitmask (the words selection_mask_kernel writes), ldm words
-  // per row; null: none.
+  // Causal rows only, threshold-only bracket kernel and the wave kernel's BITS
+  // instances: also the row's selection bitmask (the words
+  // selection_mask_kernel writes), ldm words per row; null: none.
   uint64_t* mask = nullptr;
   int64_t ldm = 0;
   // MEM instances and member_kernel: one byte per entry, n per row.
@@ -1619,7 +1619,11 @@ __global__ __launch_bounds__(NT, 8) void topk_bracket_kernel(SelectArgs a) {
 // value costs one min/max, one fma + med3 + convert for its bin (kept, 8 bits
 // each, for the gather) and one LDS add (config 2 standalone: 222 -> 177 us,
 // 60 -> 75% of HBM peak).
-template <int V, bool RAGGED, bool MEM = false>  // MEM: as in topk_reg_kernel
+// MEM: as in topk_reg_kernel.  BITS (causal rows): the row's selection bitmask
+// too, from the registers, which saves the mask kernel's launch and second read
+// of the scores (split forward B = 4, T = 2048, HI = 8, DI = 64, HQ = 8, D = 64,
+// k = 128 bf16: 92.6 -> 86.4 us).
+template <int V, bool RAGGED, bool MEM = false, bool BITS = false>
 __global__ __launch_bounds__(256, V <= 16 ? (MEM ? 6 : 8) : (V <= 32 ? (MEM ? 5 : 6) : 4)) void topk_wave_kernel(
     SelectArgs a) {
   static_assert(V % 4 == 0 && V >= 4 && V <= 64, "values per lane");
@@ -1644,7 +1648,7 @@ __global__ __launch_bounds__(256, V <= 16 ? (MEM ? 6 : 8) : (V <= 32 ? (MEM ? 5 
   const int k = a.k;
   if (nvalid < k) {
     if (lane == 0) a.thr[row] = -__builtin_huge_valf();
-    return;
+    if constexpr (!BITS) return;
   }
   uint32_t* hist = whist[wid];
   uint32_t* gl = wgl[wid];
@@ -1673,6 +1677,33 @@ __global__ __launch_bounds__(256, V <= 16 ? (MEM ? 6 : 8) : (V <= 32 ? (MEM ? 5 
           const uint32_t off = static_cast<uint32_t>(min((j * kWave + lane) * 4 + c, nv - 1)) * 4u;
           v[4 * j + c] = *reinterpret_cast<const float*>(rb + off);
         }
+    }
+  }
+  // The row's mask words, 64 keys each, up to the one of position t | 127: a
+  // chunk's eight lanes gather their four flags each into 32 bits (DPP), which
+  // the first of them stores.
+  [[maybe_unused]] auto bits = [&](float thr) __attribute__((always_inline)) {
+    uint32_t* __restrict__ mrow = reinterpret_cast<uint32_t*>(a.mask + row * a.ldm);
+    const int nd = min(static_cast<int>((a.causal_T + 63) >> 6), (((nv - 1) | 127) >> 6) + 1) * 2;  // dwords
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      if (j * 8 >= nd) break;
+      const int p0 = (j * kWave + lane) * 4;
+      uint32_t m = 0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) m |= (p0 + c < nv && v[4 * j + c] >= thr) ? 1u << c : 0u;
+      m <<= 4 * (lane & 7);
+      m |= dpp_u32<0xB1>(m);   // quad_perm [1,0,3,2]
+      m |= dpp_u32<0x4E>(m);   // quad_perm [2,3,0,1]
+      m |= dpp_u32<0x141>(m);  // row_half_mirror: the other quad of the eight
+      const int d = j * 8 + (lane >> 3);
+      if ((lane & 7) == 0 && d < nd) mrow[d] = m;
+    }
+  };
+  if constexpr (BITS) {
+    if (nvalid < k) {
+      bits(-__builtin_huge_valf());
+      return;
     }
   }
   // f(x, i) for every valid entry (i: its register index).
@@ -1938,6 +1969,7 @@ __global__ __launch_bounds__(256, V <= 16 ? (MEM ? 6 : 8) : (V <= 32 ? (MEM ? 5 
   }
   if (lane == 0) a.thr[row] = key_to_float(tk);
   if constexpr (MEM) members(key_to_float(tk));
+  if constexpr (BITS) bits(key_to_float(tk));
 }
 
 // ---------------------------------------------------------------------------
@@ -1996,6 +2028,11 @@ bool ragged(const SelectArgs& a) {
 template <int V>
 hipError_t launch_wave(const SelectArgs& a, hipStream_t stream) {
   const dim3 grid(static_cast<unsigned>((a.rows + 3) / 4));
+  if (a.mask != nullptr) {
+    if (ragged(a)) hipLaunchKernelGGL((topk_wave_kernel<V, true, false, true>), grid, dim3(256), 0, stream, a);
+    else hipLaunchKernelGGL((topk_wave_kernel<V, false, false, true>), grid, dim3(256), 0, stream, a);
+    return hipGetLastError();
+  }
   if (a.member != nullptr) hipLaunchKernelGGL((topk_wave_kernel<V, true, true>), grid, dim3(256), 0, stream, a);
   else if (ragged(a)) hipLaunchKernelGGL((topk_wave_kernel<V, true>), grid, dim3(256), 0, stream, a);
   else hipLaunchKernelGGL((topk_wave_kernel<V, false>), grid, dim3(256), 0, stream, a);
@@ -2131,6 +2168,14 @@ hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t l
     a.ldm = ldm;
     return T <= kBracketIdxMaxN ? launch_bracket<false, true>(a, stream)
                                 : launch_bracket<false, false>(a, stream);
+  }
+  if (T <= 2048) {  // rows a wave holds in registers
+    SelectArgs a{scores, rows, T, ld, k, T, thr, nullptr, B};
+    a.mask = mask;
+    a.ldm = ldm;
+    if (T <= 512) return launch_wave<8>(a, stream);
+    if (T <= 1024) return launch_wave<16>(a, stream);
+    return launch_wave<32>(a, stream);
   }
   const hipError_t e = launch_topk(scores, rows, T, ld, k, T, thr, nullptr, stream);
   if (e != hipSuccess) return e;

@@ -519,3 +519,36 @@ def test_topk_member_bytes(dev, n, k):
     _, idx = topk_indices(x, k)
     want = torch.zeros(9, n, dtype=torch.bool, device=dev).scatter_(-1, idx.long(), True)
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("T,k", [(1, 1), (2, 2), (63, 5), (64, 64), (65, 2), (128, 7), (129, 100), (255, 9),
+                                 (512, 32), (513, 40), (1023, 100), (1024, 1), (1025, 300), (2047, 128),
+                                 (2048, 64), (2048, 2048)])
+def test_wave_select_bitmask(dev, T, k):
+    """Rows a wave holds in registers: the bitmask it writes is the one made
+    from its thresholds in a second pass, words past 128-key granularity left
+    alone, with fewer than k keys, ties, zeros of both signs, NaN and
+    infinities, NaN above the diagonal, and a mask row stride above the words."""
+    import _dsa_lib as L
+    from dsa_attention import selection_mask
+
+    B, W = 3, (T + 63) // 64
+    g = torch.Generator().manual_seed(T)
+    s = torch.randn(B, T, T, generator=g)
+    s[1] = torch.randint(-1, 2, (T, T), generator=g).float() * torch.where(torch.rand(T, T, generator=g) < 0.5, 1.0, -0.0)
+    s[2, :, ::3] = float("-inf")
+    s[2, :, 1::7] = float("inf")
+    s[2, T // 2:, 2::5] = float("nan")
+    s.masked_fill_(~torch.ones(T, T, dtype=torch.bool).tril(), float("nan"))
+    s = s.to(dev)
+    thr = torch.empty(B, T, 1, device=dev)
+    mask = torch.full((B, T, W + 1), 0x5A5A, device=dev, dtype=torch.int64)
+    rc = L.lib().dsa_topk_threshold_mask(s.data_ptr(), B, T, T, k, thr.data_ptr(), mask.data_ptr(),
+                                         W + 1, L.stream_ptr(torch.device(dev)))
+    assert rc == 0
+    want = topk_threshold(s, k, causal=True)
+    assert torch.equal(thr.nan_to_num(7.0), want.nan_to_num(7.0))
+    written = (torch.arange(W, device=dev)[None, :] <= (torch.arange(T, device=dev)[:, None] | 127) // 64)
+    ref = selection_mask(s, want)
+    assert torch.equal(mask[..., :W][:, written], ref[:, written])
+    assert bool((mask[..., :W][:, ~written] == 0x5A5A).all()) and bool((mask[..., W] == 0x5A5A).all())
