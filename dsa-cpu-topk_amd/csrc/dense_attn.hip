@@ -26,7 +26,7 @@
 // added to exp2's argument, 7 costs it three bits for the largest keys).
 //
 // One pass over the scores first (prepare_kernel) writes the selection as one
-// bit per pair.  Last, redo_kernel gathers (attn_tile.h, on the bitmask) the
+// bit per pair, unless the select has done so.  Last, redo_kernel gathers (attn_tile.h, on the bitmask) the
 // 128-query tiles the pieces could not carry: those with a non-finite result
 // that selected something, and those of a head whose K or V hold a non-finite
 // value or a range beyond the scales.  Rows that select nothing get 0/0 = NaN,

@@ -17,7 +17,8 @@ hipError_t launch_topk_member(const float* scores, int64_t rows, int64_t n, int6
                               float* thr, uint8_t* member, hipStream_t stream);
 // Causal thresholds of a [B,T,T] score matrix plus the rows' selection
 // bitmask (what launch_selection_mask writes), in one pass over the scores
-// where the bracket kernel serves the rows; otherwise the two launches.
+// where the row is held in registers (T <= 4096) or the bracket kernel serves
+// it; otherwise the two launches.
 hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t ld, int k,
                             float* thr, uint64_t* mask, int64_t ldm, hipStream_t stream);
 

@@ -88,7 +88,7 @@ hipError_t launch_split(const void* qi, const void* ki, const void* wi, int idx_
     return launch_tile_attn_mask(mask, W, Q, K, V, dtype, B, T, HQ, DQ, scale, out, stream);
   }
   const AttnPick pick = pick_sparse_attn(dtype, B, T, HQ, DQ, DV, k);
-  if (pick == AttnPick::kDense && T <= 2048) {
+  if (pick == AttnPick::kDense && T <= 4096) {
     // the select holds the row in registers and writes the bitmask from there
     // (the dense kernel's workspace begins with it)
     e = launch_topk_mask(scores, B, T, T, k, thr, static_cast<uint64_t*>(att), (T + 63) / 64, stream);

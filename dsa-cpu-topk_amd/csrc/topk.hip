@@ -532,6 +532,22 @@ __device__ __forceinline__ void load_keys4(const float* __restrict__ src, int64_
   }
 }
 
+// The four flags of each of eight neighbouring lanes as 32 bits, in all of
+// them (DPP, no LDS): 32 keys of a selection bitmask.
+__device__ __forceinline__ uint32_t pack_flags(uint32_t m, int lane) {
+  m <<= 4 * (lane & 7);
+  m |= dpp_u32<0xB1>(m);   // quad_perm [1,0,3,2]
+  m |= dpp_u32<0x4E>(m);   // quad_perm [2,3,0,1]
+  m |= dpp_u32<0x141>(m);  // row_half_mirror: the other quad of the eight
+  return m;
+}
+
+// Dwords of a causal row's bitmask that are written: its 64-key words up to the
+// one of position t | 127, t = nv - 1.
+__device__ __forceinline__ int mask_dwords(int64_t T, int nv) {
+  return 2 * min(static_cast<int>((T + 63) >> 6), (((nv - 1) | 127) >> 6) + 1);
+}
+
 // ---------------------------------------------------------------------------
 // Register-resident kernel: rows up to 4*NT*(V/4) entries; first digit P1 bits.
 // ---------------------------------------------------------------------------
@@ -539,7 +555,12 @@ __device__ __forceinline__ void load_keys4(const float* __restrict__ src, int64_
 // 512 threads ask for 8 waves per SIMD there, so that four rows share a CU.
 // MEM (no indices): the row's member bytes too, for rows that may hold -inf in
 // number (masked score rows).
-template <int NT, int V, int P1, bool RAGGED, bool MEM = false>
+// BITS (causal rows, no indices): the row's selection bitmask too, from the
+// registers; the other waves then wait for the threshold instead of leaving,
+// which costs less than a second read of the scores (split forward B = 4, T =
+// 4096, HI = 8, DI = 64, HQ = 8, D = 64, k = 256 fp32: 396 -> 384 us; B = 2, T =
+// 3001, HI = 16, DI = 128, HQ = 16, D = 128, k = 300 f16: 184 -> 176).
+template <int NT, int V, int P1, bool RAGGED, bool MEM = false, bool BITS = false>
 __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void topk_reg_kernel(SelectArgs a) {
   static_assert(V % 4 == 0 && NT % kWave == 0 && NT <= 1024, "block shape");
   static_assert(P1 == 11 || P1 == 12, "first digit width");
@@ -562,7 +583,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void to
   int64_t row, nvalid;
   row_of_block(a, row, nvalid);
   const int k = a.k;
-  if (nvalid < k) {
+  if (!BITS && nvalid < k) {
     emit_short_row<NT>(a, row);
     return;
   }
@@ -606,6 +627,29 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void to
     }
 #pragma unroll
     for (int j = 0; j < V; ++j) key[j] = __float_as_uint(raw[j]);
+  }
+  // The row's mask words up to the one of position t | 127, from floats f(i).
+  [[maybe_unused]] auto bits = [&](float thr, auto&& f) __attribute__((always_inline)) {
+    uint32_t* __restrict__ mrow = reinterpret_cast<uint32_t*>(a.mask + row * a.ldm);
+    const int nd = mask_dwords(a.causal_T, nv);
+#pragma unroll
+    for (int j = 0; j < NCH; ++j) {
+      if (j * (NT / 8) >= nd) break;
+      const int p0 = (j * NT + tid) * 4;
+      uint32_t m = 0;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) m |= (p0 + c < nv && f(4 * j + c) >= thr) ? 1u << c : 0u;
+      m = pack_flags(m, lane);
+      const int d = p0 >> 5;
+      if ((lane & 7) == 0 && d < nd) mrow[d] = m;
+    }
+  };
+  if constexpr (BITS) {
+    if (nvalid < k) {
+      if (tid == 0) a.thr[row] = -__builtin_huge_valf();
+      bits(-__builtin_huge_valf(), [&](int i) { return __uint_as_float(key[i]); });
+      return;
+    }
   }
   // f(x, i) for every valid entry: x its value, i its register (chunks past
   // nch hold clamped duplicates; only the chunk the row ends inside tests
@@ -765,7 +809,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void to
     block_sync_lds();
     // Threshold only: the other waves exit now, so their registers take the
     // next rows' loads.
-    if (!MEM && a.idx == nullptr && tid >= kWave) return;
+    if (!MEM && !BITS && a.idx == nullptr && tid >= kWave) return;
     if (tid < kWave) {
       uint32_t tk, ngt;
       if (bcnt <= static_cast<uint32_t>(kWave)) {
@@ -786,7 +830,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void to
         for (uint32_t i = lane; i < bcnt; i += kWave) g += (cand[i] > tk) ? 1u : 0u;
         ngt = wave_read_lane(wave_inclusive_sum(g), kWave - 1);
       }
-      if (!MEM && a.idx == nullptr) {
+      if (!MEM && !BITS && a.idx == nullptr) {
         if (tid == 0) a.thr[row] = key_to_float(tk);
         return;
       }
@@ -843,7 +887,7 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void to
         });
         block_sync_lds();
         const uint32_t n_c = cnt;
-        if (!MEM && a.idx == nullptr) {
+        if (!MEM && !BITS && a.idx == nullptr) {
           if (tid >= kWave) return;
           const uint32_t tk = wave_select_cand(cand, n_c, prefix, S1, krem, hist);
           if (tid == 0) a.thr[row] = key_to_float(tk);
@@ -867,7 +911,11 @@ __global__ __launch_bounds__(NT, (V <= 32 && NT <= 512 && !MEM) ? 8 : 4) void to
   }
   if (tid == 0) a.thr[row] = key_to_float(thr_key);
 
-  if constexpr (MEM) {
+  if constexpr (BITS) {
+    const float th = key_to_float(thr_key);
+    if (keys_in_regs) bits(th, [&](int i) { return key_to_float(key[i]); });
+    else bits(th, [&](int i) { return __uint_as_float(key[i]); });
+  } else if constexpr (MEM) {
     if (!keys_in_regs) to_keys();
     emit_members<NT, NCH>(a.member + row * a.n, nv, key, thr_key, krem, wsum);
   } else if (a.idx != nullptr) {
@@ -1679,12 +1727,11 @@ __global__ __launch_bounds__(256, V <= 16 ? (MEM ? 6 : 8) : (V <= 32 ? (MEM ? 5 
         }
     }
   }
-  // The row's mask words, 64 keys each, up to the one of position t | 127: a
-  // chunk's eight lanes gather their four flags each into 32 bits (DPP), which
-  // the first of them stores.
+  // The row's mask words up to the one of position t | 127, 32 bits by the first
+  // of each eight lanes.
   [[maybe_unused]] auto bits = [&](float thr) __attribute__((always_inline)) {
     uint32_t* __restrict__ mrow = reinterpret_cast<uint32_t*>(a.mask + row * a.ldm);
-    const int nd = min(static_cast<int>((a.causal_T + 63) >> 6), (((nv - 1) | 127) >> 6) + 1) * 2;  // dwords
+    const int nd = mask_dwords(a.causal_T, nv);
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
       if (j * 8 >= nd) break;
@@ -1692,10 +1739,7 @@ __global__ __launch_bounds__(256, V <= 16 ? (MEM ? 6 : 8) : (V <= 32 ? (MEM ? 5 
       uint32_t m = 0;
 #pragma unroll
       for (int c = 0; c < 4; ++c) m |= (p0 + c < nv && v[4 * j + c] >= thr) ? 1u << c : 0u;
-      m <<= 4 * (lane & 7);
-      m |= dpp_u32<0xB1>(m);   // quad_perm [1,0,3,2]
-      m |= dpp_u32<0x4E>(m);   // quad_perm [2,3,0,1]
-      m |= dpp_u32<0x141>(m);  // row_half_mirror: the other quad of the eight
+      m = pack_flags(m, lane);
       const int d = j * 8 + (lane >> 3);
       if ((lane & 7) == 0 && d < nd) mrow[d] = m;
     }
@@ -2048,6 +2092,13 @@ hipError_t launch_reg(const SelectArgs& a, hipStream_t stream) {
   const bool two_d = a.causal_T > 1 && a.causal_T <= 65535 && nb <= 0x7fffffff;
   const dim3 grid = two_d ? dim3(static_cast<unsigned>(nb), static_cast<unsigned>(a.causal_T))
                           : dim3(static_cast<unsigned>(a.rows));
+  if constexpr (NT == 256 && V == 16) {  // rows of 2049 to 4096
+    if (a.mask != nullptr) {
+      if (ragged(a)) hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, true, false, true>), grid, dim3(NT), 0, stream, a);
+      else hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, false, false, true>), grid, dim3(NT), 0, stream, a);
+      return hipGetLastError();
+    }
+  }
   if constexpr (V <= 16) {
     if (a.member != nullptr) {
       hipLaunchKernelGGL((topk_reg_kernel<NT, V, P1, true, true>), grid, dim3(NT), 0, stream, a);
@@ -2169,13 +2220,14 @@ hipError_t launch_topk_mask(const float* scores, int64_t B, int64_t T, int64_t l
     return T <= kBracketIdxMaxN ? launch_bracket<false, true>(a, stream)
                                 : launch_bracket<false, false>(a, stream);
   }
-  if (T <= 2048) {  // rows a wave holds in registers
+  if (T <= 4096) {  // rows a wave or a block holds in registers
     SelectArgs a{scores, rows, T, ld, k, T, thr, nullptr, B};
     a.mask = mask;
     a.ldm = ldm;
     if (T <= 512) return launch_wave<8>(a, stream);
     if (T <= 1024) return launch_wave<16>(a, stream);
-    return launch_wave<32>(a, stream);
+    if (T <= 2048) return launch_wave<32>(a, stream);
+    return launch_reg<256, 16, 11>(a, stream);
   }
   const hipError_t e = launch_topk(scores, rows, T, ld, k, T, thr, nullptr, stream);
   if (e != hipSuccess) return e;

@@ -125,7 +125,8 @@ def test_dense_arguments(dev):
         sparse_attention_hip(s, t, x, x, x, kernel="dense")
 
 
-@pytest.mark.parametrize("B,T,k,HQ,D,dtype", [(8, 1024, 64, 8, 64, F32), (2, 2048, 256, 16, 128, HF)])
+@pytest.mark.parametrize("B,T,k,HQ,D,dtype", [(8, 1024, 64, 8, 64, F32), (2, 2048, 256, 16, 128, HF),
+                                                (2, 3001, 300, 16, 128, HF), (4, 4096, 256, 8, 64, F32)])
 def test_split_forward_takes_it(dev, B, T, k, HQ, D, dtype):
     """The split forward at shapes the rule gives to the dense kernel equals
     its stages run apart."""

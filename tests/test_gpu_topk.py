@@ -523,9 +523,9 @@ def test_topk_member_bytes(dev, n, k):
 
 @pytest.mark.parametrize("T,k", [(1, 1), (2, 2), (63, 5), (64, 64), (65, 2), (128, 7), (129, 100), (255, 9),
                                  (512, 32), (513, 40), (1023, 100), (1024, 1), (1025, 300), (2047, 128),
-                                 (2048, 64), (2048, 2048)])
-def test_wave_select_bitmask(dev, T, k):
-    """Rows a wave holds in registers: the bitmask it writes is the one made
+                                 (2048, 64), (2048, 2048), (2049, 300), (3001, 64), (4095, 4000), (4096, 256)])
+def test_register_select_bitmask(dev, T, k):
+    """Rows a wave or a block holds in registers: the bitmask it writes is the one made
     from its thresholds in a second pass, words past 128-key granularity left
     alone, with fewer than k keys, ties, zeros of both signs, NaN and
     infinities, NaN above the diagonal, and a mask row stride above the words."""
