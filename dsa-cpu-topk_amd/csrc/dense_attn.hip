@@ -18,19 +18,32 @@
 //   f16 inputs  S as is; P in two f16 pieces:   O = V.Pl + V.Ph
 //   bf16 inputs S as is; P in three bf16 pieces (24 bits, exact):
 //               O = V.P3 + V.P2 + V.P1
-// Scales are powers of two, so exact: a Q row and a head's 64-key tile of K are
-// scaled to put their largest element in [2^14, 2^15), a tile of V in [2^7,
-// 2^15), in steps of 2^8, so that the tiles of a head nearly always share one
-// scale.  Where they do not, the probabilities carry the difference, times 2^7
-// to stay clear of f16's subnormals (a multiplication apart from the exponent:
-// added to exp2's argument, 7 costs it three bits for the largest keys).
+// Scales are powers of two, so exact: a Q row, a head's 64-key tile of K or V
+// and, where P takes f16 pieces, a query's probabilities in a tile are scaled
+// to put their largest in [2^14, 2^15).  (The scale of the probabilities is a
+// multiplication apart from the exponent: added to exp2's argument, 14 would
+// cost it four bits for the largest keys.)  A tile's products are summed apart
+// and added to O with the scales undone.
+//
+// Two f16 pieces hold 23 bits down to 2^-15 of what the scale is taken from and
+// an absolute error of 2^-39 of it below.  So a probability far below its tile's
+// largest loses bits, which matters where the large ones meet a V of next to
+// nothing (a key that takes up the attention without adding to it): the result
+// is off by at most 2^-32 of sum_tiles (largest p of the tile) (largest |V| of
+// the tile) over the normaliser (f16: of the largest |V| of all tiles, no less).
+// Rows whose largest output is less than 2^-13 of that are left to redo_kernel,
+// so the pieces cost no row more than 2^-19 of its largest output, and most of
+// them less than the rounding of fp32 sums (T = 1500, k = 256 fp32, one key with V
+// = 0 at a logit 10 above the rest: relative error against float64 4.1e-7, the
+// gathers' 7.1e-7; from 12 above on such rows are gathered.  N(0, 1) operands:
+// 1.9e-7 against 3.9e-7).
 //
 // One pass over the scores first (prepare_kernel) writes the selection as one
 // bit per pair, unless the select has done so.  Last, redo_kernel gathers (attn_tile.h, on the bitmask) the
 // 128-query tiles the pieces could not carry: those with a non-finite result
-// that selected something, and those of a head whose K or V hold a non-finite
-// value or a range beyond the scales.  Rows that select nothing get 0/0 = NaN,
-// as the reference.
+// that selected something or a row below that bound, and those whose keys' K or
+// V hold a non-finite value or one beyond the scales.  Rows that select nothing
+// get 0/0 = NaN, as the reference.
 //
 // What bounds the dense kernel at D = 64 fp32: per wave and 64-key tile 96
 // MFMAs (1536 cycles), ~290 VALU instructions (32 of them exp2 at a quarter of
@@ -68,14 +81,6 @@ struct DenseArgs {
 
 constexpr uint32_t kBadTile = 0xffffffffu;  // kmax / vmax of a tile the pieces cannot carry
 
-// V's scale exponents come in steps of 8: x * 2^sh puts a tile whose largest
-// magnitude has these bits in [2^7, 2^15).
-__device__ __forceinline__ bool split_scale_v(uint32_t maxbits, int& sh) {
-  const int e = static_cast<int>(maxbits >> 23);
-  sh = maxbits == 0u ? 0 : 138 - ((e + 4) & ~7);
-  return maxbits == 0u || (e >= 127 - 60 && e <= 127 + 60);
-}
-
 // ---------------------------------------------------------------------------
 // One launch prepares the dense kernel's operands, HBM-bound throughout.
 //
@@ -105,7 +110,7 @@ struct PrepareArgs {
   uint64_t* mask;
 };
 
-template <int D, bool V>
+template <int D>
 __device__ __forceinline__ void convert_tile(const float* __restrict__ X, int64_t b, int h, int tile,
                                              int T, int HQ, uint16_t* __restrict__ hi,
                                              uint16_t* __restrict__ lo, uint32_t* __restrict__ maxbits,
@@ -130,7 +135,7 @@ __device__ __forceinline__ void convert_tile(const float* __restrict__ X, int64_
   block_sync_lds();
   mx = max(max(wmax[0], wmax[1]), max(wmax[2], wmax[3]));
   int sh;
-  const bool ok = V ? split_scale_v(mx, sh) : split_scale(mx, sh);
+  const bool ok = split_scale(mx, sh);
   if (tid == 0) maxbits[bh * ((T + 63) / 64) + tile] = ok ? mx : kBadTile;
   const float sc = ok ? pow2f(sh) : 0.f;
 #pragma unroll
@@ -160,8 +165,8 @@ __global__ __launch_bounds__(256) void prepare_kernel(PrepareArgs a) {
       const uint32_t bt = blockIdx.x / static_cast<uint32_t>(a.HQ);
       const int tile = static_cast<int>(bt / static_cast<uint32_t>(a.B));
       const int64_t b = bt % static_cast<uint32_t>(a.B);
-      convert_tile<D, false>(a.K, b, h, tile, T, a.HQ, a.pieces, a.pieces + a.plane, a.kmax, wmax[0]);
-      convert_tile<D, true>(a.V, b, h, tile, T, a.HQ, a.pieces + 2 * a.plane, a.pieces + 3 * a.plane,
+      convert_tile<D>(a.K, b, h, tile, T, a.HQ, a.pieces, a.pieces + a.plane, a.kmax, wmax[0]);
+      convert_tile<D>(a.V, b, h, tile, T, a.HQ, a.pieces + 2 * a.plane, a.pieces + 3 * a.plane,
                       a.vmax, wmax[1]);
       return;
     }
@@ -209,6 +214,7 @@ struct Pieces {  // pieces of K/V/Q, and of P
   static constexpr bool kF32 = __is_same(Tag, F32);
   static constexpr int X = kF32 ? 2 : 1;
   static constexpr int P = __is_same(Tag, BF16) ? 3 : 2;
+  static constexpr bool kApart = P == 2;  // tiles summed apart, P scaled per tile
   using Half = std::conditional_t<__is_same(Tag, BF16), BF16, F16>;
 };
 
@@ -229,6 +235,7 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   using M = Mfma16x16x32<typename PC::Half>;
   using L = TileLds<D, KT>;
   constexpr bool F = PC::kF32;
+  constexpr bool AP = PC::kApart;
   constexpr int NX = PC::X, NP = PC::P;
   constexpr int NJ = KT / 16;   // 16-key tiles
   constexpr int NJJ = KT / 32;  // P fragments (32 keys each)
@@ -236,16 +243,16 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   constexpr int NDT = D / 16;   // 16-dim output tiles
   // 16-key tiles whose K fragments are read at once, and 16-dim output tiles
   // whose V fragments are (twice: the next ones are on their way): 64 and 32
-  // registers, at D = 128 32 and 32 (fp32: 16).
+  // registers, at D = 128 32 and 32 (sums apart: 16).
   constexpr int KF = D == 128 ? 8 : 16;
   constexpr int KJ = NJ * NKS * NX <= KF ? NJ : KF / (NKS * NX);
-  constexpr int VG = (F && D == 128 ? 4 : 8) / (NJJ * NX);
+  constexpr int VG = (AP && D == 128 ? 4 : 8) / (NJJ * NX);
   constexpr int GB = NX * L::BYTES;  // bytes of a group's K (or V) tile
   __shared__ __align__(16) uint8_t k0[KS * GB], k1[KS * GB], v0[KS * GB], v1[KS * GB];
   // bias of the four keys a nibble of a mask word covers (tile_attn.hip), at
   // LDS address 0
   __shared__ __align__(1024) float btab[64];
-  __shared__ uint32_t redo;
+  __shared__ uint32_t redo, vtop;  // vtop (f16): largest |V| bits the block has seen
 
   const int tid = threadIdx.x;
   const int kg = KS == 2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;  // key group
@@ -255,7 +262,7 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   const int T = a.T;
   const int HQ = a.HQ;
   if (tid < 64) btab[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_huge_valf();
-  if (tid == 0) redo = 0u;
+  if (tid == 0) redo = vtop = 0u;
   const DSA_LDS uint8_t* const btabl = (const DSA_LDS uint8_t*)btab;
 
   // Block -> (tile, batch, head): tiles longest first, then batch, head fastest.
@@ -272,8 +279,6 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   const int nkt = (s_hi + KT - 1) / KT;
   uint32_t* const flag = a.flags + (b * ntile + tile) * HQ + h;
 
-  int vsh = 0;         // scale exponent of the head's largest V tile
-  bool mixed = false;  // some V tile has another one
   const int n64 = (T + 63) / 64;
   const uint32_t* const kmx = F ? a.kmax + bh * n64 : nullptr;
   const int64_t rowE = static_cast<int64_t>(HQ) * D;  // elements per Q/K/V row
@@ -357,6 +362,8 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
 
   float m[2] = {-__builtin_huge_valf(), -__builtin_huge_valf()};
   float lpart[2] = {0.f, 0.f};  // this lane's part of the normaliser, fp32
+  // fp32: sum over the tiles of their largest p times their largest |V|
+  [[maybe_unused]] float esum[2] = {0.f, 0.f};
   f32x4 o[NDT][2];
 #pragma unroll
   for (int dt = 0; dt < NDT; ++dt)
@@ -512,9 +519,16 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
       (void)split_scale(xb[0], ksh);
       kx = pow2f(-ksh);
     }
+    [[maybe_unused]] float vx = 1.f;  // the V tile's inverse scale
+    if constexpr (F) {
+      int vsh;
+      (void)split_scale(xb[1], vsh);
+      vx = pow2f(-vsh);
+    }
     u32x4 pf[NP][2][NJJ];
     bool grow = false;
     float alpha[2];
+    [[maybe_unused]] float back[2];  // undoes the scales of P and V
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
       const float cs = F ? cq[qt] * kx : cq[qt];
@@ -544,16 +558,18 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
 #pragma unroll
       for (int j = 0; j < NJ; ++j) ls += (p[j][0] + p[j][1]) + (p[j][2] + p[j][3]);
       lpart[qt] = fmaf(lpart[qt], alpha[qt], ls);
-      if constexpr (F) {
-        if (mixed) {
-          int tsh;
-          (void)split_scale_v(xb[1], tsh);
-          const float pc = xb[1] == 0u ? 1.f : pow2f(7 + vsh - tsh);
+      if constexpr (AP) {
+        // pm: the largest p, by the operations that made it.  Tiles 2^-107 below
+        // the running max share a scale (their products leave fp32's range).
+        const float pm = __builtin_amdgcn_exp2f(fmaf(mx, cs, -m_use));
+        const uint32_t eb = max(__float_as_uint(pm) >> 23, 20u);
+        const float pc = __uint_as_float((268u - eb) << 23);
+        back[qt] = __uint_as_float((eb - 14u) << 23) * vx;
+        if constexpr (F) esum[qt] = fmaf(esum[qt], alpha[qt], pm * __uint_as_float(xb[1]));
 #pragma unroll
-          for (int j = 0; j < NJ; ++j)
+        for (int j = 0; j < NJ; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) p[j][r] *= pc;
-        }
+          for (int r = 0; r < 4; ++r) p[j][r] *= pc;
       }
 #pragma unroll
       for (int jj = 0; jj < NJJ; ++jj)
@@ -599,9 +615,9 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
         __builtin_amdgcn_sched_barrier(0);
       }
       const u32x4(&vg)[NX][VG][NJJ] = vf[(dg / VG) & 1];
-      if constexpr (F) {
-        // The tile's products are summed apart and added to O once: one
-        // rounding at O's magnitude per tile instead of one per MFMA.
+      if constexpr (AP) {
+        // Summed apart also means one rounding at O's magnitude per tile
+        // instead of one per MFMA.
         f32x4 t[VG][2];
 #pragma unroll
         for (int d = 0; d < VG; ++d)
@@ -616,13 +632,16 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
               for (int qt = 0; qt < 2; ++qt)
                 t[d][qt] = M::run(vg[pv][d][jj], pf[pp][qt][jj], t[d][qt]);
         };
-        sum(NX - 1, 0);
+        if constexpr (F) sum(NX - 1, 0);
         sum(0, NP - 1);
         sum(0, 0);
 #pragma unroll
         for (int d = 0; d < VG; ++d)
 #pragma unroll
-          for (int qt = 0; qt < 2; ++qt) o[dg + d][qt] += t[d][qt];
+          for (int qt = 0; qt < 2; ++qt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+              o[dg + d][qt][r] = fmaf(t[d][qt][r], back[qt], o[dg + d][qt][r]);
       } else {
 #pragma unroll
         for (int p = NP - 1; p >= 0; --p)
@@ -636,6 +655,25 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
       }
     }
     __builtin_amdgcn_s_setprio(0);
+  };
+
+  // f16: the largest and lowest V of this thread's share of the tiles seen, read
+  // behind a tile's products (before them it holds up the K fragments: 9 us of
+  // the 117 at B = 2, T = 3001, HQ = 16, D = 128 against 2.5).
+  typedef _Float16 h16x2 __attribute__((ext_vector_type(2)));
+  [[maybe_unused]] h16x2 vhi = {0, 0}, vlo = {0, 0};
+  [[maybe_unused]] auto see_v = [&](const DSA_LDS uint8_t* vl) __attribute__((always_inline)) {
+    constexpr int N = L::BYTES / 16 / kNT;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+      const u32x4 x = *reinterpret_cast<const DSA_LDS u32x4*>(vl + (i * kNT + (tid & (kNT - 1))) * 16);
+#pragma unroll
+      for (int e = 0; e < 4; e += 2) {
+        const h16x2 y = __builtin_bit_cast(h16x2, x[e]), z = __builtin_bit_cast(h16x2, x[e + 1]);
+        vhi = __builtin_elementwise_maximum(__builtin_elementwise_maximum(vhi, y), z);
+        vlo = __builtin_elementwise_minimum(__builtin_elementwise_minimum(vlo, y), z);
+      }
+    }
   };
 
   // Per tile: the next tile's copy and mask words go out first (in that
@@ -657,29 +695,19 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
       __builtin_amdgcn_sched_barrier(0);
     }
     if (act) compute(xc, mwc, kc, vc);
+    if constexpr (AP && !F) {
+      if (kt < nkt) see_v(vc);
+    }
     if (more) wait_dma_keep<NSL>();
     else wait_dma_keep<0>();
     block_sync_lds();
   };
-  // Left to redo_kernel: K / V values the pieces cannot carry.
+  // Left to redo_kernel: tiles with a key whose K or V the pieces cannot carry.
   if constexpr (F) {
-    uint32_t vm = 0u, vlow = 0xffffffffu, kbad = 0u;
-    for (int i = lane; i < n64; i += kWave) {
-      const uint32_t v = a.vmax[bh * n64 + i];
-      vm = max(vm, v);
-      if (v != 0u) vlow = min(vlow, v);
-      kbad |= kmx[i] == kBadTile ? 1u : 0u;
-    }
-    vm = wave_extreme_u32<true>(vm);
-    vlow = wave_extreme_u32<false>(vlow);
-    // V tiles two scale steps apart would cost the probabilities low bits
-    int lsh = 0;
-    const bool vok = vm != kBadTile && split_scale_v(vm, vsh);
-    if (vlow != 0xffffffffu) (void)split_scale_v(vlow, lsh);
-    else lsh = vsh;
-    const bool skip = ballot(kbad != 0u) != 0u || !vok || lsh - vsh > 8;
-    mixed = __builtin_amdgcn_readfirstlane(lsh != vsh);
-    if (__builtin_amdgcn_readfirstlane(skip)) {  // the same in every wave
+    uint32_t bad = 0u;
+    for (int i = lane; i < (s_hi + 63) / 64; i += kWave)
+      bad |= (kmx[i] == kBadTile || a.vmax[bh * n64 + i] == kBadTile) ? 1u : 0u;
+    if (__builtin_amdgcn_readfirstlane(ballot(bad != 0u) != 0u)) {  // the same in every wave
       wait_dma_keep<0>();  // the first tile's copy writes this block's LDS
       if (tid == 0) *flag = 1u;
       return;
@@ -700,9 +728,9 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
 
   // The second group hands its sums to the first through the tile buffers:
   // O tile dt of query tile qt in buffer qt + 2 (dt % 2), [slot][lane] floats,
-  // the running max behind the even tiles and the normaliser behind the odd.
+  // the running max behind the even tiles, the normaliser and esum behind the odd.
   if constexpr (KS == 2) {
-    constexpr int NS = NDT * 2 + 1;  // slots per wave and buffer
+    constexpr int NS = NDT * 2 + 2;  // slots per wave and buffer
     static_assert(NS * 4 * 256 <= KS * GB, "the partial sums fit the tile buffers");
     DSA_LDS float* const buf[4] = {(DSA_LDS float*)k0 + wave * NS * 64 + lane,
                                    (DSA_LDS float*)k1 + wave * NS * 64 + lane,
@@ -715,19 +743,21 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) buf[qt + 2 * (dt & 1)][((dt >> 1) * 4 + r) * 64] = o[dt][qt][r];
-        buf[qt][(NS - 1) * 64] = m[qt];
-        buf[qt + 2][(NS - 1) * 64] = lpart[qt];
+        buf[qt][(NS - 2) * 64] = m[qt];
+        buf[qt + 2][(NS - 2) * 64] = lpart[qt];
+        if constexpr (F) buf[qt + 2][(NS - 1) * 64] = esum[qt];
       }
     }
     block_sync_lds();
     if (kg == 0) {
 #pragma unroll
       for (int qt = 0; qt < 2; ++qt) {
-        const float m1 = buf[qt][(NS - 1) * 64], l1 = buf[qt + 2][(NS - 1) * 64];
+        const float m1 = buf[qt][(NS - 2) * 64], l1 = buf[qt + 2][(NS - 2) * 64];
         const float mn = fmaxf(m[qt], m1);
         const float mu = mn == -__builtin_huge_valf() ? 0.f : mn;
         const float a0 = exp2f(m[qt] - mu), a1 = exp2f(m1 - mu);
         lpart[qt] = fmaf(lpart[qt], a0, l1 * a1);
+        if constexpr (F) esum[qt] = fmaf(esum[qt], a0, buf[qt + 2][(NS - 1) * 64] * a1);
 #pragma unroll
         for (int dt = 0; dt < NDT; ++dt)
 #pragma unroll
@@ -738,7 +768,15 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   }
 
   // O = O^T / l, lane l: query tq[qt], dims 16dt + 4g .. +3.
-  const float vx = F ? pow2f(-vsh - (mixed ? 7 : 0)) : 1.f;
+  // f16: the largest |V| of all tiles, whose sums of p are at least their largest
+  [[maybe_unused]] float vcap = 0.f;
+  if constexpr (AP && !F) {
+    const uint32_t w = __builtin_bit_cast(uint32_t, __builtin_elementwise_maximum(vhi, -vlo));
+    const uint32_t v = wave_extreme_u32<true>(max(w & 0xffffu, w >> 16));
+    if (lane == 0) atomicMax(&vtop, v);
+    block_sync_lds();
+    vcap = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(vtop)));
+  }
   bool bad = false;
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
@@ -750,15 +788,19 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
 #pragma unroll
       for (int dt = 0; dt < NDT; ++dt) {
         float4 v;
-        v.x = o[dt][qt][0] * inv * vx;
-        v.y = o[dt][qt][1] * inv * vx;
-        v.z = o[dt][qt][2] * inv * vx;
-        v.w = o[dt][qt][3] * inv * vx;
+        v.x = o[dt][qt][0] * inv;
+        v.y = o[dt][qt][1] * inv;
+        v.z = o[dt][qt][2] * inv;
+        v.w = o[dt][qt][3] * inv;
         mxb = max(max(mxb, __float_as_uint(v.x) & 0x7fffffffu), __float_as_uint(v.y) & 0x7fffffffu);
         mxb = max(max(mxb, __float_as_uint(v.z) & 0x7fffffffu), __float_as_uint(v.w) & 0x7fffffffu);
         *reinterpret_cast<float4*>(orow + 16 * dt + 4 * g) = v;
       }
       bad |= mxb >= 0x7f800000u && l != 0.f;
+      if constexpr (AP) {
+        mxb = max_xor32_u32(max_xor16_u32(mxb));  // over the query's four lanes
+        bad |= __uint_as_float(mxb) < (F ? esum[qt] * inv : vcap) * 0x1p-13f;  // false for NaN
+      }
     }
   }
   if (ballot(bad) != 0 && lane == 0) redo = 1u;

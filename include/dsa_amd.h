@@ -351,8 +351,8 @@ int dsa_sparse_attn_uses_mask(int dtype, int64_t T, int HQ, int DQ, int DV);
  * tiles under a selection bitmask: 128 queries of one head share every K/V
  * tile, fp32 operands and the probabilities are split into 16-bit pieces
  * whose products are exact.  Tiles the pieces cannot carry (non-finite K, V or
- * results, values beyond 2^+-60) are gathered per query instead, decided on the
- * device.
+ * results, values beyond 2^+-60, rows whose output is next to nothing beside the
+ * V they read) are gathered per query instead, decided on the device.
  *   dsa_sparse_attn_dense_workspace_bytes: the workspace it needs (device
  *     memory of the stream's device, 16-byte aligned, used by no other work
  *     until the launches complete, contents on entry free); 0 for shapes it

@@ -28,14 +28,20 @@ def case(T, HQ, D, k, dtype, B=1, seed=0):
 
 
 def bound(Q, K, V, T):
-    """Elementwise bound on the difference of two fp32 evaluations: a logit
-    is off by at most 16 * 2^-24 |q||k| scale (products to 2^-22, sums) and
-    exp2's argument by 2^-24 of its size (<= 64), a probability by that
+    """Elementwise bound on the difference of two fp32 evaluations: rel_bound
+    of the largest |V|, which bounds the pieces' share (2^-32 of it) too."""
+    return rel_bound(Q, K, T) * float(V.double().abs().max())
+
+
+def rel_bound(Q, K, T):
+    """Bound on what fp32 evaluation changes, relative to sum p |V| / sum p: a
+    logit is off by at most 16 * 2^-24 |q||k| scale (products to 2^-22, sums)
+    and exp2's argument by 2^-24 of its size (<= 64), a probability by that
     relative to itself, numerator and normaliser both; the sums over the
     keys add (T/32 + 8) * 2^-24."""
     D = Q.shape[-1]
     lg = float(Q.double().norm(dim=-1).max() * K.double().norm(dim=-1).max()) / math.sqrt(D)
-    return (2 * (16 * lg + 64) + T / 32 + 8) * 2.0 ** -24 * float(V.double().abs().max())
+    return (2 * (16 * lg + 64) + T / 32 + 8) * 2.0 ** -24
 
 
 @pytest.mark.parametrize("dtype", [F32, BF, HF])
@@ -95,11 +101,69 @@ def test_dense_nonfinite(dev, dtype, D):
     assert bool(torch.isfinite(a[1]).all())
 
 
+def _own_norm(out, s, thr, Q, K, V, T):
+    """Every element within rel_bound of its own sum p |V| / sum p, plus the
+    2^-19 of its row's largest output that the 16-bit pieces may cost."""
+    want = O.sparse_attn_threshold(s, thr, Q, K, V)
+    cap = O.sparse_attn_threshold(s, thr, Q, K, V.abs())
+    lim = rel_bound(Q, K, T) * cap + 2.0 ** -19 * want.abs().amax(dim=-1, keepdim=True)
+    worst = float(((out.double() - want).abs() / lim.clamp(min=1e-300)).max())
+    assert worst <= 1.0, worst
+
+
+@pytest.mark.parametrize("dtype,HQ,D", [(F32, 16, 64), (F32, 8, 128), (BF, 16, 64), (BF, 16, 128),
+                                        (HF, 16, 64), (HF, 16, 128)])
+@pytest.mark.parametrize("groups", [1, 2])
+@pytest.mark.parametrize("gap", [6.0, 10.0, 13.0, 16.0, 30.0])
+def test_dense_sink(dev, dtype, HQ, D, groups, gap):
+    """A key that every query selects at a logit far above the rest, with V = 0:
+    the output is what the small probabilities carry, and has their relative
+    accuracy, not the large one's; one and two key groups per block."""
+    T, k, sink = 300, 90, 70
+    B = 2 if groups == 2 else 2 * 256 // (HQ * ((T + 127) // 128)) + 1
+    say(f"dense sink B={B} HQ={HQ} D={D} {dtype} gap={gap}")
+    s, _, Q, K, V = case(T, HQ, D, k, F32, B=B, seed=int(gap))
+    Q[..., 0], K[..., 0] = 4.0, 0.0
+    K[:, sink] = 0.0
+    K[:, sink, :, 0] = gap * math.sqrt(D) / 4.0
+    V[:, sink] = 0.0
+    s[:, :, sink] = 9.0
+    masked = s.masked_fill(~torch.ones(T, T, dtype=torch.bool).tril(), -math.inf)
+    thr = O.topk_threshold(masked, k)
+    Q, K, V = (x.to(dtype) for x in (Q, K, V))
+    out = sparse_attention_hip(*(x.to(dev) for x in (s, thr, Q, K, V)), kernel="dense").cpu()
+    _own_norm(out, s, thr, Q, K, V, T)
+
+
+@pytest.mark.parametrize("dtype,HQ,D", [(F32, 16, 64), (F32, 8, 128), (BF, 16, 64), (HF, 16, 128)])
+@pytest.mark.parametrize("groups", [1, 2])
+def test_dense_large_logits(dev, dtype, HQ, D, groups):
+    """Logits of N(0, 64^2): the running max moves often, probabilities span
+    all of fp32, and two key groups merge across that."""
+    T, k = 300, 120
+    B = 2 if groups == 2 else 2 * 256 // (HQ * ((T + 127) // 128)) + 1
+    say(f"dense large logits B={B} HQ={HQ} D={D} {dtype}")
+    s, thr, Q, K, V = case(T, HQ, D, k, F32, B=B, seed=3)
+    Q, K, V = (Q * 8).to(dtype), (K * 8).to(dtype), V.to(dtype)
+    out = sparse_attention_hip(*(x.to(dev) for x in (s, thr, Q, K, V)), kernel="dense").cpu()
+    _own_norm(out, s, thr, Q, K, V, T)
+
+
+@pytest.mark.parametrize("dtype,D", [(F32, 64), (F32, 128), (HF, 64), (HF, 128)])
+def test_dense_does_ordinary_rows_itself(dev, dtype, D):
+    """N(0, 1) operands leave no tile to the gathers: every 128-query tile's
+    output differs from theirs in rounding."""
+    T, HQ, k = 1024, 4, 200
+    args = tuple(x.to(dev) for x in case(T, HQ, D, k, dtype, seed=4))
+    a, b = (sparse_attention_hip(*args, kernel=n).view(T // 128, -1) for n in ("dense", "gather"))
+    assert bool((a != b).any(dim=1).all())
+
+
 @pytest.mark.parametrize("span", [4, 9, 30, 70])
 def test_dense_fp32_ranges(dev, span):
-    """fp32 operands of very different magnitude: V tiles on one, on two
-    neighbouring and on far-apart scales (the last gathered), Q and K rows
-    scaled against each other, rows of zeros, and rows beyond the scales."""
+    """fp32 operands of very different magnitude: V tiles on neighbouring and on
+    far-apart scales (beyond 2^-60 gathered), Q and K rows scaled against each
+    other, rows of zeros, and rows beyond the scales."""
     T, HQ, D, k = 300, 2, 64, 25
     s, thr, Q, K, V = case(T, HQ, D, k, F32, seed=span)
     say(f"dense ranges span={span}")
