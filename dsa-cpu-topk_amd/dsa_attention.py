@@ -94,10 +94,9 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
     read once per head) and the tile kernel reads that (dsa_sparse_attn_mask):
     the same output, bit for bit.
     kernel="tiled" (or tiled=True) / "staged" / "mask" / "dense" / "gather" runs that
-    kernel at any T (AssertionError for shapes it does not cover); "staged"
-    is the dense one for the shapes of the staged kernel that the library gives
-    to the dense one (T >= 3072).  Where the dense kernel's workspace does not
-    fit, a call that did not ask for it by name takes one of the others."""
+    kernel at any T (AssertionError for shapes it does not cover).  Where the
+    dense kernel's workspace does not fit, a call that did not ask for it by
+    name takes one of the others."""
     L.require_gpu(scores, threshold, Q, K, V)
     B, T, _ = scores.shape
     HQ, DQ = Q.shape[-2], Q.shape[-1]
@@ -118,14 +117,11 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
     if kernel == "mask":
         return _sparse_attention_mask(scores, thr, Q, K, V, out)
     code = L.dtype_code(dt)
-    if kernel is None or (kernel == "staged" and T >= 3072):
-        # a forced staged kernel: top_k 0, the rule that takes staged shapes only
-        k = int(top_k) if kernel is None else 0
+    picked = kernel
+    if kernel is None:
         with L.on_device(Q.device):
-            picked = {0: kernel, 1: "dense", 2: "gather"}[
-                L.lib().dsa_sparse_attn_pick(code, B, T, HQ, DQ, DV, k)]
-    else:
-        picked = kernel
+            picked = {0: None, 1: "dense", 2: "gather"}[
+                L.lib().dsa_sparse_attn_pick(code, B, T, HQ, DQ, DV, int(top_k))]
     if picked == "dense":
         nws = L.lib().dsa_sparse_attn_dense_workspace_bytes(code, B, T, HQ, DQ, DV)
         try:

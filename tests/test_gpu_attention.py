@@ -432,9 +432,10 @@ def test_staged_and_gather_agree(dev):
 
 def test_staged_auto_at_config3_shape(dev):
     """B = 4, T = 4096 fp32, HQ = 8, D = 64 (config 3's attention): the
-    threshold entry point runs the staged kernel (256 tiles of 64 queries, at
-    least one per compute unit; long key ranges split over two blocks);
-    sampled rows against the oracle."""
+    threshold entry point runs the dense kernel (1024 blocks, four per compute
+    unit); the staged kernel asked for by name (256 tiles of 64 queries, long
+    key ranges split over two blocks) is another kernel, with and without a
+    workspace; sampled rows of each against the oracle."""
     from helpers import sample_rows
 
     B, T, HQ, D, k = 4, 4096, 8, 64, 256
@@ -443,14 +444,17 @@ def test_staged_auto_at_config3_shape(dev):
     thr = kth(k)(scores)
     out = sparse_attention_with_threshold_triton(scores.to(dev), thr.to(dev), Q.to(dev),
                                                  K.to(dev), V.to(dev))
-    forced = sparse_attention_hip(scores.to(dev), thr.to(dev), Q.to(dev), K.to(dev), V.to(dev),
-                                  kernel="staged")
+    args = tuple(x.to(dev) for x in (scores, thr, Q, K, V))
+    dense, staged = (sparse_attention_hip(*args, kernel=n) for n in ("dense", "staged"))
+    plain = _staged_plain(*args)
     torch.cuda.synchronize()
-    assert torch.equal(out, forced), "T = 4096 fp32 must take the staged kernel"
+    assert torch.equal(out, dense), "T = 4096 fp32 must take the dense kernel"
+    assert not torch.equal(staged, dense), "kernel='staged' must run the staged kernel"
     rows = sample_rows(T, 40, seed=3, include=(0, 1, 255, 256, 4095))
     want = O.sparse_attn_threshold(scores[:, rows], thr[:, rows], Q, K, V, rows=rows)
-    ok, err, _ = close(out[:, rows].cpu(), want, 1e-4, 1e-4)
-    assert ok, f"max abs err {err}"
+    for got in (out, staged, plain):
+        ok, err, _ = close(got[:, rows].cpu(), want, 1e-4, 1e-4)
+        assert ok, f"max abs err {err}"
 
 
 def _staged_plain(scores, thr, Q, K, V):
