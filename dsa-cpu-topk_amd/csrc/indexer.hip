@@ -446,22 +446,25 @@ __global__ __launch_bounds__((64 * qtile_waves<Tag, DI, NQ>())) void indexer_qti
 // two that puts its largest element in [2^14, 2^15) -- exact, with elements
 // down to 2^-15 of the row's largest keeping all 23 bits and smaller ones an
 // absolute error of 2^-39 of it, far below what the fp32 sum itself drops.
-// Positive scales leave the ReLU: q's inverse is folded into w, k's multiplies
-// each finished score.  A super-block whose q rows, w rows or k rows hold a
-// non-finite value, or a scale too far out for that folding (rows beyond
-// 2^+-60, w outside [2^-40, 2^30]), is summed in plain fp32 from memory
-// instead: the split would turn inf into inf - inf.  Before k's scale is undone
-// a sum is at most |w||q| 2^15 DI HI < 2^30 2^61 2^15 2^18, a finite float.
+// Positive scales leave the ReLU: q's inverse is folded into w, and each
+// query's weights are scaled by the power of two that puts the largest |w| 2^-(q's
+// exponent) in [2^59, 2^60), so that a sum is at most 2^60 2^30 DI HI, a finite
+// float, and weights of any size (a softmax gate of 1e-30 among others) keep
+// their bits.  The query's and k's exponents are undone together, by one ldexp
+// of the finished score.  A super-block whose q rows, w rows or k rows hold a
+// non-finite value, a row beyond 2^+-60 or weights of one query further apart
+// than 2^160 is summed in plain fp32 from memory instead: the split would turn
+// inf into inf - inf.
 // ---------------------------------------------------------------------------
 template <int DI>
 size_t split_lds_bytes(QTileShape sh) {
-  // both q pieces, w, and the inverse q scales
-  return static_cast<size_t>(sh.nq) * sh.nhg * (2 * (DI / 32) * 1024 + 64 + 64);
+  // both q pieces, w, the q scales, and each query's weight scale
+  return static_cast<size_t>(sh.nq) * (sh.nhg * (2 * (DI / 32) * 1024 + 64 + 64) + 16);
 }
 
 // LDS layout: qf[quad][hg][chunk][piece][lane] : uint4 (chunk = 8 of the lane
-// group's DI/4 dims), wf as in the kernel above, then the inverse q scales in
-// wf's layout.
+// group's DI/4 dims), wf as in the kernel above, then the q scale exponents in
+// wf's layout, then the queries' weight exponents.
 template <int DI, int KB, int NQ, int NW>
 __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a) {
   constexpr int E = DI / 4;      // dims per lane
@@ -491,8 +494,11 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
 
   uint4* qf = lds;
   float* wf = reinterpret_cast<float*>(lds + static_cast<size_t>(NQ) * nhg * NCH * 2 * 64);
-  float* qs = wf + static_cast<size_t>(NQ) * nhg * 16;
+  constexpr int kNoExp = -100000;  // of a q row or a weight of zero
+  int* qs = reinterpret_cast<int*>(wf + static_cast<size_t>(NQ) * nhg * 16);
+  int* wexp = qs + static_cast<size_t>(NQ) * nhg * 16;
   if (tid == 0) qbad = 0u;
+  if (tid < TQ) wexp[tid] = kNoExp;
   __syncthreads();
 
   // Stage q: one 8-dim chunk (32 bytes) per thread-iteration; the DI/8
@@ -531,24 +537,35 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
       qf[(2 * at) * 64 + ln] = hv;
       qf[(2 * at + 1) * 64 + ln] = lv;
       if (c8 == 0) {
-        qs[((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3)] = pow2f(-sh);
+        qs[((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3)] = mb == 0u ? kNoExp : -sh;
         if (!ok) qbad = 1u;
       }
     }
   }
   __syncthreads();
+  // Weights: their largest exponent per query, then each at that scale.
   {
     const int hp4 = 4 * nhg;
-    for (int u = tid; u < TQ * hp4; u += NT) {
-      const int tl = u / hp4;
-      const int h = u - tl * hp4;
-      const int t = t0 + tl;
-      const float wv = (t < T && h < HI) ? w[static_cast<int64_t>(t) * a.ldw + h] : 0.f;
-      const uint32_t wb = __float_as_uint(wv) & 0x7fffffffu;
-      if (wb != 0u && (wb < (127u - 40u) << 23 || wb > (127u + 30u) << 23)) qbad = 1u;
-      const int at = ((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3);
-      wf[at] = wv * qs[at];
-    }
+    auto weights = [&](auto&& f) __attribute__((always_inline)) {
+      for (int u = tid; u < TQ * hp4; u += NT) {
+        const int tl = u / hp4;
+        const int h = u - tl * hp4;
+        const int t = t0 + tl;
+        const float wv = (t < T && h < HI) ? w[static_cast<int64_t>(t) * a.ldw + h] : 0.f;
+        const int at = ((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3);
+        const bool none = wv == 0.f || qs[at] == kNoExp;
+        f(wv, tl, at, none ? kNoExp : __builtin_amdgcn_frexp_expf(wv) + qs[at]);
+      }
+    };
+    weights([&](float wv, int tl, int, int e) {
+      if (e != kNoExp) atomicMax(&wexp[tl], e);
+      if ((__float_as_uint(wv) & 0x7fffffffu) >= 0x7f800000u) qbad = 1u;
+    });
+    __syncthreads();
+    weights([&](float wv, int tl, int at, int e) {
+      wf[at] = e == kNoExp ? 0.f : __builtin_amdgcn_ldexpf(wv, qs[at] + 60 - wexp[tl]);
+      if (e != kNoExp && e < wexp[tl] - 160) qbad = 1u;
+    });
   }
   __syncthreads();
   const bool bad_q = qbad != 0u;
@@ -579,7 +596,7 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
     for (int kb = 0; kb < KB; ++kb)
       load_f32<E>(k + static_cast<int64_t>(min(s0 + 16 * kb + r16, T - 1)) * a.ldk + g * E, x[kb]);
     uint4 bh[KB][NCH], bl[KB][NCH];
-    float kinv[KB];
+    int kexp[KB];
     bool ok = true;
 #pragma unroll
     for (int kb = 0; kb < KB; ++kb) {
@@ -589,7 +606,7 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
       mb = max_xor32_u32(max_xor16_u32(mb));
       int sh;
       ok &= split_scale(mb, sh);
-      kinv[kb] = pow2f(-min(max(sh, -120), 120));
+      kexp[kb] = -sh;
       const float sc = pow2f(min(max(sh, -120), 120));
 #pragma unroll
       for (int c = 0; c < NCH; ++c) {
@@ -653,8 +670,9 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
           sc[kb] = fmaf(wv.w, relu_f32(acc[kb][3]), sc[kb]);
         }
       }
+      const int we = wexp[4 * qd + g] - 60;  // no weight at all: sc is 0
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) sc[kb] *= kinv[kb];
+      for (int kb = 0; kb < KB; ++kb) sc[kb] = __builtin_amdgcn_ldexpf(sc[kb], we + kexp[kb]);
       store(qd, s0, sc);
     }
   }

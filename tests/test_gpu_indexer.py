@@ -391,8 +391,8 @@ def test_fp32_pieces_nonfinite_rows(dev):
 
 def test_fp32_pieces_large_weights_times_large_rows(dev):
     """A finite score of large q rows and weights and small k rows stays
-    finite (k's scale is undone last; the product before it would pass fp32's
-    range, so such weights take the plain fp32 sum: DI + HI + 2 roundings)."""
+    finite (the weights' scale and k's are undone together; bound: the plain
+    fp32 sum's DI + HI + 2 roundings)."""
     T, HI, DI = 70, 8, 64
     q, k, w, *_ = O.make_inputs(1, T, HI, DI, 1, 1, 1, seed0=11)
     q, k, w = q * 2.0 ** 56, k * 2.0 ** -40, w * 2.0 ** 55
@@ -403,3 +403,25 @@ def test_fp32_pieces_large_weights_times_large_rows(dev):
     causal = torch.ones(T, T, dtype=torch.bool).tril()
     bound = (DI + HI + 2) * 2.0 ** -24 * l1
     assert bool(((out.double() - ref).abs() <= bound)[:, causal].all())
+
+
+@pytest.mark.parametrize("T,HI,DI", [(70, 8, 64), (130, 5, 32), (40, 64, 128), (33, 3, 256)])
+def test_fp32_pieces_weights_of_any_size(dev, T, HI, DI):
+    """Weights far below or above 1 stay on the pieces: a power of two times a
+    query's weights is that power times its scores, bit for bit, and a weight
+    too small to show leaves the scores as they are without it."""
+    q, k, w, *_ = O.make_inputs(2, T, HI, DI, 1, 1, 1, seed0=T)
+    q, k = q.to(dev), k.to(dev)
+    w[:, :, HI // 2] = 0.0
+    w[0, 5] = 0.0
+    base = indexer_scores_hip(q, k, w.to(dev)).cpu()
+    e = torch.randint(-110, 100, (2, T, 1), generator=torch.Generator().manual_seed(T)).float()
+    e[1, ::7] = -10.0
+    got = indexer_scores_hip(q, k, (w * torch.exp2(e)).to(dev)).cpu()
+    # (above 2^-126: smaller scores round to fp32's subnormals)
+    sure = (base.abs() * torch.exp2(e) > 2.0 ** -120) | (base == 0) | torch.isinf(base)
+    assert torch.equal(torch.where(sure, got, 0.0), torch.where(sure, base * torch.exp2(e), 0.0))
+    w[:, ::3, HI // 2] = 1e-30
+    got = indexer_scores_hip(q, k, w.to(dev)).cpu()
+    shows = base.abs() > 1e-15
+    assert torch.equal(got[shows], base[shows])
