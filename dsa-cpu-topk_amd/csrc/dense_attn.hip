@@ -40,9 +40,9 @@
 //
 // One pass over the scores first (prepare_kernel) writes the selection as one
 // bit per pair, unless the select has done so.  Last, redo_kernel gathers (attn_tile.h, on the bitmask) the
-// 128-query tiles the pieces could not carry: those with a non-finite result
-// that selected something or a row below that bound, and those whose keys' K or
-// V hold a non-finite value or one beyond the scales.  Rows that select nothing
+// rows the pieces could not carry: those with a non-finite result that selected
+// something or below that bound, and 128-query tiles whose keys' K or V hold a
+// non-finite value or one beyond the scales.  Rows that select nothing
 // get 0/0 = NaN, as the reference.
 //
 // What bounds the dense kernel at D = 64 fp32: per wave and 64-key tile 96
@@ -74,7 +74,7 @@ struct DenseArgs {
   float scale_log2;
   float* out;
   const uint64_t* mask;  // [B*T][W]
-  uint32_t* flags;       // [B][128-query tiles][HQ]: redo this tile's rows
+  uint32_t* flags;       // [B][128-query tiles][4][HQ]: 32 queries' bits, redo this row
   const uint32_t* kmax;  // fp32: largest |K| bits per [B][HQ][64-key tile]
   const uint32_t* vmax;
 };
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   // bias of the four keys a nibble of a mask word covers (tile_attn.hip), at
   // LDS address 0
   __shared__ __align__(1024) float btab[64];
-  __shared__ uint32_t redo, vtop;  // vtop (f16): largest |V| bits the block has seen
+  __shared__ uint32_t vtop;  // f16: largest |V| bits the block has seen
 
   const int tid = threadIdx.x;
   const int kg = KS == 2 ? __builtin_amdgcn_readfirstlane(tid >> 8) : 0;  // key group
@@ -262,7 +262,7 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   const int T = a.T;
   const int HQ = a.HQ;
   if (tid < 64) btab[tid] = (((tid >> 2) >> (tid & 3)) & 1) ? 0.f : -__builtin_huge_valf();
-  if (tid == 0) redo = vtop = 0u;
+  if (tid == 0) vtop = 0u;
   const DSA_LDS uint8_t* const btabl = (const DSA_LDS uint8_t*)btab;
 
   // Block -> (tile, batch, head): tiles longest first, then batch, head fastest.
@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
   const int tw = t0 + 32 * wave;  // first query of this wave
   const int s_hi = min(T, t0 + kTQ);
   const int nkt = (s_hi + KT - 1) / KT;
-  uint32_t* const flag = a.flags + (b * ntile + tile) * HQ + h;
+  uint32_t* const flag = a.flags + (b * ntile + tile) * 4 * HQ + h;  // a wave's: HQ apart
 
   const int n64 = (T + 63) / 64;
   const uint32_t* const kmx = F ? a.kmax + bh * n64 : nullptr;
@@ -709,7 +709,7 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
       bad |= (kmx[i] == kBadTile || a.vmax[bh * n64 + i] == kBadTile) ? 1u : 0u;
     if (__builtin_amdgcn_readfirstlane(ballot(bad != 0u) != 0u)) {  // the same in every wave
       wait_dma_keep<0>();  // the first tile's copy writes this block's LDS
-      if (tid == 0) *flag = 1u;
+      if (tid < 4) flag[tid * HQ] = 0xffffffffu;
       return;
     }
   }
@@ -777,9 +777,10 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
     block_sync_lds();
     vcap = static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(vtop)));
   }
-  bool bad = false;
+  uint32_t redo = 0u;  // the wave's 32 queries
 #pragma unroll
   for (int qt = 0; qt < 2; ++qt) {
+    bool bad = false;
     const float l = sum_xor32(sum_xor16(lpart[qt]));
     const float inv = 1.f / l;  // l == 0 only if nothing passed: NaN, as the reference
     if (kg == 0 && tq[qt] < T) {
@@ -802,16 +803,25 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
         bad |= __uint_as_float(mxb) < (F ? esum[qt] * inv : vcap) * 0x1p-13f;  // false for NaN
       }
     }
+    uint64_t any = ballot(bad);  // lanes c16, c16 + 16, .. hold query c16
+    any |= any >> 32;
+    any |= any >> 16;
+    redo |= static_cast<uint32_t>(any & 0xffffu) << (16 * qt);
   }
-  if (ballot(bad) != 0 && lane == 0) redo = 1u;
-  __syncthreads();
-  if (tid == 0) *flag = redo;
+  if (kg == 0 && lane == 0) flag[wave * HQ] = redo;
 }
 
 // ---------------------------------------------------------------------------
-// The gathers of attn_tile.h on the bitmask, for the tiles left to them: one
-// block of 8 waves per 128-query tile (and head chunk), so that the launch
-// costs little where, as nearly always, no tile is flagged.
+// The gathers of attn_tile.h on the bitmask, for the rows left to them: a wave
+// per query (and head chunk), as sparse_attn.hip has it, that leaves at once
+// where, as nearly always, none of the row's heads is flagged.  With every row
+// flagged it is the gathers' time on top of the dense kernel's (B = 4, T = 4096,
+// HQ = 8, D = 64, k = 256 fp32: 0.99 ms in all, the gathers 0.75; f16 B = 2, T =
+// 3001, HQ = 16, D = 128, k = 300: 0.99 and 0.86; eight waves per 128 queries and
+// whole tiles flagged took 2.07 and 4.88 ms, and 0.5 and 1.08 where one row was).
+// With none flagged the forwards at these sizes take 1 and 2 us more than with those
+// fewer blocks.  Blocks of eight waves: up to 1 us more; waves that stay for several rows: 2 more (their index
+// arithmetic), and no faster with every row flagged.
 // ---------------------------------------------------------------------------
 struct RedoArgs {
   const uint64_t* mask;
@@ -828,23 +838,34 @@ struct RedoArgs {
   int nchunk;  // HQ / HQc
 };
 
+constexpr int kRedoQ = 4;
+
 template <typename Tag, int E>
-__global__ __launch_bounds__(512) void redo_kernel(RedoArgs a) {
+__global__ __launch_bounds__(64 * kRedoQ) void redo_kernel(RedoArgs a) {
   using raw = typename Tag::raw;
   constexpr bool PAIR = __is_same(Tag, F32) && E == 2;
-  __shared__ __align__(16) int lists[8][kListCap];
-  const int wave = threadIdx.x >> 6;
+  __shared__ __align__(16) int lists[kRedoQ][kListCap];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lane = lane_id();
   const int T = a.T;
   const int ntile = (T + kTQ - 1) / kTQ;
-  const int chunk = static_cast<int>(blockIdx.x % static_cast<uint32_t>(a.nchunk));
-  int64_t b;
-  int tile;
-  causal_block_tile(blockIdx.x / static_cast<uint32_t>(a.nchunk), a.B, ntile, b, tile);
-  const uint32_t* fl = a.flags + (b * ntile + tile) * a.HQ;
-  uint32_t any = 0u;
-  for (int i = lane; i < a.HQ; i += kWave) any |= fl[i];
-  if (ballot(any != 0u) == 0u) return;
+  // blocks in chunk, batch, longest-rows-first order (32-bit: the grid is)
+  uint32_t i = blockIdx.x, chunk = 0u, bb = 0u;
+  if (a.nchunk > 1) {
+    chunk = i % static_cast<uint32_t>(a.nchunk);
+    i /= static_cast<uint32_t>(a.nchunk);
+  }
+  if (a.B > 1) {
+    bb = i % static_cast<uint32_t>(a.B);
+    i /= static_cast<uint32_t>(a.B);
+  }
+  const int64_t b = bb;
+  const int t = ((T + kRedoQ - 1) / kRedoQ - 1 - static_cast<int>(i)) * kRedoQ + wave;
+  if (t >= T) return;
+  const uint32_t* fl = a.flags + ((b * ntile + t / kTQ) * 4 + (t % kTQ) / 32) * a.HQ;
+  uint32_t rows = 0u;
+  for (int h = lane; h < a.HQ; h += kWave) rows |= fl[h];
+  if (ballot((rows >> (t % 32)) & 1u) == 0u) return;
   const int64_t E64 = static_cast<int64_t>(a.HQ) * a.D;
   const int64_t c0 = static_cast<int64_t>(chunk) * a.HQc * a.D;  // chunk's first element
   const raw* Q = static_cast<const raw*>(a.Q) + b * T * E64 + c0;
@@ -852,30 +873,28 @@ __global__ __launch_bounds__(512) void redo_kernel(RedoArgs a) {
   const raw* V = static_cast<const raw*>(a.V) + b * T * E64 + c0;
   const int W = (T + 63) / 64;
   int* list = lists[wave];
-  for (int t = tile * kTQ + wave; t < min(T, (tile + 1) * kTQ); t += 8) {
-    const int64_t qrow = b * T + t;
-    const uint8_t* mrow = reinterpret_cast<const uint8_t*>(a.mask + qrow * W);
-    // keys s0 .. s0 + 511 of the row: lane l's byte holds keys s0 + 8l .. + 7
-    // (bits of keys past t are 0 in the words that hold them)
-    auto segment = [&](int s0) {
-      const int sb = s0 + 8 * lane;
-      uint32_t bits = sb <= t ? mrow[sb >> 3] : 0u;
-      const int cnt = __popc(bits);
-      const int incl = wave_inclusive_sum(cnt);
-      int p = incl - cnt;
-      while (bits != 0u) {
-        list[p++] = sb + __ffs(static_cast<int>(bits)) - 1;
-        bits &= bits - 1u;
-      }
-      return wave_read_lane(incl, kWave - 1);
-    };
-    if constexpr (PAIR)
-      attend_query_pair_on(Q, K, V, t, a.D, a.scale_log2, segment, list, a.out + qrow * E64);
-    else
-      attend_query_on<Tag, E, E>(Q, K, V, t, a.HQc, a.D, a.D, a.scale_log2, segment, list,
-                                 a.out + qrow * E64 + c0, nullptr, static_cast<int>(E64),
-                                 static_cast<int>(E64));
-  }
+  const int64_t qrow = b * T + t;
+  const uint8_t* mrow = reinterpret_cast<const uint8_t*>(a.mask + qrow * W);
+  // keys s0 .. s0 + 511 of the row: lane l's byte holds keys s0 + 8l .. + 7
+  // (bits of keys past t are 0 in the words that hold them)
+  auto segment = [&](int s0) {
+    const int sb = s0 + 8 * lane;
+    uint32_t bits = sb <= t ? mrow[sb >> 3] : 0u;
+    const int cnt = __popc(bits);
+    const int incl = wave_inclusive_sum(cnt);
+    int p = incl - cnt;
+    while (bits != 0u) {
+      list[p++] = sb + __ffs(static_cast<int>(bits)) - 1;
+      bits &= bits - 1u;
+    }
+    return wave_read_lane(incl, kWave - 1);
+  };
+  if constexpr (PAIR)
+    attend_query_pair_on(Q, K, V, t, a.D, a.scale_log2, segment, list, a.out + qrow * E64);
+  else
+    attend_query_on<Tag, E, E>(Q, K, V, t, a.HQc, a.D, a.D, a.scale_log2, segment, list,
+                               a.out + qrow * E64 + c0, nullptr, static_cast<int>(E64),
+                               static_cast<int>(E64));
 }
 
 // Two key groups per block while every block has a CU to itself or shares it
@@ -904,9 +923,9 @@ hipError_t dispatch_dense(const DenseArgs& a, int D, hipStream_t stream) {
 
 template <typename Tag>
 hipError_t dispatch_redo(const RedoArgs& a, int E, hipStream_t stream) {
-  const dim3 grid(static_cast<unsigned>(a.B * ((a.T + kTQ - 1) / kTQ) * a.nchunk));
+  const dim3 grid(static_cast<unsigned>(a.B * ((a.T + kRedoQ - 1) / kRedoQ) * a.nchunk));
 #define DSA_REDO_CASE(e) \
-  case e: hipLaunchKernelGGL((redo_kernel<Tag, e>), grid, dim3(512), 0, stream, a); break;
+  case e: hipLaunchKernelGGL((redo_kernel<Tag, e>), grid, dim3(64 * kRedoQ), 0, stream, a); break;
   switch (E) {
     DSA_REDO_CASE(1)
     DSA_REDO_CASE(2)
@@ -915,7 +934,7 @@ hipError_t dispatch_redo(const RedoArgs& a, int E, hipStream_t stream) {
     DSA_REDO_CASE(16)
     case 32:
       if constexpr (!__is_same(Tag, F32)) {
-        hipLaunchKernelGGL((redo_kernel<Tag, 32>), grid, dim3(512), 0, stream, a);
+        hipLaunchKernelGGL((redo_kernel<Tag, 32>), grid, dim3(64 * kRedoQ), 0, stream, a);
         break;
       }
       return hipErrorInvalidValue;
@@ -942,7 +961,7 @@ Layout dense_layout(int dtype, int64_t B, int64_t T, int HQ, int D) {
   const int64_t n64 = (T + 63) / 64;
   Layout l{};
   l.flags = up(B * T * n64 * 8);  // behind the bitmask
-  l.kmax = l.flags + up(B * ((T + kTQ - 1) / kTQ) * HQ * 4);
+  l.kmax = l.flags + up(B * ((T + kTQ - 1) / kTQ) * 4 * HQ * 4);
   l.total = l.kmax;
   if (dtype == 0) {
     l.vmax = l.kmax + up(B * HQ * n64 * 4);

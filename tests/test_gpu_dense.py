@@ -159,6 +159,31 @@ def test_dense_does_ordinary_rows_itself(dev, dtype, D):
     assert bool((a != b).any(dim=1).all())
 
 
+@pytest.mark.parametrize("dtype,HQ,D", [(F32, 4, 64), (F32, 16, 128), (HF, 16, 64), (HF, 4, 128),
+                                        (BF, 4, 64), (BF, 16, 128)])
+@pytest.mark.parametrize("B", [1, 40])
+def test_dense_gathers_single_rows(dev, dtype, HQ, D, B):
+    """A row the pieces cannot carry is gathered by itself, all its heads: it
+    equals the gathers bit for bit, and its neighbours keep the dense sums."""
+    T, k = 300, 150
+    say(f"dense single rows B={B} HQ={HQ} D={D} {dtype}")
+    s, thr, Q, K, V = case(T, HQ, D, k, dtype, B=B, seed=9)
+    b, rows = B - 1, [64, 95, 96, 127, 128, 191, 255, 256, T - 1]
+    if dtype is F32:
+        Q[b, rows, HQ - 1] *= 2.0 ** 62  # beyond the scales
+    elif dtype is HF:  # only keys of V = 0 selected
+        V[b, 7] = 0.0
+        s[b, rows], thr[b, rows] = -9.0, 0.0
+        s[b, rows, 7] = 9.0
+    else:
+        Q[b, rows, HQ - 1] = math.nan
+    args = tuple(x.to(dev) for x in (s, thr, Q, K, V))
+    d, g = (sparse_attention_hip(*args, kernel=n)[b].cpu() for n in ("dense", "gather"))
+    assert torch.equal(torch.nan_to_num(d[rows], nan=7e7), torch.nan_to_num(g[rows], nan=7e7))
+    others = [t for t in range(64, T) if t not in rows]
+    assert bool((d != g)[others].flatten(1).any(dim=1).all())
+
+
 @pytest.mark.parametrize("span", [4, 9, 30, 70])
 def test_dense_fp32_ranges(dev, span):
     """fp32 operands of very different magnitude: V tiles on neighbouring and on
