@@ -349,10 +349,12 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32
 }
 // Scale exponent of a row whose largest magnitude has these bits (sign
 // cleared): x * 2^sh puts it in [2^14, 2^15); 0 for a row of zeros.
-__device__ __forceinline__ bool split_scale(uint32_t maxbits, int& sh) {
+// False if it is beyond 2^60 (non-finite ones among them) or below 2^low (-113:
+// the least whose scale is a float).
+__device__ __forceinline__ bool split_scale(uint32_t maxbits, int& sh, int low = -60) {
   const int e = static_cast<int>(maxbits >> 23);
   sh = maxbits == 0u ? 0 : 141 - e;
-  return maxbits == 0u || (e >= 127 - 60 && e <= 127 + 60);
+  return maxbits == 0u || (e >= 127 + low && e <= 127 + 60);
 }
 __device__ __forceinline__ float pow2f(int e) {  // 2^e, -126 <= e <= 127
   return __uint_as_float(static_cast<uint32_t>(e + 127) << 23);

@@ -451,11 +451,16 @@ __global__ __launch_bounds__((64 * qtile_waves<Tag, DI, NQ>())) void indexer_qti
 // exponent) in [2^59, 2^60), so that a sum is at most 2^60 2^30 DI HI, a finite
 // float, and weights of any size (a softmax gate of 1e-30 among others) keep
 // their bits.  The query's and k's exponents are undone together, by one ldexp
-// of the finished score.  A super-block whose q rows, w rows or k rows hold a
-// non-finite value, a row beyond 2^+-60 or weights of one query further apart
-// than 2^160 is summed in plain fp32 from memory instead: the split would turn
-// inf into inf - inf.
+// of the finished score.  The split would turn inf into inf - inf: the scores of
+// a q, w or k row with a non-finite value, of a row beyond 2^60 (whose dots may
+// pass fp32's range, as the pieces' do not) or below 2^-113, and of a query whose
+// weights are further apart than 2^160 are summed again in plain fp32 from memory.
+// That pass waits on loads (B = 4, T = 2047, HI = 8, DI = 64: one such query 0.20 ms,
+// one key 0.09, a query in every 16 0.52; with whole 16-query tiles sent there
+// 3.8, 0.8 and 11.2; the fp32 MFMA took 0.10 whatever the data).
 // ---------------------------------------------------------------------------
+constexpr int kSplitLow = -113;  // rows whose largest element is below 2^this take plain fp32
+
 template <int DI>
 size_t split_lds_bytes(QTileShape sh) {
   // both q pieces, w, the q scales, and each query's weight scale
@@ -473,7 +478,7 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
   constexpr int SB = 16 * KB;
   constexpr int NT = 64 * NW;
   extern __shared__ __align__(16) uint4 lds[];
-  __shared__ uint32_t qbad;
+  __shared__ uint32_t qbad;  // queries left to the plain fp32 pass, a bit each
   const int T = a.T;
   const int HI = a.HI;
   const int nhg = (HI + 3) >> 2;
@@ -523,7 +528,7 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
 #pragma unroll
       for (int o = 1; o < RL; o <<= 1) mb = max(mb, static_cast<uint32_t>(__shfl_xor(static_cast<int>(mb), o, kWave)));
       int sh;
-      const bool ok = split_scale(mb, sh);
+      const bool ok = split_scale(mb, sh, kSplitLow);
       const float sc = ok ? pow2f(sh) : 0.f;
       uint4 hv, lv;
       split_pair(x[0] * sc, x[1] * sc, hv.x, lv.x);
@@ -538,7 +543,7 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
       qf[(2 * at + 1) * 64 + ln] = lv;
       if (c8 == 0) {
         qs[((tl >> 2) * nhg + (h >> 2)) * 16 + (tl & 3) * 4 + (h & 3)] = mb == 0u ? kNoExp : -sh;
-        if (!ok) qbad = 1u;
+        if (!ok) atomicOr(&qbad, 1u << tl);
       }
     }
   }
@@ -559,16 +564,16 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
     };
     weights([&](float wv, int tl, int, int e) {
       if (e != kNoExp) atomicMax(&wexp[tl], e);
-      if ((__float_as_uint(wv) & 0x7fffffffu) >= 0x7f800000u) qbad = 1u;
+      if ((__float_as_uint(wv) & 0x7fffffffu) >= 0x7f800000u) atomicOr(&qbad, 1u << tl);
     });
     __syncthreads();
     weights([&](float wv, int tl, int at, int e) {
       wf[at] = e == kNoExp ? 0.f : __builtin_amdgcn_ldexpf(wv, qs[at] + 60 - wexp[tl]);
-      if (e != kNoExp && e < wexp[tl] - 160) qbad = 1u;
+      if (e != kNoExp && e < wexp[tl] - 160) atomicOr(&qbad, 1u << tl);
     });
   }
   __syncthreads();
-  const bool bad_q = qbad != 0u;
+  const uint32_t bad_q = qbad;
 
   const float ninf = -__builtin_huge_valf();
   const int t_end = (t0 + TQ < T) ? t0 + TQ : T;  // keys [0, t_end) can be causal
@@ -586,8 +591,8 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
     }
   };
 
-  bool any_bad = bad_q;  // some super-block of this wave is left to the plain fp32 pass below
-  for (int sb = wave; sb < nsb && !bad_q; sb += NW) {
+  bool any_bad = bad_q != 0u;  // some rows of this wave are left to the plain fp32 pass below
+  for (int sb = wave; sb < nsb; sb += NW) {
     const int s0 = sb * SB;
     // k rows of the super-block: loads first, then each block's scale and
     // pieces (rows past T are clamped to row T-1, never stored).
@@ -605,9 +610,9 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
       for (int e = 0; e < E; ++e) mb = max(mb, __float_as_uint(x[kb][e]) & 0x7fffffffu);
       mb = max_xor32_u32(max_xor16_u32(mb));
       int sh;
-      ok &= split_scale(mb, sh);
+      ok &= split_scale(mb, sh, kSplitLow);
       kexp[kb] = -sh;
-      const float sc = pow2f(min(max(sh, -120), 120));
+      const float sc = pow2f(min(max(sh, -126), 126));
 #pragma unroll
       for (int c = 0; c < NCH; ++c) {
         split_pair(x[kb][8 * c] * sc, x[kb][8 * c + 1] * sc, bh[kb][c].x, bl[kb][c].x);
@@ -616,10 +621,7 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
         split_pair(x[kb][8 * c + 6] * sc, x[kb][8 * c + 7] * sc, bh[kb][c].w, bl[kb][c].w);
       }
     }
-    if (ballot(!ok) != 0u) {
-      any_bad = true;
-      continue;
-    }
+    any_bad |= ballot(!ok) != 0u;  // (a bad row reaches its own scores only)
     const uint4* qa = qf + lane;
     const float4* wq = reinterpret_cast<const float4*>(wf) + g;
 #pragma unroll 1
@@ -677,42 +679,44 @@ __global__ __launch_bounds__(64 * NW, 4) void indexer_split_kernel(IndexerArgs a
     }
   }
 
-  // The super-blocks skipped above, in plain fp32 from memory, each lane its
-  // own (query, key) pairs.
+  // The scores of the rows the pieces cannot carry, in plain fp32 from memory
+  // over what was stored above, each lane its own (query, key) pairs.
   for (int sb = wave; sb < nsb && any_bad; sb += NW) {
     const int s0 = sb * SB;
-    if (!bad_q) {
-      bool ok = true;
-      for (int kb = 0; kb < KB; ++kb) {
-        const float* kr = k + static_cast<int64_t>(min(s0 + 16 * kb + r16, T - 1)) * a.ldk + g * E;
-        uint32_t mb = 0u;
-        for (int e = 0; e < E; ++e) mb = max(mb, __float_as_uint(kr[e]) & 0x7fffffffu);
-        mb = max_xor32_u32(max_xor16_u32(mb));
-        int sh;
-        ok &= split_scale(mb, sh);
-      }
-      if (ballot(!ok) == 0u) continue;
+    uint32_t bad_k = 0u;  // this lane's keys, a bit each
+    for (int kb = 0; kb < KB; ++kb) {
+      const float* kr = k + static_cast<int64_t>(min(s0 + 16 * kb + r16, T - 1)) * a.ldk + g * E;
+      uint32_t mb = 0u;
+      for (int e = 0; e < E; ++e) mb = max(mb, __float_as_uint(kr[e]) & 0x7fffffffu);
+      mb = max_xor32_u32(max_xor16_u32(mb));
+      int sh;
+      if (!split_scale(mb, sh, kSplitLow)) bad_k |= 1u << kb;
     }
 #pragma unroll 1
-    for (int qd = 0; qd < NQ; ++qd) {
-      const int tq = min(t0 + 4 * qd + g, T - 1);
-      float sc[KB];
-#pragma unroll
-      for (int kb = 0; kb < KB; ++kb) sc[kb] = 0.f;
+    for (int u = 0; u < NQ * KB; ++u) {
+      const int kb = u % KB, tl = 4 * (u / KB) + g;
+      const int tq = t0 + tl, s = s0 + 16 * kb + r16;
+      const bool mine = (((bad_q >> tl) | (bad_k >> kb)) & 1u) != 0u && tq < T && s <= tq;
+      if (ballot(mine) == 0u) continue;
+      if (mine) {
+        const float* kr = k + static_cast<int64_t>(s) * a.ldk;
+        float sc = 0.f;
 #pragma unroll 1
-      for (int h = 0; h < HI; ++h) {
-        const float* qr = q + static_cast<int64_t>(tq) * a.ldq + h * DI;
-        const float wv = w[static_cast<int64_t>(tq) * a.ldw + h];
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) {
-          const float* kr = k + static_cast<int64_t>(min(s0 + 16 * kb + r16, T - 1)) * a.ldk;
+        for (int h = 0; h < HI; ++h) {
+          const float* qr = q + static_cast<int64_t>(tq) * a.ldq + h * DI;
           float d = 0.f;
-#pragma unroll 1
-          for (int e = 0; e < DI; ++e) d = fmaf(qr[e], kr[e], d);
-          sc[kb] = fmaf(wv, relu_f32(d), sc[kb]);
+#pragma unroll 2
+          for (int e = 0; e < DI; e += 8) {
+            float x[8], y[8];
+            load_f32<8>(qr + e, x);
+            load_f32<8>(kr + e, y);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) d = fmaf(x[i], y[i], d);
+          }
+          sc = fmaf(w[static_cast<int64_t>(tq) * a.ldw + h], relu_f32(d), sc);
         }
+        out[static_cast<int64_t>(tq) * a.ld + s] = sc;
       }
-      store(qd, s0, sc);
     }
   }
 

@@ -425,3 +425,54 @@ def test_fp32_pieces_weights_of_any_size(dev, T, HI, DI):
     got = indexer_scores_hip(q, k, w.to(dev)).cpu()
     shows = base.abs() > 1e-15
     assert torch.equal(got[shows], base[shows])
+
+
+@pytest.mark.parametrize("T,HI,DI", [(70, 8, 64), (130, 5, 32), (40, 64, 128), (33, 3, 256)])
+def test_fp32_pieces_rows_of_any_small_size(dev, T, HI, DI):
+    """Rows far below 1 stay on the pieces: a power of two times a k row, a
+    query's q rows or its weights is that power times the scores, bit for bit."""
+    q, k, w, *_ = O.make_inputs(2, T, HI, DI, 1, 1, 1, seed0=T + 3)
+    base = indexer_scores_hip(q.to(dev), k.to(dev), w.to(dev)).cpu()
+    g = torch.Generator().manual_seed(T)
+    ek = torch.randint(-100, 1, (2, T, 1), generator=g).float()
+    eq = torch.randint(-100, 1, (2, T, 1), generator=g).float()
+    got = indexer_scores_hip((q * torch.exp2(eq).unsqueeze(-1)).to(dev), (k * torch.exp2(ek)).to(dev),
+                             (w * 2.0 ** 100).to(dev)).cpu()
+    e = (eq + 100).double() + ek.double().transpose(1, 2)
+    want = base.double() * torch.exp2(e)
+    # (above 2^-126: smaller scores round to fp32's subnormals)
+    sure = (want.abs() > 2.0 ** -120) | torch.isinf(base)
+    assert torch.equal(got.double()[sure], want[sure])
+
+
+@pytest.mark.parametrize("T,HI,DI", [(150, 8, 64), (130, 5, 32), (100, 80, 128), (70, 3, 256)])
+def test_fp32_pieces_bad_rows_alone(dev, T, HI, DI):
+    """Rows the pieces cannot carry (non-finite, beyond 2^60 or subnormal, and
+    weights of one query too far apart) leave every other score as it is, bit
+    for bit, and their own within the plain fp32 sum's bound."""
+    q, k, w, *_ = O.make_inputs(2, T, HI, DI, 1, 1, 1, seed0=T + 7)
+    clean = indexer_scores_hip(q.to(dev), k.to(dev), w.to(dev)).cpu()
+    bq, bk = [3, 16, 40, 63, T - 1], [0, 17, 64, T - 2]
+    q[1, 3, HI - 1, 7] = math.inf
+    q[1, 16, 0, 0] = math.nan
+    q[1, 40] *= 2.0 ** 62
+    w[1, 63, 0], w[1, 63, HI - 1] = 2.0 ** 90, 2.0 ** -90
+    w[1, T - 1, 0] = math.nan
+    k[1, 0, DI - 1] = math.nan
+    k[1, 17, 1] = -math.inf
+    k[1, 64] *= 2.0 ** 62
+    k[1, T - 2] *= 2.0 ** -130
+    out = indexer_scores_hip(q.to(dev), k.to(dev), w.to(dev)).cpu()
+    assert torch.equal(out[0], clean[0])
+    a, b = out[1].clone(), clean[1].clone()
+    for x in (a, b):
+        x[bq], x[:, bk] = 0.0, 0.0
+    assert torch.equal(a, b)
+    ref = O.indexer_scores(q, k, w)
+    causal = torch.ones(T, T, dtype=torch.bool).tril()
+    # (fp32 sums of such rows may pass fp32's range where float64 does not)
+    fin = torch.isfinite(ref) & torch.isfinite(out) & causal
+    l1 = torch.einsum("bth,bths->bts", w.double().abs(),
+                      torch.einsum("bthd,bsd->bths", q.double().abs(), k.double().abs()))
+    assert bool(((out.double() - ref).abs() <= (DI + HI + 4) * 2.0 ** -24 * l1 + 1e-37)[fin].all())
+    assert not bool((torch.isfinite(out) & torch.isnan(ref))[:, causal].any())
