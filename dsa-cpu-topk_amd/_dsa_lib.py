@@ -62,6 +62,7 @@ _SIGNATURES = {
                                _I),
     "dsa_sparse_attn_dense": ([_P, _I64, _P, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _F, _P, _P,
                                _I64, _P], _I),
+    "dsa_forward_split_min_T": ([_I], _I64),
     "dsa_forward_uses_split": ([_I, _I64, _I64, _I, _I, _I, _I, _I, _I], _I),
     "dsa_split_workspace_bytes": ([_I, _I64, _I64, _I, _I, _I, _I], _I64),
     "dsa_split_forward": ([_P, _P, _P, _I, _P, _P, _P, _I, _I64, _I64, _I, _I, _I, _I, _I, _I, _F,

@@ -415,6 +415,8 @@ int64_t dsa_split_workspace_bytes(int dtype, int64_t B, int64_t T, int HQ, int D
   return dsa::split_workspace(dtype, B, T, HQ, DQ, DV, top_k < T ? top_k : T);
 }
 
+int64_t dsa_forward_split_min_T(int DI) { return dsa::forward_split_min_T(DI); }
+
 int dsa_forward_uses_split(int dtype, int64_t B, int64_t T, int HI, int DI, int HQ, int DQ, int DV,
                            int top_k) {
   if (!dtype_ok(dtype) || B <= 0 || T <= 0 || HI < 1 || DI < 1 || HQ < 1 || DQ < 1 || DV < 1 || top_k < 1)

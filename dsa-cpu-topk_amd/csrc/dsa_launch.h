@@ -153,7 +153,9 @@ hipError_t launch_split(const void* qi, const void* ki, const void* wi, int idx_
                         int HQ, int DQ, int DV, int k, float scale, float* out, void* ws,
                         hipStream_t stream);
 
-// Whether launch_split is expected to be faster than launch_fused.
+// Whether launch_split is expected to be faster than launch_fused; never below
+// forward_split_min_T.
+int64_t forward_split_min_T(int DI);
 bool forward_uses_split(int dtype, int64_t B, int64_t T, int HI, int DI, int HQ, int DQ, int DV,
                         int64_t k);
 

@@ -58,11 +58,15 @@ int64_t split_workspace(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV,
 //     8, DI = 64 fp32 68 / 55, but T = 2048, B = 2, HI = 4, DI = 32 62 / 69;
 //   - everything else fused: T = 512, B = 16, HI = 4, DI = 32 fp32 25 / 35, T =
 //     697, B = 19, HI = 16, DI = 32 bf16 100 / 118.
+// Below forward_split_min_T never; a caller may ask that first.
+int64_t forward_split_min_T(int DI) { return DI >= 128 ? 200 : 512; }
+
 bool forward_uses_split(int dtype, int64_t B, int64_t T, int HI, int DI, int HQ, int DQ, int DV,
                         int64_t k) {
+  if (T < forward_split_min_T(DI)) return false;
   const double work = static_cast<double>(B) * T * T * HI * DI;
   if (T >= 512 && pick_sparse_attn(dtype, B, T, HQ, DQ, DV, k) == AttnPick::kDense) return true;
-  if (DI >= 128 && T >= 200 && work >= 6e8) return true;
+  if (DI >= 128 && work >= 6e8) return true;
   return T >= 900 && work >= (HI * DI >= 512 ? 1e9 : 2e9);
 }
 

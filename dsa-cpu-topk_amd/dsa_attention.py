@@ -20,6 +20,7 @@ functions, kept as API; no *_triton path calls them.
 """
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -276,11 +277,16 @@ def dsa_fused_hip(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> torch.Tensor:
     return out
 
 
+@functools.lru_cache(maxsize=64)
+def _split_min_T(DI: int) -> int:
+    return L.lib().dsa_forward_split_min_T(DI)
+
+
 def _split_is_faster(q_idx, k_idx, w_idx, Q, K, V, top_k: int) -> bool:
     """The library's rule, for inputs of one type on one GPU (the fused kernel
     takes mixed ones in fp32)."""
     B, T, HQ, DQ = Q.shape
-    if T < 200 or (T < 512 and q_idx.shape[3] < 128):
+    if T < _split_min_T(q_idx.shape[3]):
         return False  # never by that rule; such calls are launch-bound, so asking it counts
     dt = Q.dtype
     if not Q.is_cuda or dt not in (torch.float32, torch.bfloat16, torch.float16) or \

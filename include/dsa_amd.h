@@ -392,7 +392,9 @@ int dsa_sparse_attn_dense(const float* scores, int64_t ld, const float* thr, con
  * Replaces: dsa_attention_split_triton, reference dsa_attention.py:327-345.
  */
 /* 1 where dsa_split_forward is expected to be faster than dsa_fused_forward
- * (every T the latter refuses included).  Needs the device. */
+ * (every T the latter refuses included).  Needs the device, except below
+ * dsa_forward_split_min_T (host arithmetic on DI), where it is always 0. */
+int64_t dsa_forward_split_min_T(int DI);
 int dsa_forward_uses_split(int dtype, int64_t B, int64_t T, int HI, int DI, int HQ, int DQ, int DV,
                            int top_k);
 int64_t dsa_split_workspace_bytes(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int top_k);

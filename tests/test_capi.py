@@ -503,3 +503,18 @@ def test_forward_takes_fused_where_the_split_workspace_does_not_fit(monkeypatch,
     x = torch.empty(1, x.shape[1] + 1, 1, 64)
     with pytest.raises(error):
         DA.dsa_forward_hip(x, x, x, x, x, x, 4)
+
+
+@pytest.mark.parametrize("DI", [16, 32, 64, 127, 128, 256])
+def test_forward_never_splits_below_its_least_T(DI):
+    """dsa_forward_uses_split is 0 below dsa_forward_split_min_T, however much
+    work there is, and the Python rule stops at that same T."""
+    import dsa_attention as DA
+
+    T = L.lib().dsa_forward_split_min_T(DI)
+    assert T == DA._split_min_T(DI) > 1
+    f = L.lib().dsa_forward_uses_split
+    assert all(f(dt, 4096, t, 64, DI, 16, 128, 128, k) == 0
+               for dt in (L.DSA_F32, L.DSA_BF16) for t in (1, T // 2, T - 1) for k in (8, T))
+    if DI >= 128:  # from there on by the work alone, which needs no device
+        assert f(L.DSA_BF16, 4096, T, 64, DI, 16, 128, 128, 8) == 1
