@@ -95,3 +95,18 @@ def test_stream_default_form_matches_split(dev):
     assert len({o.data_ptr() for o in outs}) == len(outs), "each batch gets its own output"
     for bt, o in zip(batches, outs):
         assert torch.equal(o, dsa_split_hip(*bt, 32))
+
+
+def test_stream_pointer_without_the_private_query(dev, monkeypatch):
+    """The stream pointer the C entries get is the current stream's, with
+    torch's private query and without it."""
+    import _dsa_lib as L
+
+    side = torch.cuda.Stream(dev)
+    for s in (torch.cuda.current_stream(dev), side):
+        with torch.cuda.stream(s):
+            got = [L.stream_ptr(torch.device("cuda")), L.stream_ptr(torch.device("cuda", 0))]
+            with monkeypatch.context() as m:
+                m.setattr(L, "_raw_stream", None)
+                got += [L.stream_ptr(torch.device("cuda")), L.stream_ptr(torch.device("cuda", 0))]
+            assert got == [s.cuda_stream] * 4
