@@ -79,17 +79,11 @@ struct TileLds {
   static constexpr int BYTES = KT * D * 2;
   // K is read as 16-byte A fragments by 16 consecutive rows at one chunk:
   // row % NCH spreads them over NCH chunk positions.
-  // (At D = 32 four rows span the banks once, so the position moves every
-  // fourth row.)
-  static __device__ __forceinline__ int swz_k(int r) {
-    return D == 32 ? (r >> 2) & (NCH - 1) : r & (NCH - 1);
-  }
+  static __device__ __forceinline__ int swz_k(int r) { return r & (NCH - 1); }
   // V is read by the transposing 8-byte reads: 4 consecutive rows at one
   // chunk pair {2m, 2m+1} per 16-lane group; 2*(r % (NCH/2)) keeps the pair
   // together and moves it per row.
-  static __device__ __forceinline__ int swz_v(int r) {
-    return D == 32 ? (r >> 1) & 2 : (2 * r) & (NCH - 1);
-  }
+  static __device__ __forceinline__ int swz_v(int r) { return (2 * r) & (NCH - 1); }
 };
 
 // Buffer resource over one head's K or V rows from row s1 on (`head_base`
