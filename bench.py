@@ -200,13 +200,13 @@ C3 = dict(B=4, T=4096, k=256, HI=8, DI=64, HQ=8, DQ=64, DV=64)
 
 
 def bench_split_long(dev, cfg, dtype, name, reps, fp8_indexer=False):
-    """Split forward at a long-row config: indexer (causal half), causal
-    radix-select, attention (the tile kernel where it applies), each stage
-    timed with HIP events on the stream it runs on."""
+    """Split forward at a long-row config, as the one call a program makes
+    (dsa_split_hip), and its stages run apart: indexer (causal half), causal
+    radix-select, attention, each timed with HIP events on the stream it runs on."""
     import torch
 
     import _dsa_lib as L
-    from dsa_attention import sparse_attention_from_mask, sparse_attention_hip
+    from dsa_attention import dsa_split_hip, sparse_attention_from_mask, sparse_attention_hip
     from lightning_indexer import indexer_scores_hip
     from topk_threshold import topk_threshold_into, topk_threshold_mask
 
@@ -217,8 +217,9 @@ def bench_split_long(dev, cfg, dtype, name, reps, fp8_indexer=False):
     thr = torch.empty(B, T, 1, device=dev)
     out = torch.empty(B, T, cfg["HQ"], cfg["DV"], device=dev)
     ix = lambda: indexer_scores_hip(*ins[:3], write_upper=False, out=scores)  # noqa: E731
-    # The stages as dsa_split_hip runs them: where the attention runs on
-    # tiles from a bitmask, the select writes that bitmask in its own pass.
+    # Where the tile kernel takes the attention, its bitmask comes from the
+    # select; the dense kernel's, which the one call's select writes too up to T =
+    # 4096, has no entry of its own: run apart, the attention makes its bitmask.
     uses_mask = bool(L.lib().dsa_sparse_attn_uses_mask(L.dtype_code(dtype), T, cfg["HQ"],
                                                        cfg["DQ"], cfg["DV"]))
     if uses_mask:
@@ -227,13 +228,16 @@ def bench_split_long(dev, cfg, dtype, name, reps, fp8_indexer=False):
         att = lambda: sparse_attention_from_mask(mask, *ins[3:], out=out)  # noqa: E731
     else:
         sel = lambda: topk_threshold_into(scores, min(k, T), thr, causal=True)  # noqa: E731
-        att = lambda: sparse_attention_hip(scores, thr, *ins[3:], out=out)  # noqa: E731
+        att = lambda: sparse_attention_hip(scores, thr, *ins[3:], out=out, top_k=k)  # noqa: E731
 
-    def fwd():
+    def apart():
         ix()
         sel()
         att()
 
+    fwd = lambda: dsa_split_hip(*ins, k)  # noqa: E731
+    warm(apart)
+    t_apart = time_events(apart, reps, stream)
     warm(fwd)
     t_ix = time_events(ix, reps, stream)
     t_sel = time_events(sel, reps, stream)
@@ -249,7 +253,10 @@ def bench_split_long(dev, cfg, dtype, name, reps, fp8_indexer=False):
            "select_ms": round(t_sel * 1e3, 4),
            "select_GB_per_s": round((4.0 * B * T * (T + 1) / 2 + 4.0 * B * T) / t_sel / 1e9, 1),
            "attention_ms": round(t_att * 1e3, 4),
-           "select_writes_selection_bitmask": uses_mask}
+           "stages_apart_ms": round(t_apart * 1e3, 4),
+           "stages_note": "stage times are of the stages run apart: " +
+                          ("the select writes the tile kernel's selection bitmask" if uses_mask else
+                           "thresholds only from the select, the attention makes its own bitmask")}
     if fp8_indexer:
         # the same indexer on e4m3 q_idx/k_idx (w fp32): informational, the
         # split forward above runs the input dtype

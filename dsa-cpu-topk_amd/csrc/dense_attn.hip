@@ -39,19 +39,20 @@
 // 1.9e-7 against 3.9e-7).
 //
 // One pass over the scores first (prepare_kernel) writes the selection as one
-// bit per pair, unless the select has done so.  Last, redo_kernel gathers (attn_tile.h, on the bitmask) the
-// rows the pieces could not carry: those with a non-finite result that selected
-// something or below that bound, and 128-query tiles whose keys' K or V hold a
-// non-finite value or one beyond the scales.  Rows that select nothing
-// get 0/0 = NaN, as the reference.
+// bit per pair, unless the select has done so.  Last, redo_kernel gathers
+// (attn_tile.h, on the bitmask) the rows the pieces could not carry: those with a
+// non-finite result that selected something or below that bound, and the
+// 128-query tiles that read a K or V tile non-finite or beyond the scales.  Rows
+// that select nothing get 0/0 = NaN, as the reference.
 //
 // What bounds the dense kernel at D = 64 fp32: per wave and 64-key tile 96
-// MFMAs (1536 cycles), ~290 VALU instructions (32 of them exp2 at a quarter of
-// the rate, ~1500 cycles) and 42 KB of LDS reads; one SIMD's two waves overlap
-// the first two only in part (5400 cycles for two tiles).  B = 4, T = 4096,
-// HQ = 8, k = 256 fp32: 245 us in all (prepare 48, dense 185, redo 5) against
-// 0.45 ms staged, relative error against float64 2.1e-7 against 3.7e-7.
-// B = 2, T = 3001, HQ = 16, D = 128, k = 300 f16: 124 us against 862 gathered.
+// MFMAs (1536 cycles), ~440 VALU instructions (36 of them exp2 at a quarter of
+// the rate, ~2200 cycles) and 42 KB of LDS reads; one SIMD's two waves overlap
+// the first two only in part (about 5600 cycles for two tiles).  B = 4, T = 4096,
+// HQ = 8, k = 256 fp32: 253 us in all (prepare 48, 25 where the select has written
+// the bitmask; dense 192-200, redo 4.5) against 0.44 ms staged, relative error
+// against float64 2.1e-7 against 3.7e-7.
+// B = 2, T = 3001, HQ = 16, D = 128, k = 300 f16: 141 us against 862 gathered.
 #include <algorithm>
 #include <type_traits>
 
@@ -90,8 +91,9 @@ constexpr uint32_t kBadTile = 0xffffffffu;  // kmax / vmax of a tile the pieces 
 // record that magnitude.
 //
 // The others (none if the select has written the mask: scores null) write the
-// selection bitmask: one wave per row, rows longest first, each causal score read once (nontemporal, 16 loads
-// in flight per lane), as selection_mask_kernel (tile_attn.hip) does.
+// selection bitmask: one wave per row, rows longest first, each causal score
+// read once (nontemporal, 16 loads in flight per lane), as selection_mask_kernel
+// (tile_attn.hip) does.
 // ---------------------------------------------------------------------------
 struct PrepareArgs {
   const float* scores;
@@ -819,9 +821,9 @@ __global__ __launch_bounds__(kNT * KS, 2) void dense_attn_kernel(DenseArgs a) {
 // HQ = 8, D = 64, k = 256 fp32: 0.99 ms in all, the gathers 0.75; f16 B = 2, T =
 // 3001, HQ = 16, D = 128, k = 300: 0.99 and 0.86; eight waves per 128 queries and
 // whole tiles flagged took 2.07 and 4.88 ms, and 0.5 and 1.08 where one row was).
-// With none flagged the forwards at these sizes take 1 and 2 us more than with those
-// fewer blocks.  Blocks of eight waves: up to 1 us more; waves that stay for several rows: 2 more (their index
-// arithmetic), and no faster with every row flagged.
+// With none flagged the launch takes 4.5 us, 1 to 2 more than with those fewer
+// blocks.  Blocks of eight waves: up to 1 us more; waves that stay for several
+// rows: 2 more (their index arithmetic), and no faster with every row flagged.
 // ---------------------------------------------------------------------------
 struct RedoArgs {
   const uint64_t* mask;
@@ -899,10 +901,10 @@ __global__ __launch_bounds__(64 * kRedoQ) void redo_kernel(RedoArgs a) {
 
 // Two key groups per block while every block has a CU to itself or shares it
 // with one other (they end with their longest block: B = 4, T = 2048, HQ = 8,
-// D = 64 fp32, 512 blocks, 95 us against 106); past that two independent
+// D = 64 fp32, 512 blocks, 98 us against 108); past that two independent
 // blocks per CU overlap one's products with the other's softmax, which a
 // block's own groups, tied by its barriers, do not (B = 4, T = 4096, 1024
-// blocks, 245 us against 285; f16 D = 128, 768 blocks, 125 against 145).
+// blocks, 252 us against 294; f16 D = 128, 768 blocks, 142 against 159).
 template <typename Tag, int D>
 hipError_t launch_dense(const DenseArgs& a, hipStream_t stream) {
   const int64_t nblk = a.B * a.HQ * ((a.T + kTQ - 1) / kTQ);
@@ -1042,12 +1044,12 @@ hipError_t launch_dense_attn(const float* scores, int64_t ld, const float* thr, 
 //     longest block's chain where two key groups share a block (1.3 us per 64
 //     keys), the scores and K / V through prepare_kernel at 5.5 TB/s, and 15
 //     for the launches' fixed parts.
-// (B = 4, T = 2048, HQ = 8, D = 64 fp32: k = 128 92 us dense against 175
-// gathered, k = 64 92 / 103, k = 32 92 / 62; bf16 k = 128 67 / 97, k = 32 67 /
-// 35.)  Where top_k is unknown the dense kernel takes only the shapes the
+// (B = 4, T = 2048, HQ = 8, D = 64 fp32: k = 128 95 us dense against 168
+// gathered, k = 64 93 / 98, k = 32 93 / 59; bf16 k = 128 69 / 93, k = 32 66 /
+// 32.)  Where top_k is unknown the dense kernel takes only the shapes the
 // staged kernel would have had, which streams every key whatever is selected
-// (B = 4, T = 4096, HQ = 8, D = 64: 360-450 us at any k against 245), with
-// enough blocks that it wins at any k (B = 1, T = 4096: 122 us against 94 at
+// (B = 4, T = 4096, HQ = 8, D = 64: 360-450 us at any k against 253), with
+// enough blocks that it wins at any k (B = 1, T = 4096: 123 us against 94 at
 // k = 16).
 AttnPick pick_sparse_attn(int dtype, int64_t B, int64_t T, int HQ, int DQ, int DV, int64_t top_k) {
   if (!dense_attn_supported(dtype, T, HQ, DQ, DV) || sparse_attn_uses_tiles(dtype, T, HQ, DQ, DV))

@@ -94,7 +94,10 @@ hipError_t launch_split(const void* qi, const void* ki, const void* wi, int idx_
   const AttnPick pick = pick_sparse_attn(dtype, B, T, HQ, DQ, DV, k);
   if (pick == AttnPick::kDense && T <= 4096) {
     // the select holds the row in registers and writes the bitmask from there
-    // (the dense kernel's workspace begins with it)
+    // (the dense kernel's workspace begins with it).  Longer rows leave it to
+    // prepare_kernel, though the bracket select's bitmask costs less than that
+    // second read of the scores there too (B = 2, k = 256: T = 5000 8 us against
+    // 19, T = 8192 17 against 45).
     e = launch_topk_mask(scores, B, T, T, k, thr, static_cast<uint64_t*>(att), (T + 63) / 64, stream);
     if (e != hipSuccess) return e;
     return launch_dense_attn(nullptr, T, thr, Q, K, V, dtype, B, T, HQ, DQ, scale, out, att, stream);

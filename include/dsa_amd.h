@@ -350,9 +350,10 @@ int dsa_sparse_attn_uses_mask(int dtype, int64_t T, int HQ, int DQ, int DV);
  * probabilities and sums for every input type) computed densely on MFMA
  * tiles under a selection bitmask: 128 queries of one head share every K/V
  * tile, fp32 operands and the probabilities are split into 16-bit pieces
- * whose products are exact.  Tiles the pieces cannot carry (non-finite K, V or
- * results, values beyond 2^+-60, rows whose output is next to nothing beside the
- * V they read) are gathered per query instead, decided on the device.
+ * whose products are exact.  Rows the pieces cannot carry (a non-finite result,
+ * an output that is next to nothing beside the V it weighs; all rows of a
+ * 128-query tile that reads K or V non-finite or beyond 2^+-60) are gathered
+ * instead, decided on the device.
  *   dsa_sparse_attn_dense_workspace_bytes: the workspace it needs (device
  *     memory of the stream's device, 16-byte aligned, used by no other work
  *     until the launches complete, contents on entry free); 0 for shapes it
