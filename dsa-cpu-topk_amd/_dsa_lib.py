@@ -204,6 +204,14 @@ def ready_ptrs(dtype: torch.dtype, xs) -> list | None:
     return ptrs
 
 
+def check_out(out: torch.Tensor, n: int, device: torch.device) -> None:
+    """`out` can take n fp32 values from a kernel on `device`, which knows its
+    pointer alone (AssertionError)."""
+    assert out.dtype == torch.float32 and out.is_contiguous() and out.numel() >= n \
+        and out.device == device, \
+        f"out: {n} contiguous fp32 values on {device} (got {tuple(out.shape)} {out.dtype} on {out.device})"
+
+
 def require_gpu(*xs: torch.Tensor) -> None:
     for x in xs:
         if not x.is_cuda:

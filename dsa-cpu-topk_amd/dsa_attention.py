@@ -102,6 +102,7 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
     B, T, _ = scores.shape
     HQ, DQ = Q.shape[-2], Q.shape[-1]
     DV = V.shape[-1]
+    assert scores.shape == (B, T, T), f"scores shape {tuple(scores.shape)} != {(B, T, T)}"
     assert Q.shape == (B, T, HQ, DQ) and K.shape == (B, T, HQ, DQ), "Q/K shape"
     assert V.shape == (B, T, HQ, DV), "V shape"
     assert threshold.numel() == B * T, "threshold must hold one value per query"
@@ -110,6 +111,8 @@ def sparse_attention_hip(scores: torch.Tensor, threshold: torch.Tensor, Q, K, V,
     dt, Q, K, V = _attn_inputs(Q, K, V)
     if out is None:
         out = torch.empty(B, T, HQ, DV, device=Q.device, dtype=torch.float32)
+    else:
+        L.check_out(out, B * T * HQ * DV, Q.device)
     if tiled:
         kernel = "tiled"
     assert kernel in (None, "tiled", "staged", "mask", "dense", "gather"), f"unknown kernel {kernel!r}"
@@ -164,6 +167,7 @@ def selection_mask(scores: torch.Tensor, threshold: torch.Tensor) -> torch.Tenso
     range up to its 128-query block are 0, later ones are not written)."""
     L.require_gpu(scores, threshold)
     B, T, _ = scores.shape
+    assert scores.shape == (B, T, T), f"scores shape {tuple(scores.shape)} != {(B, T, T)}"
     assert threshold.numel() == B * T, "threshold must hold one value per query"
     scores = L.prep(scores, torch.float32)
     thr = L.prep(threshold, torch.float32)
@@ -190,6 +194,8 @@ def sparse_attention_from_mask(mask: torch.Tensor, Q, K, V,
     dt, Q, K, V = _attn_inputs(Q, K, V)
     if out is None:
         out = torch.empty(B, T, HQ, DV, device=Q.device, dtype=torch.float32)
+    else:
+        L.check_out(out, B * T * HQ * DV, Q.device)
     rc = L.lib().dsa_sparse_attn_mask(
         mask.data_ptr(), mask.shape[-1], Q.data_ptr(), K.data_ptr(), V.data_ptr(), L.dtype_code(dt),
         B, T, HQ, DQ, DV, 1.0 / math.sqrt(DQ), out.data_ptr(), L.stream_ptr(Q.device))

@@ -88,7 +88,8 @@ def indexer_scores_hip(q: torch.Tensor, k: torch.Tensor, w: torch.Tensor, *,
         if out is None:
             out = torch.empty((B, T, T), device=q.device, dtype=torch.float32)
         else:
-            assert out.shape == (B, T, T) and out.dtype == torch.float32 and out.is_contiguous()
+            assert out.shape == (B, T, T) and out.dtype == torch.float32 and out.is_contiguous() \
+                and out.device == q.device
         rc = L.lib().dsa_indexer_scores_fp8_scaled(
             q.data_ptr(), k.data_ptr(), w.data_ptr(),
             q_scale.data_ptr() if q_scale is not None else None,
@@ -106,7 +107,8 @@ def indexer_scores_hip(q: torch.Tensor, k: torch.Tensor, w: torch.Tensor, *,
     if out is None:
         out = torch.empty((B, T, T), device=q.device, dtype=torch.float32)
     else:
-        assert out.shape == (B, T, T) and out.dtype == torch.float32 and out.is_contiguous()
+        assert out.shape == (B, T, T) and out.dtype == torch.float32 and out.is_contiguous() \
+            and out.device == q.device
     rc = L.lib().dsa_indexer_scores(q.data_ptr(), k.data_ptr(), w.data_ptr(), L.dtype_code(dt),
                                     B, T, H, d, out.data_ptr(), T, 1 if write_upper else 0,
                                     L.stream_ptr(q.device))

@@ -518,3 +518,41 @@ def test_forward_never_splits_below_its_least_T(DI):
                for dt in (L.DSA_F32, L.DSA_BF16) for t in (1, T // 2, T - 1) for k in (8, T))
     if DI >= 128:  # from there on by the work alone, which needs no device
         assert f(L.DSA_BF16, 4096, T, 64, DI, 16, 128, 128, 8) == 1
+
+
+class _OnGpu(torch.Tensor):
+    """A CPU tensor that says it is on the GPU: what the host refuses is
+    refused before a kernel could be given its pointer."""
+
+    is_cuda = True
+
+
+@pytest.mark.parametrize("out", [
+    lambda B, T, H, D: torch.empty(3),                                   # too few values
+    lambda B, T, H, D: torch.empty(B, T, H, D, dtype=torch.bfloat16),    # half the bytes
+    lambda B, T, H, D: torch.empty(B, T, H, 2 * D)[..., ::2],            # another layout
+    lambda B, T, H, D: torch.empty(B, T, H, D, device="meta")])          # another device
+def test_attention_refuses_an_output_it_would_write_past(monkeypatch, out):
+    import dsa_attention as DA
+
+    monkeypatch.setattr(L, "lib", lambda: pytest.fail("reached the library"))
+    B, T, H, D = 1, 64, 2, 64
+    x = torch.zeros(B, T, H, D).as_subclass(_OnGpu)
+    s, thr = (torch.zeros(B, T, n).as_subclass(_OnGpu) for n in (T, 1))
+    mask = torch.zeros(B, T, 1, dtype=torch.int64).as_subclass(_OnGpu)
+    with pytest.raises(AssertionError, match="out: "):
+        DA.sparse_attention_hip(s, thr, x, x, x, out=out(B, T, H, D))
+    with pytest.raises(AssertionError, match="out: "):
+        DA.sparse_attention_from_mask(mask, x, x, x, out=out(B, T, H, D))
+
+
+def test_attention_refuses_scores_that_are_not_square(monkeypatch):
+    import dsa_attention as DA
+
+    monkeypatch.setattr(L, "lib", lambda: pytest.fail("reached the library"))
+    x = torch.zeros(1, 64, 2, 64).as_subclass(_OnGpu)
+    s, thr = (torch.zeros(1, 64, n).as_subclass(_OnGpu) for n in (32, 1))
+    with pytest.raises(AssertionError, match="scores shape"):
+        DA.sparse_attention_hip(s, thr, x, x, x)
+    with pytest.raises(AssertionError, match="scores shape"):
+        DA.selection_mask(s, thr)
