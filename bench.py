@@ -792,13 +792,14 @@ def pmc_workload(args, dev):
         D.sparse_attention_hip(scores, thr, Q, K, V, out=out)
     torch.cuda.synchronize()
     del scores, thr, Q, K, V, out
-    # config 3: indexer (fp32), select, and 2 attention launches
+    # config 3: indexer (fp32), select, and the attention on both kernels for it
     ins = gpu_inputs(C3, torch.float32, dev, seed=3)
     scores = indexer_scores_hip(*ins[:3], write_upper=False)
     thr = topk_threshold(scores, C3["k"], causal=True)
     out = torch.empty(C3["B"], C3["T"], C3["HQ"], C3["DV"], device=dev)
-    for _ in range(2):
-        D.sparse_attention_hip(scores, thr, *ins[3:], out=out)  # the dense kernel at this shape
+    for kernel in ("dense", "staged"):  # the first is what the call picks by itself here
+        for _ in range(2):
+            D.sparse_attention_hip(scores, thr, *ins[3:], out=out, kernel=kernel)
     torch.cuda.synchronize()
     log("pmc workload done")
 
@@ -836,7 +837,7 @@ def main():
                          "device-to-device copy (counter calibration), then --steps eager "
                          "fused launches at config 1, the config-4 indexer, 3 causal "
                          "selects and 2 tile-attention launches at config 4, then the "
-                         "config-3 indexer, select and 2 attention launches")
+                         "config-3 indexer, select, and 2 dense and 2 staged attentions")
     args = ap.parse_args()
     if args.gpus != 1:
         print(f"bench.py runs on one GPU only (got --gpus {args.gpus}): this build has no "

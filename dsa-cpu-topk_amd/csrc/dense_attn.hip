@@ -46,9 +46,9 @@
 // that select nothing get 0/0 = NaN, as the reference.
 //
 // What bounds the dense kernel at D = 64 fp32: per wave and 64-key tile 96
-// MFMAs (1536 cycles), ~440 VALU instructions (36 of them exp2 at a quarter of
-// the rate, ~2200 cycles) and 42 KB of LDS reads; one SIMD's two waves overlap
-// the first two only in part (about 5600 cycles for two tiles).  B = 4, T = 4096,
+// MFMAs (1536 cycles), ~350 VALU instructions (36 of them exp2 at a quarter of
+// the rate, ~1800 cycles) and 42 KB of LDS reads; one SIMD's two waves overlap
+// the first two only in part (about 5600 cycles for two tiles, MFMA busy 41%).  B = 4, T = 4096,
 // HQ = 8, k = 256 fp32: 253 us in all (prepare 48, 25 where the select has written
 // the bitmask; dense 192-200, redo 4.5) against 0.44 ms staged, relative error
 // against float64 2.1e-7 against 3.7e-7.

@@ -345,8 +345,8 @@ def _split_bound(q, k, w):
                                      (333, 9, 64), (50, 4, 256), (100, 40, 128), (90, 80, 128)])
 def test_fp32_pieces_shapes_and_scales(dev, T, HI, DI):
     """Edges of the query and key tiles, one and two blocks per CU, one-quad
-    tiles; rows of very different magnitude (scales 2^-50 .. 2^50, and beyond
-    the split's 2^+-60, which takes the plain fp32 pass)."""
+    tiles; rows of very different magnitude (scales 2^-50 .. 2^50, and 2^-66 ..
+    2^66, whose rows beyond the split's 2^60 take the plain fp32 pass)."""
     q, k, w, *_ = O.make_inputs(2, T, HI, DI, 1, 1, 1, seed0=T)
     g = torch.Generator().manual_seed(T + 1)
     for span in (0, 50, 66):
